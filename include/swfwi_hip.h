@@ -124,8 +124,8 @@ int swfwi_calgradient(swfwi_solver h, const float *encsrc, int shot, const float
  * shot loop, main-fm-damp.cpp:241-256): wlt [nt] -> dobs [ns][nt][ng]. */
 int swfwi_forward_shots(swfwi_solver h, const float *wlt, float *dobs);
 /* Grid-point updates (entry-weighted; the backward kernel counts its two
- * fields) and stencil launches issued by this handle so far, [0] forward
- * step kernel, [1] backward step kernel. */
+ * fields) and time steps run by this handle so far, one launch each or inside
+ * a resident time loop, [0] forward, [1] backward. */
 int swfwi_solver_counters(swfwi_solver h, double *point_updates, long long *launches);
 /* Capture time loops into HIP graphs and replay them when the same buffers
  * recur: 0 off, 1 batches of up to 8 entries (larger batches are not
@@ -148,6 +148,13 @@ int swfwi_solver_get_tile_x(swfwi_solver h, int kind, int entries, int *tile_x);
  * while the batch's wavefields fit the last-level cache, fused beyond).
  * Same results. */
 int swfwi_solver_set_bwd_split(swfwi_solver h, int mode);
+/* The resident time loop: -1 by rule (the default: batches small enough to
+ * keep their tiles on the chip run a whole time loop as one launch), 0 never,
+ * 1 wherever the tiles fit.  wait_us bounds how long a block of that launch
+ * waits for its neighbours (5e5 by default) before the run is done again with
+ * one launch per step (and, by rule, so are the handle's later runs).  A fixed tile width or backward form also means one
+ * launch per step.  Same results. */
+int swfwi_solver_set_resident(swfwi_solver h, int mode, double wait_us);
 /* Record a HIP event pair around every forward / backward time loop on the
  * handle's stream (graph replays included); swfwi_solver_kernel_times waits
  * for them and returns the accumulated milliseconds and step-kernel launch

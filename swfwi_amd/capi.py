@@ -60,6 +60,7 @@ SIGNATURES = {
     "swfwi_solver_kernel_times": (_I, [_VP, _f64, np.ctypeslib.ndpointer(np.int64, flags="C_CONTIGUOUS")]),
     "swfwi_solver_time_steps": (_I, [_VP, _I, _I, _I, _I, C.POINTER(_F)]),
     "swfwi_solver_set_bwd_split": (_I, [_VP, _I]),
+    "swfwi_solver_set_resident": (_I, [_VP, _I, C.c_double]),
     "swfwi_enkf_create": (_I, [C.POINTER(_VP), _VP, _f32, _f32, _F, _I]),
     "swfwi_enkf_destroy": (_I, [_VP]),
     "swfwi_enkf_set_members": (_I, [_VP, _f32]),
@@ -295,6 +296,11 @@ class Solver:
     def set_bwd_split(self, mode):
         """-1: by batch size (default), 0: fused backward blocks, 1: split."""
         check(load().swfwi_solver_set_bwd_split(self.h, int(mode)))
+
+    def set_resident(self, mode, wait_us=5e5):
+        """The resident time loop: -1 by rule, 0 never, 1 wherever it fits;
+        wait_us bounds one wait of a block before the per-step launches take over."""
+        check(load().swfwi_solver_set_resident(self.h, int(mode), float(wait_us)))
 
     def time_steps(self, kind, entries, tile_x, reps=100):
         """Microseconds per launch of back-to-back step kernels on scratch fields."""

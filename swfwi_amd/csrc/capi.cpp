@@ -420,6 +420,13 @@ int swfwi_solver_time_steps(swfwi_solver h, int kind, int entries, int tile_x, i
   });
 }
 
+int swfwi_solver_set_resident(swfwi_solver h, int mode, double wait_us) {
+  return guarded([&] {
+    NEED(h);
+    h->s->prop().set_resident(mode, wait_us);
+  });
+}
+
 int swfwi_solver_set_bwd_split(swfwi_solver h, int mode) {
   return guarded([&] {
     NEED(h);

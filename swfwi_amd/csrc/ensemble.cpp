@@ -122,7 +122,6 @@ void EnsembleFwi::epoch(int iter) {
   const std::vector<float> obj1 = s_.residual(obs_.get(), m, dcal_.get(), res_.get(), N);
   vsrc_.resize((size_t)N * m);
   op_trans_vsrc(res_.get(), vsrc_.get(), nt, ng, N, s);
-  launch_fill(g1_.get(), (long long)N * n, 0.f, s);
   s_.prop().backward(N, rv_.get(), n, src, vsrc_.get(), m, band_.get(), g1_.get(), n, w_);
   op_scale_mask(g1_.get(), n, N, g.gridgeom(), s);
   update_grads(iter);

@@ -161,6 +161,8 @@ Propagator::Propagator(const Geometry& g, int precision) : g_(g), prec_(precisio
     build_points(si, g_.ld, g_.ntz, ntx, kTileWidths[w], 0, src_[w], s);
     build_points(gi, g_.ld, g_.ntz, ntx, kTileWidths[w], 0, rec_[w], s);
   }
+  src_idx_ = si;
+  rec_idx_ = gi;
   sxp_.upload(sxp, s);
   szp_.upload(szp, s);
   gxp_.upload(gxp, s);
@@ -434,6 +436,16 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
                          Fields& w, int rvdiv) {
   const long long np = g_.npts();
   w.ensure(E, np, true);
+  if (resident_forward(E, rv, rvstride, src, dcal, band, w, rvdiv)) {
+    // (the widths a run of this size would fall back to, untimed)
+    tile_choice(0, E, rv, rvstride, rvdiv, w, false);
+    tile_choice(1, E, rv, rvstride, rvdiv, w, false);
+    plan_forward(w);  // sets the final state
+    flush_timing_if_full();
+    fwd_launches += g_.nt;
+    fwd_point_updates += (double)E * (g_.nxpad - 2 * kHalo) * (g_.nzpad - 2 * kHalo) * g_.nt;
+    return;
+  }
   // tile widths for this batch, chosen now while the workspace is free
   // (backward() runs on the state this forward leaves behind)
   const int tw = tile_choice(0, E, rv, rvstride, rvdiv, w, true);
@@ -592,6 +604,7 @@ void Propagator::flush_timing_if_full() {
 }
 
 Propagator::~Propagator() {
+  if (abort_host_) (void)hipHostFree(abort_host_);
   for (auto& ge : graph_cache_) (void)hipGraphExecDestroy(ge.exec);
   for (const TimedLoop& t : pending_) {
     (void)hipEventDestroy(t.start);
@@ -610,7 +623,17 @@ int Propagator::backward(int E, const float* rv, long long rvstride, const Sourc
   w.ensure(E, np, true);
   std::vector<float> wts;
   const int it_min = xcorr_range(g_.dt, g_.nt, wts);
-  if (it_min >= g_.nt) return 0;
+  if (it_min >= g_.nt) {
+    launch_fill(grad, (long long)E * np, 0.f, stream());
+    return 0;
+  }
+  const int iters = g_.nt - it_min;
+  if (resident_backward(E, rv, rvstride, src, vsrc, vstride, band, grad, gstride, w, rvdiv, it_min, wts)) {
+    flush_timing_if_full();
+    bwd_launches += iters;
+    bwd_point_updates += 2.0 * E * (g_.nxpad - 2 * kHalo) * (g_.nzpad - 2 * kHalo) * iters;
+    return iters;
+  }
   const int tw = tile_choice(1, E, rv, rvstride, rvdiv, w, false);
   const uintptr_t key[] = {2,
                            (uintptr_t)tw,
@@ -638,7 +661,6 @@ int Propagator::backward(int E, const float* rv, long long rvstride, const Sourc
     backward_body(E, rv, rvstride, src, vsrc, vstride, band, grad, gstride, w, rvdiv, it_min, wts, tw);
   }, stream());
   flush_timing_if_full();
-  const int iters = g_.nt - it_min;
   bwd_launches += iters;
   bwd_point_updates += 2.0 * E * (g_.nxpad - 2 * kHalo) * (g_.nzpad - 2 * kHalo) * iters;
   return iters;
@@ -654,6 +676,7 @@ void Propagator::backward_body(int E, const float* rv, long long rvstride, const
   float* s_prv = fw.s_nxt;
   float* g_cur = fw.spare0;
   float* g_prv = fw.spare1;
+  launch_fill(grad, (long long)E * np, 0.f, s);
   launch_fill(g_cur, (long long)E * np, 0.f, s);
   launch_fill(g_prv, (long long)E * np, 0.f, s);
 

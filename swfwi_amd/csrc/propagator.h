@@ -11,6 +11,7 @@
 #include "device.h"
 #include "kernels.h"
 #include "ops.h"
+#include "resident.h"
 
 namespace swfwi {
 
@@ -118,9 +119,9 @@ class Propagator {
   void forward_external(const float* rv, const Sources& src, float* dcal, float* fa, float* fb);
 
   // The backward half of calgradient on the state forward() left in w:
-  // vsrc [E][nt][ng] adjoint sources (+e*vstride), grad accumulates the
-  // imaging condition (+e*gstride; caller zeroes it).  Returns the number of
-  // backward iterations run.
+  // vsrc [E][nt][ng] adjoint sources (+e*vstride), grad receives the imaging
+  // condition (entries back to back, gstride npts(), 0 for one entry).
+  // Returns the number of backward iterations run.
   int backward(int E, const float* rv, long long rvstride, const Sources& src, const float* vsrc, long long vstride,
                const float* band, float* grad, long long gstride, Fields& w, int rvdiv = 1);
 
@@ -128,7 +129,14 @@ class Propagator {
   // (it = nt-1 down to the returned value), with their taper weights.
   static int xcorr_range(float dt, int nt, std::vector<float>& weights);
 
-  // launch counters for throughput accounting
+  // The resident time loop (resident.h): -1 by rule (the default: batches
+  // whose tiles fit the chip), 0 never, 1 wherever it fits.  wait_us bounds
+  // one wait of a block for its neighbours, after which the run is done again
+  // by the per-step kernels.  A fixed tile width or backward form also
+  // means the per-step kernels.
+  void set_resident(int mode, double wait_us);
+
+  // step counters for throughput accounting (a resident loop counts its steps)
   long long fwd_launches = 0, bwd_launches = 0;
   double fwd_point_updates = 0, bwd_point_updates = 0;
 
@@ -198,6 +206,28 @@ class Propagator {
   void backward_body(int E, const float* rv, long long rvstride, const Sources& src, const float* vsrc,
                      long long vstride, const float* band, float* grad, long long gstride, Fields& fw, int rvdiv,
                      int it_min, const std::vector<float>& wts, int w);
+  // The resident loop: the tiles of a run (kind 0 forward, 1 backward) and
+  // whether it can and should take that path; the runs (false: a wait ran
+  // out, nothing of the caller's but scratch was written that the per-step
+  // loop does not write itself).
+  bool plan_resident(int kind, int E, ResTiles& t);
+  struct ResLayout {
+    ResTiles t;
+    DBuf<int> sptr, rptr;
+    DBuf<int2> sitems, ritems;
+    bool fits = false;  // no tile holds more points than a block stages
+    ResPoints src() const { return ResPoints{sptr.get(), sitems.get()}; }
+    ResPoints rec() const { return ResPoints{rptr.get(), ritems.get()}; }
+  };
+  ResLayout& res_layout(const ResTiles& t);
+  ResGrid res_grid(const ResTiles& t) const;
+  bool res_begin(int fields, int E, int steps, ResComm& x);  // call with the device's lock held
+  bool res_end(int kind, long long steps, hipEvent_t t0);
+  bool resident_forward(int E, const float* rv, long long rvstride, const Sources& src, float* dcal, float* band,
+                        Fields& w, int rvdiv);
+  bool resident_backward(int E, const float* rv, long long rvstride, const Sources& src, const float* vsrc,
+                         long long vstride, const float* band, float* grad, long long gstride, Fields& w, int rvdiv,
+                         int it_min, const std::vector<float>& wts);
   // Tile width (index into kTileWidths) for a kernel kind (0 forward,
   // 1 backward) and batch size: fixed override, cached choice, or a timed
   // trial of every width on scratch wavefields (the tile tuner).
@@ -249,6 +279,20 @@ class Propagator {
   int bwd_split_ = -1;
   std::vector<std::pair<long long, int>> tile_cache_;  // (kind*2^32 + E) -> width index
   DBuf<int> sxp_, szp_, gxp_, gzp_;
+
+  int resident_ = -1;
+  double res_wait_us_ = kResWaitUs;
+  bool res_gave_up_ = false;  // a run's wait ran out: by rule, the handle then keeps to the per-step kernels
+  static constexpr double kResWaitUs = 5e5;
+  double ticks_per_us_ = 100;  // of the kernels' wall clock
+  std::vector<std::unique_ptr<ResLayout>> res_layouts_;
+  std::vector<long long> src_idx_, rec_idx_;  // grid indices of the points
+  int res_cap_[2][2] = {{-1, -1}, {-1, -1}};  // [kind][precision] blocks on the chip at once
+  DBuf<unsigned long long> xbuf_;
+  unsigned xbase_ = 0;
+  DBuf<int> abort_dev_;
+  int* abort_host_ = nullptr;
+  DBuf<float> res_wts_;
 };
 
 }  // namespace swfwi

@@ -1,0 +1,285 @@
+// Host side of the resident time loop: which runs take it, the tiles and point
+// lists of a run, its exchange buffer, and the launch under the device's lock.
+#include <algorithm>
+#include <map>
+#include <mutex>
+
+#include "propagator.h"
+
+namespace swfwi {
+
+namespace {
+
+// One resident run at a time onto a device: two of them could each hold part
+// of the chip and wait for blocks that cannot start.
+constexpr int kMaxDevices = 64;
+std::mutex& device_lock(int dev) {
+  static std::mutex mu[kMaxDevices];
+  return mu[dev >= 0 && dev < kMaxDevices ? dev : 0];
+}
+
+struct HostPoints {
+  std::vector<int> ptr;
+  std::vector<int2> items;
+  int most = 0;
+};
+
+HostPoints bucket(const std::vector<long long>& idx, int ld, const ResTiles& t) {
+  std::vector<std::vector<int2>> lists(t.n());
+  for (size_t i = 0; i < idx.size(); i++) {
+    const int ix = (int)(idx[i] / ld) - kHalo, iz = (int)(idx[i] % ld) - kHalo;
+    const int tx = ix / t.w, tz = iz / t.h;
+    lists[(size_t)tx * t.ntz + tz].push_back(make_int2(((ix - tx * t.w) << 6) | (iz - tz * t.h + 1), (int)i));
+  }
+  HostPoints h;
+  h.ptr.push_back(0);
+  for (const auto& l : lists) {
+    h.items.insert(h.items.end(), l.begin(), l.end());
+    h.ptr.push_back((int)h.items.size());
+    h.most = std::max(h.most, (int)l.size());
+  }
+  return h;
+}
+
+}  // namespace
+
+void Propagator::set_resident(int mode, double wait_us) {
+  if (mode < -1 || mode > 1) fail(kErrArg, "resident mode must be -1 (by rule), 0 or 1");
+  if (!(wait_us >= 0)) fail(kErrArg, "the resident wait limit must not be negative");
+  resident_ = mode;
+  res_wait_us_ = wait_us;
+  res_gave_up_ = false;
+}
+
+bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
+  if (resident_ == 0 || tile_override_ || (kind == 1 && bwd_split_ >= 0) || g_.nt < 2) return false;
+  const int most = kind == 1 ? kResMaxWidthBwd : kResMaxWidthFwd;
+  int& cap = res_cap_[kind][prec_];
+  if (cap < 0) {  // every width's kernel fits at least one block a CU
+    cap = resident_capacity(kind == 1, prec_, 1);
+    for (int w = kResWaves; w <= most; w += kResWaves) cap = std::min(cap, resident_capacity(kind == 1, prec_, w));
+  }
+  const int ux = g_.nxpad - 2 * kHalo, uz = g_.nzpad - 2 * kHalo;
+  t.ntz = (uz + kResTileZ - 1) / kResTileZ;
+  t.h = (uz + t.ntz - 1) / t.ntz;
+  t.ntz = (uz + t.h - 1) / t.h;
+  const int cols = cap / E / t.ntz;  // tile columns of an entry
+  if (cols < 1) return false;
+  t.w = std::max(kResWaves, (ux + cols - 1) / cols);
+  t.ntx = (ux + t.w - 1) / t.w;
+  if (t.w > most) return false;
+  if (resident_ == 1) return true;
+  if (res_gave_up_) return false;  // the chip is shared: a run of this handle has waited in vain
+  // Measured over E (forward / backward microseconds a step, per-step kernels
+  // -> resident): 201x301 E=1 4.7 -> 1.74, E=4 4.7 -> 2.7 / 8.1 -> 4.4, E=8
+  // 6.2 -> 3.6 / 10.4 -> 7.7, E=11 6.9 -> 5.3, E=16 7.9 -> 6.1, E=21 9.8 -> 8.1;
+  // 301x921 E=1 5.2 -> 2.7 / 6.7 -> 4.5; 501x1501 E=1 6.8 -> 3.8 / 10.4 -> 8.4.
+  // Side by side on streams, 2 to 4 entries of wide tiles are better left to
+  // the per-step kernels (301x921 E=4 5.4 against 7.1, 501x1501 E=2 7.0
+  // against 7.3).
+  return kind == 1 || E == 1 || E > kLanes || t.w <= kResLanesWidth;
+}
+
+Propagator::ResLayout& Propagator::res_layout(const ResTiles& t) {
+  for (auto& l : res_layouts_)
+    if (l->t.w == t.w && l->t.h == t.h) return *l;
+  hipStream_t s = stream();
+  auto l = std::make_unique<ResLayout>();
+  l->t = t;
+  const HostPoints src = bucket(src_idx_, g_.ld, t), rec = bucket(rec_idx_, g_.ld, t);
+  l->fits = src.most <= kResMaxPts && rec.most <= kResMaxPts;
+  l->sptr.upload(src.ptr, s);
+  l->sitems.upload(src.items, s);
+  l->rptr.upload(rec.ptr, s);
+  l->ritems.upload(rec.items, s);
+  SWFWI_HIP(hipStreamSynchronize(s));  // the host vectors end here
+  if (res_layouts_.size() >= 16) res_layouts_.erase(res_layouts_.begin());
+  res_layouts_.push_back(std::move(l));
+  return *res_layouts_.back();
+}
+
+ResGrid Propagator::res_grid(const ResTiles& t) const {
+  ResGrid g;
+  g.nx = g_.nxpad;
+  g.nz = g_.nzpad;
+  g.ld = g_.ld;
+  g.nb = g_.bx0;
+  g.zdamp = damp_.zdamp;
+  g.bx0 = g_.bx0;
+  g.bxn = g_.bxn;
+  g.bz0 = g_.bz0;
+  g.bzn = g_.bzn;
+  g.delta_x = damp_.dx.get();
+  g.delta_z = damp_.dz.get();
+  g.t = t;
+  return g;
+}
+
+bool Propagator::res_begin(int fields, int E, int steps, ResComm& x) {
+  hipStream_t s = stream();
+  if (!abort_host_) {
+    SWFWI_HIP(hipHostMalloc(reinterpret_cast<void**>(&abort_host_), sizeof(int), hipHostMallocMapped));
+    int dev = 0, khz = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0)
+      ticks_per_us_ = khz * 1e-3;
+    abort_dev_.resize(1);
+    *abort_host_ = 1;  // cleared below
+  }
+  const size_t words = (size_t)2 * fields * E * (size_t)g_.npts();
+  // no word of the buffer carries a stamp of this run: stamps grow, and the
+  // words are cleared when the buffer is new or the stamps would wrap
+  if (words > xbuf_.size() || xbase_ > 0xffffffffu - (unsigned)steps - 2) {
+    xbuf_.resize(std::max(words, xbuf_.size()));
+    launch_fill(reinterpret_cast<float*>(xbuf_.get()), 2 * (long long)xbuf_.size(), 0.f, s);
+    xbase_ = 0;
+  }
+  if (*abort_host_) {
+    launch_fill(reinterpret_cast<float*>(abort_dev_.get()), 1, 0.f, s);
+    *abort_host_ = 0;
+  }
+  x.buf = xbuf_.get();
+  x.base = xbase_;
+  xbase_ += (unsigned)steps + 1;
+  x.abort_dev = abort_dev_.get();
+  void* mapped = nullptr;
+  SWFWI_HIP(hipHostGetDevicePointer(&mapped, abort_host_, 0));
+  x.abort_host = static_cast<int*>(mapped);
+  x.limit = (long long)(res_wait_us_ * ticks_per_us_);
+  return true;
+}
+
+bool Propagator::res_end(int kind, long long steps, hipEvent_t t0) {
+  hipEvent_t t1 = nullptr;
+  if (timing_) {
+    t1 = pooled_event();
+    SWFWI_HIP(hipEventRecord(t1, stream()));
+  }
+  SWFWI_HIP(hipGetLastError());
+  SWFWI_HIP(hipStreamSynchronize(stream()));
+  const bool ok = *static_cast<volatile int*>(abort_host_) == 0;
+  if (!ok) res_gave_up_ = true;
+  if (timing_) {
+    if (ok) {
+      pending_.push_back(TimedLoop{t0, t1, kind, steps});
+    } else {
+      event_pool_.push_back(t0);
+      event_pool_.push_back(t1);
+    }
+  }
+  return ok;
+}
+
+bool Propagator::resident_forward(int E, const float* rv, long long rvstride, const Sources& src, float* dcal,
+                                  float* band, Fields& w, int rvdiv) {
+  ResTiles t;
+  if (!plan_resident(0, E, t)) return false;
+  ResLayout& l = res_layout(t);
+  if (!l.fits) return false;
+  hipStream_t s = stream();
+  const long long np = g_.npts();
+  std::lock_guard<std::mutex> lock(device_lock(dev_));
+  ResFwdArgs a;
+  res_begin(1, E, g_.nt, a.x);
+  hipEvent_t t0 = nullptr;
+  if (timing_) {
+    t0 = pooled_event();
+    SWFWI_HIP(hipEventRecord(t0, s));
+  }
+  launch_fill(w.a.get(), (long long)E * np, 0.f, s);
+  launch_fill(w.b.get(), (long long)E * np, 0.f, s);
+  Inject inj;
+  inj.pts = src_[0].view();
+  inj.amp = src.amp;
+  inj.ld = src.ld;
+  inj.estride = src.estride;
+  inj.lo = src.lo;
+  inj.hi = src.hi;
+  inj.t = 0;
+  launch_point_inject(w.b.get(), np, inj, g_.ns(), E, s);
+  a.g = res_grid(t);
+  a.E = E;
+  a.nt = g_.nt;
+  a.fstride = np;
+  a.fa = w.a.get();
+  a.fb = w.b.get();
+  a.rv = rv;
+  a.rvstride = rvstride;
+  a.rvdiv = rvdiv;
+  a.src = l.src();
+  a.rec = l.rec();
+  a.amp = src.amp;
+  a.amp_ld = src.ld;
+  a.amp_estride = src.estride;
+  a.lo = src.lo;
+  a.hi = src.hi;
+  a.dcal = dcal;
+  a.ng = g_.ng();
+  a.band = band;
+  a.bsize = g_.bsize;
+  launch_resident_fwd(a, prec_, s);
+  return res_end(0, g_.nt, t0);
+}
+
+bool Propagator::resident_backward(int E, const float* rv, long long rvstride, const Sources& src, const float* vsrc,
+                                   long long vstride, const float* band, float* grad, long long gstride, Fields& w,
+                                   int rvdiv, int it_min, const std::vector<float>& wts) {
+  ResTiles t;
+  if (!plan_resident(1, E, t)) return false;
+  ResLayout& l = res_layout(t);
+  if (!l.fits) return false;
+  hipStream_t s = stream();
+  const long long np = g_.npts();
+  const int nt = g_.nt, ng = g_.ng();
+  if (res_wts_.size() != wts.size()) {  // the taper weights follow from dt and nt alone
+    res_wts_.upload(wts, s);
+    SWFWI_HIP(hipStreamSynchronize(s));
+  }
+  std::lock_guard<std::mutex> lock(device_lock(dev_));
+  ResBwdArgs a;
+  res_begin(2, E, nt, a.x);
+  hipEvent_t t0 = nullptr;
+  if (timing_) {
+    t0 = pooled_event();
+    SWFWI_HIP(hipEventRecord(t0, s));
+  }
+  launch_fill(grad, (long long)E * np, 0.f, s);
+  launch_fill(w.spare0, (long long)E * np, 0.f, s);
+  Inject ginj;
+  ginj.pts = rec_[0].view();
+  ginj.amp = vsrc;
+  ginj.ld = ng;
+  ginj.estride = vstride;
+  ginj.t = nt - 1;
+  launch_point_inject(w.spare0, np, ginj, ng, E, s);
+  a.g = res_grid(t);
+  a.E = E;
+  a.nt = nt;
+  a.it_min = it_min;
+  a.fstride = np;
+  a.s_cur = w.s_cur;
+  a.s_nxt = w.s_nxt;
+  a.g_cur = w.spare0;
+  a.rv = rv;
+  a.rvstride = rvstride;
+  a.rvdiv = rvdiv;
+  a.src = l.src();
+  a.rec = l.rec();
+  a.amp = src.amp;
+  a.amp_ld = src.ld;
+  a.amp_estride = src.estride;
+  a.lo = src.lo;
+  a.hi = src.hi;
+  a.vsrc = vsrc;
+  a.ng = ng;
+  a.vstride = vstride;
+  a.band = band;
+  a.bsize = g_.bsize;
+  a.weights = res_wts_.get();
+  a.grad = grad;
+  a.gstride = gstride;
+  launch_resident_bwd(a, prec_, s);
+  return res_end(1, nt - it_min, t0);
+}
+
+}  // namespace swfwi

@@ -146,7 +146,6 @@ void Solver::calgradient(const float* encsrc, int shot, const float* vsrc_host, 
   vsrc.upload(vsrc_host, (size_t)nt * ng, s);
   band.resize((size_t)nt * g.bsize);
   grad.resize((size_t)npts());
-  launch_fill(grad.get(), npts(), 0.f, s);
   prop_.forward(1, rv_.get(), 0, src, nullptr, band.get(), w);
   prop_.backward(1, rv_.get(), 0, src, vsrc.get(), 0, band.get(), grad.get(), 0, w);
   grad.download(grad_host, (size_t)npts(), s);
@@ -337,7 +336,6 @@ void Inversion::ess_epoch(int iter) {
   st_.initobj = iter == 0 ? obj1 : st_.initobj;
   s_.vsrc.resize((size_t)m);
   op_trans_vsrc(s_.res.get(), s_.vsrc.get(), nt, ng, 1, s);
-  launch_fill(g1_.get(), n, 0.f, s);
   s_.prop().backward(1, s_.rv(), 0, src, s_.vsrc.get(), 0, s_.band.get(), g1_.get(), 0, s_.w);
   op_scale_mask(g1_.get(), 0, 1, g.gridgeom(), s);
   update_grad(g1_.get(), iter);
@@ -420,7 +418,6 @@ void Inversion::fwi_epoch(int iter) {
   s_.vsrc.resize((size_t)ns * m);
   op_trans_vsrc(s_.res.get(), s_.vsrc.get(), nt, ng, ns, s);
   s_.grad.resize((size_t)ns * n);
-  launch_fill(s_.grad.get(), (long long)ns * n, 0.f, s);
   s_.prop().backward(ns, s_.rv(), 0, src, s_.vsrc.get(), m, s_.band.get(), s_.grad.get(), n, s_.w);
   op_scale_mask(s_.grad.get(), n, ns, g.gridgeom(), s);
   op_sum_entries(s_.grad.get(), n, ns, n, g1_.get(), s);
