@@ -248,9 +248,11 @@ int swfwi_batch_set_snapshot_precision(swfwi_batch b, int snap_prec);
 int swfwi_batch_set_graphs(swfwi_batch b, int on);
 /* The tuner (1, the default) or the rules alone (0): the first forward run
  * times the step kernels at tile widths 16, 24 and 32 and both block orders
- * over every entry, and keeps the rules' choice (width 24 from 8000 tiles of
- * 64 x 16, else 16; order 1) unless another is faster by 3% in both timed
- * rounds.  swfwi_batch_tile_x receives the width in use. */
+ * over every entry, and keeps the rules' choice (a width by the batch's size;
+ * order 1) unless another is faster by 3% in both timed rounds.
+ * swfwi_batch_tile_x receives the width in use.  (A width stands for how many
+ * rows along x a wave of the step kernel advances: 6, 10 or 14, and 14, 22 or
+ * 30 in large batches.) */
 int swfwi_batch_set_tuning(swfwi_batch b, int on);
 /* A fixed tile width, 16, 24 or 32, or 0 for the rule and the tuner. */
 int swfwi_batch_set_tile_x(swfwi_batch b, int tile_x);

@@ -71,6 +71,11 @@ void Batch::set_block_order(int order) {
   set_tuning(tune_);
 }
 
+int Batch::strip_count(int uz) const {
+  const int most = order_ == kOrder4 ? kBatchStrip4 : kBatchStrip10;
+  return (uz + most - 1) / most;
+}
+
 void Batch::layout_tiles(int tx, int order) {
   hipStream_t s = stream_.get();
   SWFWI_HIP(hipStreamSynchronize(s));  // no launch in flight reads the old layout
@@ -81,11 +86,17 @@ void Batch::layout_tiles(int tx, int order) {
   // hold whole runs of shots of a model: each run's blocks are contiguous
   std::vector<int> blk;
   tile0_.assign(ent_.size() + 1, 0);
-  for (BatchEntry& e : ent_) e.ntx = (e.nxpad - 2 * kHalo + tx - 1) / tx;
+  for (BatchEntry& e : ent_) {
+    const int ux = e.nxpad - 2 * kHalo, uz = e.nzpad - 2 * kHalo;
+    e.nstrip = strip_count(uz);
+    e.h = 2 * ((uz + 2 * e.nstrip - 1) / (2 * e.nstrip));
+    e.rows = strip_rows_ < kBatchLongWalks ? tx / 2 - 2 : tx - 2;
+    e.nchunk = (ux + e.rows - 1) / e.rows;
+  }
   for (size_t r = 0; r < ent_.size();) {
     size_t r1 = r + 1;
     while (r1 < ent_.size() && ent_[r1].model == ent_[r].model) r1++;
-    const int nt_e = ent_[r].ntz * ent_[r].ntx;
+    const int nt_e = ent_[r].nstrip * ent_[r].nchunk;
     if (nt_e >= (1 << kBlkTileBits)) fail(kErrRange, "too many tiles per batch entry");
     if (order == 1) {
       for (int t = 0; t < nt_e; t++)
@@ -151,16 +162,14 @@ void Batch::tune() {
       for (int r = 0; r < kReps; r++) {
         a.it_or_k = r;
         a.rot = r;
-        a.nblocks = tile0_[n];
-        launch_batch_fwd(a, prec_, order_, tile_x_, s);
+        launch_batch_step(a, true, prec_, order_, tile0_[n], s);
       }
       if (bwd) {
         BatchKernelArgs b = args(false);
         for (int r = 0; r < kReps; r++) {
           b.it_or_k = r;
           b.rot = r;
-          b.nblocks = tile0_[n];
-          launch_batch_bwd(b, prec_, order_, tile_x_, s);
+          launch_batch_step(b, false, prec_, order_, tile0_[n], s);
         }
       }
       SWFWI_HIP(hipEventRecord(e1, s));
@@ -205,13 +214,14 @@ void Batch::build() {
   std::vector<float> amp, wts;
   long long model_len = 0, dcal_len = 0, grad_len = 0;
   int mbase = 0;
-  // tile width from the batch's size in 64 x 16 tiles
-  long long t16 = 0;
+  // chunk length from the batch's size in strip rows
   for (const BatchGroup& G : g_) {
-    const long long ux = G.nx + 2 * G.nb, uz = G.nz + G.nb;  // update region
-    t16 += (long long)G.nmodels * (long long)G.sx.size() * ((uz + kBatchTileZ - 1) / kBatchTileZ) * ((ux + 15) / 16);
+    const int strips = strip_count(G.nz + G.nb);
+    strip_rows_ += (long long)G.nmodels * (long long)G.sx.size() * strips * (G.nx + 2 * G.nb);
   }
-  tile_x_ = rule_x_ = t16 >= kBatchWideTiles ? 24 : 16;
+  rule_x_ = strip_rows_ < 14000 ? 16 : strip_rows_ < 25000 ? 24 : strip_rows_ < kBatchLongWalks ? 32
+            : strip_rows_ < 120000 ? 24 : 32;
+  tile_x_ = rule_x_;
   for (size_t gi = 0; gi < g_.size(); gi++) {
     const BatchGroup& G = g_[gi];
     const int ns = (int)G.sx.size();
@@ -252,8 +262,6 @@ void Batch::build() {
         BatchEntry e{};
         e.nxpad = nxpad;
         e.nzpad = nzpad;
-        e.ntz = (nzpad - 2 * kHalo + kBatchTileZ - 1) / kBatchTileZ;
-        e.ntx = (nxpad - 2 * kHalo + tile_x_ - 1) / tile_x_;
         e.damp = bx0;
         e.dscale = G.dscale;
         e.nt = G.nt;
@@ -371,11 +379,15 @@ void Batch::run_loop(bool fwd) {
       while (act > 0 && ent_[act - 1].nt <= it) act--;
       a.it_or_k = it;
       a.rot = it;
-      a.nblocks = tile0_[act];
-      a.tap_k = -1;
       for (size_t k = 0; k < taps_.size(); k++)
-        if (taps_[k] == it) a.tap_k = (int)k;
-      launch_batch_fwd(a, prec_, order_, tile_x_, s);
+        if (taps_[k] == it) a.tap_k = (int)k;  // the last listed slot of the step
+      if (a.tap_k >= 0) {
+        int columns = 0;
+        for (const BatchEntry& e : ent_) columns = std::max(columns, e.tap_nx);
+        launch_batch_tap(a, columns, n, s);
+        a.tap_k = -1;
+      }
+      launch_batch_step(a, true, prec_, order_, tile0_[act], s);
       if (hook_ && (it + 2) % kSnapEvery == 0) {
         // after step it the buffer step it wrote holds the field at it+1
         float* cur = (it & 1) == 0 ? fa_.get() : fb_.get();
@@ -393,8 +405,7 @@ void Batch::run_loop(bool fwd) {
       while (act > 0 && ent_[act - 1].nt - ent_[act - 1].it_last <= k) act--;
       a.it_or_k = k;
       a.rot = k;
-      a.nblocks = tile0_[act];
-      launch_batch_bwd(a, prec_, order_, tile_x_, s);
+      launch_batch_step(a, false, prec_, order_, tile0_[act], s);
     }
   }
 }
@@ -486,8 +497,7 @@ void Batch::step_from(const float* prev_host, const float* cur_host, int it0, in
     while (act > 0 && ent_[act - 1].nt <= it) act--;
     a.it_or_k = it;
     a.rot = k;
-    a.nblocks = tile0_[act];
-    launch_batch_fwd(a, kSnapNone, order_, tile_x_, s);
+    launch_batch_step(a, true, kSnapNone, order_, tile0_[act], s);
     if (hook_ && (it + 2) % kSnapEvery == 0) {  // the correction, as in forward runs
       float* cur = (k & 1) == 0 ? fa_.get() : fb_.get();
       float* prev = (k & 1) == 0 ? fb_.get() : fa_.get();

@@ -18,17 +18,19 @@
 namespace swfwi {
 
 constexpr int kSnapEvery = 4;
-// Step-kernel tile: 64 z x 16, 24 or 32 x output points per block of 256
-// threads (each thread 4, 6 or 8 consecutive x at one z).  The rule: 24 when
-// the batch holds at least kBatchWideTiles tiles of 64 x 16, else 16
-// (measured with a model's shots tile by tile: 16 entries of the 501x1501
-// grid, 14 112 such tiles, forward + backward 300.6 ms at 24 against 310.4 at
-// 32 and 329.4 at 16; the 112 mixed-size entries 1033 ms at 24 against 1068 at
-// 32; 16 entries of the 793x277 padded coarse grid, 3 920 tiles, 54.4 ms at
-// 16, 55.1 at 24, 61.1 at 32).  At 24 a block's LDS (17.8 KB) leaves room for
-// 8 blocks per CU, at 32 (22.4 KB) for 7.
-constexpr int kBatchTileZ = 64;
-constexpr int kBatchWideTiles = 8000;
+// A wave's work in the step kernel is a strip of z (up to kBatchStrip10 or
+// kBatchStrip4 outputs) walked along x for a chunk of rows.  A chunk of n rows
+// reads n + 12 of the field, so long chunks move less and short ones are more
+// waves.  "Tile width" 16, 24 or 32 stands for 6, 10 or 14 rows, and for 14, 22
+// or 30 from kBatchLongWalks strip rows (strips x rows of x, over all entries)
+// on.  The rule, measured (forward microseconds a step): 16 below 14000 strip
+// rows (one 201x301 entry, 682: 5.6 / 6.8 / 8.1 with 6 / 10 / 14 rows), 24 below
+// 25000 (24 such entries: 10.3 / 10.0 / 11.4), 32 below kBatchLongWalks (12
+// entries of 301x921, 35316: 16.1 / 15.1 / 14.7, 30 rows 17.9), 24 below
+// 120000, else 32 (the 112 mixed entries, 268000: 72.1 with 14, 71.9 with 22
+// or 30, 74 with 46, 78 with 62; backward 27.4 / 26.2 / 26.2).
+constexpr int kBatchStrip10 = 116, kBatchStrip4 = 124;
+constexpr int kBatchLongWalks = 60000;
 constexpr int kBlkTileBits = 20;  // tiles per entry < 2^20, entries < 2^11
 constexpr int kRuleOrder = 1;      // block order without tuning: a model's shots tile by tile
 constexpr float kBatchTuneMargin = 0.03f;
@@ -57,7 +59,8 @@ struct BatchGroup {
 // Device description of one entry (one shot of one model).
 struct BatchEntry {
   int nxpad, nzpad;      // padded grid; z contiguous (ld = nzpad)
-  int ntz, ntx;          // tiles over the update region [6, n-6)
+  int nstrip, h;         // strips along z of the update region [6, n-6), h outputs each
+  int nchunk, rows;      // chunks along x of `rows` rows each
   int damp;              // width of the sponge profile (bx0 = nb + 6)
   float dscale;          // sponge strength factor
   int nt, it_last;       // forward steps; last backward iteration run
@@ -90,15 +93,17 @@ struct BatchKernelArgs {
   float* grad;
   int it_or_k;           // forward: step it; backward: iteration count k (it = nt - 1 - k)
   int rot;               // buffer rotation: even reads cur from fb, odd from fa
-  int nblocks;
+  int nblocks, nunits;   // blocks and waves of work of the launch
   float* tap;            // restrictions of cur to the 2x-coarser grid (or null)
   int tap_k;             // tap slot written by this launch, -1 for none
 };
 
 void launch_batch_init_fwd(const BatchKernelArgs& a, int nentries, hipStream_t s);
-void launch_batch_fwd(const BatchKernelArgs& a, int prec, int order, int tile_x, hipStream_t s);
+// one step of the first `units` waves of work of the block list
+void launch_batch_step(const BatchKernelArgs& a, bool fwd, int prec, int order, int units, hipStream_t s);
+// tap slot a.tap_k of every entry (columns: the most coarse columns of one)
+void launch_batch_tap(const BatchKernelArgs& a, int columns, int nentries, hipStream_t s);
 void launch_batch_init_bwd(const BatchKernelArgs& a, int nentries, hipStream_t s);
-void launch_batch_bwd(const BatchKernelArgs& a, int prec, int order, int tile_x, hipStream_t s);
 void launch_fill_u32(unsigned* p, long long n, unsigned v, hipStream_t s);
 void launch_sub(const float* a, const float* b, float* out, long long n, hipStream_t s);  // out = a - b
 
@@ -210,6 +215,8 @@ class Batch {
   std::vector<int> run_of_;          // constructor order -> run index
   std::vector<Layout> lay_;
   std::vector<int> tile0_;           // per run index, prefix of tiles
+  int strip_count(int uz) const;     // strips of an update region uz high
+  long long strip_rows_ = 0;         // strips x rows of x over all entries
   int tile_x_ = 16;                  // step-kernel tile width
   int rule_x_ = 16;                  // the size rule's width
   bool tune_ = true, tuned_ = false;
