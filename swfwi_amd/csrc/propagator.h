@@ -221,7 +221,7 @@ class Propagator {
   };
   ResLayout& res_layout(const ResTiles& t);
   ResGrid res_grid(const ResTiles& t) const;
-  bool res_begin(int fields, int E, int steps, ResComm& x);  // call with the device's lock held
+  void res_begin(int kind, int E, ResComm& x);  // call with the device's lock held
   bool res_end(int kind, long long steps, hipEvent_t t0);
   bool resident_forward(int E, const float* rv, long long rvstride, const Sources& src, float* dcal, float* band,
                         Fields& w, int rvdiv);
@@ -288,7 +288,7 @@ class Propagator {
   std::vector<std::unique_ptr<ResLayout>> res_layouts_;
   std::vector<long long> src_idx_, rec_idx_;  // grid indices of the points
   int res_cap_[2][2] = {{-1, -1}, {-1, -1}};  // [kind][precision] blocks on the chip at once
-  DBuf<unsigned long long> xbuf_;
+  DBuf<unsigned long long> xbuf_[2];  // exchange words, forward and backward
   unsigned xbase_ = 0;
   DBuf<int> abort_dev_;
   int* abort_host_ = nullptr;

@@ -4,6 +4,7 @@
 #include <map>
 #include <mutex>
 
+#include "batch.h"
 #include "propagator.h"
 
 namespace swfwi {
@@ -71,12 +72,12 @@ bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   if (resident_ == 1) return true;
   if (res_gave_up_) return false;  // the chip is shared: a run of this handle has waited in vain
   // Measured over E (forward / backward microseconds a step, per-step kernels
-  // -> resident): 201x301 E=1 4.7 -> 1.74, E=4 4.7 -> 2.7 / 8.1 -> 4.4, E=8
-  // 6.2 -> 3.6 / 10.4 -> 7.7, E=11 6.9 -> 5.3, E=16 7.9 -> 6.1, E=21 9.8 -> 8.1;
-  // 301x921 E=1 5.2 -> 2.7 / 6.7 -> 4.5; 501x1501 E=1 6.8 -> 3.8 / 10.4 -> 8.4.
-  // Side by side on streams, 2 to 4 entries of wide tiles are better left to
-  // the per-step kernels (301x921 E=4 5.4 against 7.1, 501x1501 E=2 7.0
-  // against 7.3).
+  // -> resident): 201x301 E=1 4.7 -> 1.74, E=4 4.7 -> 2.7 / 8.1 -> 3.4, E=8
+  // 6.2 -> 3.6 / 10.4 -> 5.2, E=11 6.9 -> 5.3 / 11.4 -> 9.1, E=16 7.9 -> 6.1,
+  // E=21 9.8 -> 8.1; 301x921 E=1 5.2 -> 2.7 / 6.6 -> 3.4; 501x1501 E=1 6.8 ->
+  // 4.0 / 10.4 -> 6.2.  Side by side on streams, 2 to 4 entries of wide tiles
+  // are better left to the per-step kernels (301x921 E=4 5.4 against 7.1,
+  // 501x1501 E=2 7.0 against 7.3).
   return kind == 1 || E == 1 || E > kLanes || t.w <= kResLanesWidth;
 }
 
@@ -115,7 +116,7 @@ ResGrid Propagator::res_grid(const ResTiles& t) const {
   return g;
 }
 
-bool Propagator::res_begin(int fields, int E, int steps, ResComm& x) {
+void Propagator::res_begin(int kind, int E, ResComm& x) {
   hipStream_t s = stream();
   if (!abort_host_) {
     SWFWI_HIP(hipHostMalloc(reinterpret_cast<void**>(&abort_host_), sizeof(int), hipHostMallocMapped));
@@ -126,27 +127,30 @@ bool Propagator::res_begin(int fields, int E, int steps, ResComm& x) {
     abort_dev_.resize(1);
     *abort_host_ = 1;  // cleared below
   }
-  const size_t words = (size_t)2 * fields * E * (size_t)g_.npts();
-  // no word of the buffer carries a stamp of this run: stamps grow, and the
-  // words are cleared when the buffer is new or the stamps would wrap
-  if (words > xbuf_.size() || xbase_ > 0xffffffffu - (unsigned)steps - 2) {
-    xbuf_.resize(std::max(words, xbuf_.size()));
-    launch_fill(reinterpret_cast<float*>(xbuf_.get()), 2 * (long long)xbuf_.size(), 0.f, s);
+  DBuf<unsigned long long>& buf = xbuf_[kind];
+  const size_t words = (size_t)(kind == 1 ? 3 : 2) * E * (size_t)g_.npts();
+  if (kind == 1) {
+    buf.resize(std::max(words, buf.size()));
+    launch_fill_u32(reinterpret_cast<unsigned*>(buf.get()), 2 * (long long)words, 0xffffffffu, s);  // empty
+  } else if (words > buf.size() || xbase_ > 0xffffffffu - (unsigned)g_.nt - 2) {
+    // no word of the buffer carries a stamp of this run: stamps grow, and the
+    // words are cleared when the buffer is new or the stamps would wrap
+    buf.resize(std::max(words, buf.size()));
+    launch_fill_u32(reinterpret_cast<unsigned*>(buf.get()), 2 * (long long)buf.size(), 0u, s);
     xbase_ = 0;
   }
   if (*abort_host_) {
     launch_fill(reinterpret_cast<float*>(abort_dev_.get()), 1, 0.f, s);
     *abort_host_ = 0;
   }
-  x.buf = xbuf_.get();
+  x.buf = buf.get();
   x.base = xbase_;
-  xbase_ += (unsigned)steps + 1;
+  if (kind == 0) xbase_ += (unsigned)g_.nt + 1;
   x.abort_dev = abort_dev_.get();
   void* mapped = nullptr;
   SWFWI_HIP(hipHostGetDevicePointer(&mapped, abort_host_, 0));
   x.abort_host = static_cast<int*>(mapped);
   x.limit = (long long)(res_wait_us_ * ticks_per_us_);
-  return true;
 }
 
 bool Propagator::res_end(int kind, long long steps, hipEvent_t t0) {
@@ -180,7 +184,7 @@ bool Propagator::resident_forward(int E, const float* rv, long long rvstride, co
   const long long np = g_.npts();
   std::lock_guard<std::mutex> lock(device_lock(dev_));
   ResFwdArgs a;
-  res_begin(1, E, g_.nt, a.x);
+  res_begin(0, E, a.x);
   hipEvent_t t0 = nullptr;
   if (timing_) {
     t0 = pooled_event();
@@ -237,7 +241,7 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
   }
   std::lock_guard<std::mutex> lock(device_lock(dev_));
   ResBwdArgs a;
-  res_begin(2, E, nt, a.x);
+  res_begin(1, E, a.x);
   hipEvent_t t0 = nullptr;
   if (timing_) {
     t0 = pooled_event();

@@ -9,7 +9,8 @@
 // only publishes the 6-wide edge of its new field and collects its neighbours'
 // edges.
 //
-// Exchange: every published value travels as one 8-byte word (value, stamp)
+// Exchange: a published value travels as one 8-byte word (value, stamp), the
+// two fields' values of the backward loop as one word that is empty before,
 // written and read with relaxed agent-scope atomics (single-copy atomic, past
 // the per-XCD L2s), so a reader knows a value has arrived from the word
 // itself: no flags, fences or cache write-backs.  Stamps grow over the life of
@@ -36,7 +37,7 @@ constexpr int kResTileZ = 62;               // most outputs along z: lanes 1..62
 constexpr int kResLdz = 64 + 2 * 6;         // LDS row of a tile: z from -6 to 69
 constexpr int kResMaxPts = 512;             // sources or receivers of one tile, one per thread
 constexpr int kResMaxWidthFwd = 128;        // widest tile (x)
-constexpr int kResMaxWidthBwd = 56;          // (more rows a wave spill: 69 columns 16.0 us against 11.4 per step)
+constexpr int kResMaxWidthBwd = 80;          // (spills from 57 columns on; 69 columns still 9.1 against 11.4 us per step)
 constexpr int kResLanesWidth = 80;           // widest for 2 to 4 forward entries
 
 // Tiles of one entry: w x h outputs each (the last column and row may be smaller).
@@ -53,8 +54,8 @@ struct ResPoints {
 };
 
 struct ResComm {
-  unsigned long long* buf = nullptr;  // [2 parities][fields][E][npts] words
-  unsigned base = 0;                  // stamps of this run are base + 1 ...
+  unsigned long long* buf = nullptr;  // forward [2][E][npts] stamped words, backward [3][E][npts] pairs, empty
+  unsigned base = 0;                  // stamps of a forward run are base + 1 ...
   int* abort_dev = nullptr;           // set by a block that gives up
   int* abort_host = nullptr;          // the same for the host (mapped)
   long long limit = 0;                // longest wait, in 100 MHz ticks

@@ -9,9 +9,11 @@
 // ends.  Two barriers per step: cur complete (own rows and halo) -> u2 ->
 // barrier -> update, publish, collect the halo -> barrier.
 //
-// What bounds a step: the exchange (store past the L2, neighbour's poll) takes
-// 1.8-2.5 us on its own, measured without any stencil work; the arithmetic
-// adds about 0.3 us per row of a wave.
+// What bounds a step: the exchange (a store past the L2, the neighbour's poll:
+// 1.4-2.3 us on its own, measured without stencil work) and, on wide tiles, the
+// arithmetic (about 0.3 us per row of a wave).  Forward 1.74 / 2.7 / 4.0 us a
+// step on the 201x301 / 301x921 / 501x1501 grids, against 4.7 / 5.2 / 6.8 as
+// launches; backward 3.4 / 6.2 on the last two, against 6.6 / 10.4.
 #include "resident.h"
 
 #include "step_math.h"
@@ -94,13 +96,13 @@ struct Halo {
   int l[NH];       // LDS index
   unsigned on;     // bit j: point j exists
 };
-template <int NW, int NH>
+template <int NT, int NH>
 __device__ __forceinline__ void halo_points(const ResGrid& g, const Place& p, Halo<NH>& hp) {
   const int nside = 12 * p.h, nend = 12 * p.w, ntot = nside + nend + 36;
   hp.on = 0;
 #pragma unroll
   for (int j = 0; j < NH; j++) {
-    const int i = p.tid + j * 64 * NW;
+    const int i = (int)threadIdx.x + j * NT;
     int rx = 0, rz = 0;  // tile coordinates
     if (i < nside) {
       const int r = i / p.h;
@@ -131,42 +133,75 @@ __device__ __forceinline__ void halo_points(const ResGrid& g, const Place& p, Ha
 // 3.92 / 3.98 / 4.17 on the 501x1501 one).
 constexpr int kFirstPoll = 12;
 
-// Collects the halo words of stamp `want` from F fields (word arrays at w0 +
-// f * fs) into LDS (c0, c1); false when the wait ran out or another block gave up.
-template <int NH, int F>
-__device__ __forceinline__ bool collect(const ResComm& x, const u64* w0, long long fs, Halo<NH>& hp, unsigned want,
-                                        float* c0, float* c1) {
-  u64 v[F][NH];
+// Whether a wait has to end: it ran out of time (t0: when it began, 0 at the
+// first look) or another block gave up.
+__device__ __forceinline__ bool give_up(const ResComm& x, int spin, long long& t0) {
+  if ((spin & 63) != 63 && x.limit != 0) return false;
+  const long long now = wall_clock64();
+  if (t0 == 0) t0 = now;
+  if (now - t0 < x.limit && __hip_atomic_load(x.abort_dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    return false;
+  __hip_atomic_store(x.abort_dev, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(x.abort_host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  return true;
+}
+
+// Collects the halo words of stamp `want` into LDS; false when the wait ran
+// out or another block gave up.
+template <int NH>
+__device__ __forceinline__ bool collect(const ResComm& x, const u64* words, Halo<NH>& hp, unsigned want, float* c) {
+  u64 v[NH];
   refresh(hp.on);
   __builtin_amdgcn_s_sleep(kFirstPoll);
   long long t0 = 0;
   for (int spin = 0;; spin++) {
     bool all = true;
 #pragma unroll
-    for (int f = 0; f < F; f++)
+    for (int j = 0; j < NH; j++) v[j] = (hp.on >> j) & 1 ? peek(&elem(words, hp.q[j])) : (u64)want << 32;
 #pragma unroll
-      for (int j = 0; j < NH; j++) v[f][j] = (hp.on >> j) & 1 ? peek(&elem(w0 + f * fs, hp.q[j])) : (u64)want << 32;
-#pragma unroll
-    for (int f = 0; f < F; f++)
-#pragma unroll
-      for (int j = 0; j < NH; j++) all = all && (unsigned)(v[f][j] >> 32) == want;
+    for (int j = 0; j < NH; j++) all = all && (unsigned)(v[j] >> 32) == want;
     if (all) break;
-    if ((spin & 63) == 63 || x.limit == 0) {
-      const long long now = wall_clock64();
-      if (t0 == 0) t0 = now;
-      if (now - t0 >= x.limit ||
-          __hip_atomic_load(x.abort_dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-        __hip_atomic_store(x.abort_dev, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(x.abort_host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        return false;
-      }
-    }
+    if (give_up(x, spin, t0)) return false;
+  }
+#pragma unroll
+  for (int j = 0; j < NH; j++)
+    if ((hp.on >> j) & 1) c[hp.l[j]] = __uint_as_float((unsigned)v[j]);
+  return true;
+}
+
+// The exchange of two fields: a point's two values in one word, empty words
+// all ones (a pair of that NaN would wait until the limit).  Three copies in
+// turn: while step k is formed a block empties its words of the copy that step
+// k + 1 will use; every reader has taken step k - 2 from it by then, and none
+// looks for k + 1 before it has k, which the block publishes only when its
+// emptying stores have arrived.  Two stamped words a point move twice the
+// bytes: 2.8 against 2.3 us a step for the exchange alone on the 301x921 grid,
+// 4.3 against 3.1 on the 501x1501 one (one field is faster stamped, 1.75
+// against 2.0 us: it has no emptying to wait for).
+constexpr u64 kEmpty = ~(u64)0;
+__device__ __forceinline__ void put_pair(u64* p, float s, float g) {
+  __hip_atomic_store(p, ((u64)__float_as_uint(g) << 32) | __float_as_uint(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int NH>
+__device__ __forceinline__ bool collect_pairs(const ResComm& x, const u64* words, Halo<NH>& hp, float* s, float* g) {
+  u64 v[NH];
+  refresh(hp.on);
+  __builtin_amdgcn_s_sleep(kFirstPoll);
+  long long t0 = 0;
+  for (int spin = 0;; spin++) {
+    bool all = true;
+#pragma unroll
+    for (int j = 0; j < NH; j++) v[j] = (hp.on >> j) & 1 ? peek(&elem(words, hp.q[j])) : 0;
+#pragma unroll
+    for (int j = 0; j < NH; j++) all = all && v[j] != kEmpty;
+    if (all) break;
+    if (give_up(x, spin, t0)) return false;
   }
 #pragma unroll
   for (int j = 0; j < NH; j++)
     if ((hp.on >> j) & 1) {
-      c0[hp.l[j]] = __uint_as_float((unsigned)v[0][j]);
-      if constexpr (F == 2) c1[hp.l[j]] = __uint_as_float((unsigned)v[F - 1][j]);
+      s[hp.l[j]] = __uint_as_float((unsigned)v[j]);
+      g[hp.l[j]] = __uint_as_float((unsigned)(v[j] >> 32));
     }
   return true;
 }
@@ -310,9 +345,36 @@ __device__ __forceinline__ void ring_rows(const Place& p, float (&u)[R + 2], con
   if (p.wave + 1 < NW && p.row0 + R < p.w) u[R + 1] = ub[(2 * p.wave + 2) * 64 + p.lane];
 }
 
-template <int NW, int R>
-constexpr int halo_share() {
-  return (12 * kResTileZ + 12 * NW * R + 36 + 64 * NW - 1) / (64 * NW);
+// the most halo points of a tile of up to w columns per thread of NT
+constexpr int halo_share(int w, int NT) { return (12 * kResTileZ + 12 * w + 36 + NT - 1) / NT; }
+
+// This thread's share of the points a tile publishes: those within 6 of its edges.
+template <int NT, int NE>
+__device__ __forceinline__ void edge_points(const ResGrid& g, const Place& p, Halo<NE>& ep) {
+  const int rows = min(p.w, 12), cols = min(p.h, 12);  // edge rows; edge columns of the rows between
+  const int nrow = rows * p.h, ntot = nrow + (p.w - rows) * cols;
+  ep.on = 0;
+#pragma unroll
+  for (int j = 0; j < NE; j++) {
+    const int i = (int)threadIdx.x + j * NT;
+    int rx = 0, rz = 0;
+    if (i < nrow) {
+      const int r = i / p.h;
+      rz = i - r * p.h;
+      rx = r < 6 ? r : p.w - rows + r;
+    } else if (i < ntot) {
+      const int k = i - nrow, r = k % cols;
+      rx = 6 + k / cols;
+      rz = r < 6 ? r : p.h - cols + r;
+    }
+    const bool ok = i < ntot;
+    ep.q[j] = ok ? (unsigned)((p.x0 + rx) * g.ld + p.z0 + rz) : 0u;
+    ep.l[j] = ok ? (rx + 6) * LZ + rz + 6 : 0;
+    if (ok) ep.on |= 1u << j;
+  }
+}
+constexpr int edge_share(int w, int NT) {
+  return ((w <= 12 ? w * kResTileZ : 12 * kResTileZ + (w - 12) * 12) + NT - 1) / NT;
 }
 
 template <int P, int R, int NW>
@@ -366,9 +428,9 @@ __global__ __launch_bounds__(64 * NW) void k_resident_fwd(ResFwdArgs a) {
   }
   const bool band_tile = __ballot(inband != 0) != 0;  // uniform over the wave
   float* band = a.band + (long long)p.e * a.nt * a.bsize;
-  constexpr int NH = halo_share<NW, R>();
+  constexpr int NH = halo_share(NW * R, 64 * NW);
   Halo<NH> hp;
-  halo_points<NW, NH>(g, p, hp);
+  halo_points<64 * NW, NH>(g, p, hp);
   const long long words = (long long)a.E * a.fstride;  // of one parity
   __syncthreads();
   const bool chains = shared != 0;
@@ -420,7 +482,7 @@ __global__ __launch_bounds__(64 * NW) void k_resident_fwd(ResFwdArgs a) {
       }
     }
     if (has_src) sp.amp[it & 1][p.tid] = anext;
-    if (more && !collect<NH, 1>(a.x, words_now, 0, hp, stamp, cur, nullptr)) dead = 1;
+    if (more && !collect<NH>(a.x, words_now, hp, stamp, cur)) dead = 1;
     __syncthreads();
     if (dead) return;
   }
@@ -437,9 +499,12 @@ __global__ __launch_bounds__(64 * NW) void k_resident_fwd(ResFwdArgs a) {
 
 // The backward iteration with a field per half of the block: waves 0-7 the
 // source field (undamped step, subSource, imaging condition, band restore),
-// waves 8-15 the receiver field (damped step, injection).  Twice the waves
-// with half the chain each; the registers allow it up to 4 rows per wave.
-// Both halves run the same barriers.
+// waves 8-15 the receiver field (damped step, injection); a wave with both
+// fields has twice the chain and runs out of registers at 6 rows (301x921 4.8 us
+// a step, 501x1501 14).  Once both new fields are in LDS all 16 waves publish
+// the tile's edge as a list, a pair a thread, and collect the halo.  Both halves
+// run the same barriers.  (The forward kernel publishes from its registers: the
+// list there costs a barrier and gains nothing, 2.83 against 2.72 us.)
 template <int P, int R>
 struct BwdTile {
   static constexpr int NW = kResWaves, NX = NW * R + 12;
@@ -487,9 +552,9 @@ __device__ __forceinline__ void bwd_half(const ResBwdArgs& a, BwdTile<P, R>& t) 
   find_heads<R>(pt, n, p, head);
   float prv[R], rv[R], grad[R], bv[R];
   int bi[R];
-  unsigned edge = 0, inband = 0;
+  unsigned inband = 0;
   const float* band = a.band + (long long)p.e * a.nt * a.bsize;
-  unsigned q0 = (unsigned)((p.x0 + p.row0) * g.ld + iz);
+  const unsigned q0 = (unsigned)((p.x0 + p.row0) * g.ld + iz);
 #pragma unroll
   for (int k = 0; k < R; k++) {
     const int row = p.row0 + k;
@@ -500,22 +565,31 @@ __device__ __forceinline__ void bwd_half(const ResBwdArgs& a, BwdTile<P, R>& t) 
     bi[k] = SRC && in ? band_at(g, p.x0 + row, iz) : -1;
     if (bi[k] >= 0) inband |= 1u << k;
     bv[k] = bi[k] >= 0 && last - 1 >= a.it_min ? band[(long long)(last - 1) * a.bsize + bi[k]] : 0.f;
-    if (in && (p.lane <= 6 || p.lane > p.h - 6 || row < 6 || row >= p.w - 6)) edge |= 1u << k;
   }
   const bool band_tile = SRC && __ballot(inband != 0) != 0;  // uniform over the wave
-  constexpr int NH = halo_share<NW, R>();
+  constexpr int NT = 2 * 64 * NW, NH = halo_share(NW * R, NT), NE = edge_share(NW * R, NT);
   Halo<NH> hp;
-  halo_points<NW, NH>(g, p, hp);
-  const long long fs = (long long)a.E * a.fstride;  // words of one field
+  Halo<NE> ep;
+  halo_points<NT, NH>(g, p, hp);
+  edge_points<NT, NE>(g, p, ep);
+  const long long copy = (long long)a.E * a.fstride;  // words of one of the three copies
+  u64* words = a.x.buf + fo;
+  int turn = 0;  // the copy that the field being formed goes to
   __syncthreads();
   const bool chains = t.shared[F] != 0;
 
   for (int it = last; it >= a.it_min; it--) {
     const bool more = it - 1 >= a.it_min, more2 = it - 2 >= a.it_min;
-    refresh(edge);
     refresh(inband);
-    refresh(q0);
+    refresh(ep.on);
     head.fresh();
+    const int next = turn == 2 ? 0 : turn + 1;
+    if (more2) {
+#pragma unroll
+      for (int j = 0; j < NE; j++)
+        if ((ep.on >> j) & 1)
+          __hip_atomic_store(&elem(words + next * copy, ep.q[j]), kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     float win[R + 10], u[R + 2], rc[R];
     float anext = 0.f, weight = 0.f;
     if (has && (SRC ? more : more2)) anext = elem(amp + (long long)(it - 1) * amp_ld, pid);
@@ -532,8 +606,6 @@ __device__ __forceinline__ void bwd_half(const ResBwdArgs& a, BwdTile<P, R>& t) 
     }
     __syncthreads();
     ring_rows<NW, R>(p, u, t.ub[F]);
-    const unsigned stamp = a.x.base + (unsigned)(a.nt - it);
-    u64* words = a.x.buf + ((it & 1) * 2 + F) * fs + fo;
 #pragma unroll
     for (int k = 0; k < R; k++) {
       const int row = p.row0 + k;
@@ -551,14 +623,22 @@ __device__ __forceinline__ void bwd_half(const ResBwdArgs& a, BwdTile<P, R>& t) 
           if (band_tile && more && ((inband >> k) & 1)) v = bv[k];
         }
         prv[k] = c;
-        if (zin) {
-          if (more && ((edge >> k) & 1)) put(&elem(words, q0 + k * g.ld), v, stamp);
-          cur[(row + 6) * LZ + p.lane + 5] = v;
-        }
+        if (zin) cur[(row + 6) * LZ + p.lane + 5] = v;
       }
     }
     if (has) pt.amp[(it - 1) & 1][p.tid] = anext;
-    if (more && !collect<NH, 1>(a.x, words, 0, hp, stamp, cur, nullptr)) t.dead = 1;
+    if (more) {
+      __syncthreads();  // both fields' new edges are in LDS
+      // the emptied words have arrived before any word of this step leaves
+      __builtin_amdgcn_s_waitcnt(0);
+      asm volatile("" ::: "memory");
+      u64* now = words + turn * copy;
+#pragma unroll
+      for (int j = 0; j < NE; j++)
+        if ((ep.on >> j) & 1) put_pair(&elem(now, ep.q[j]), t.f[0][ep.l[j]], t.f[1][ep.l[j]]);
+      if (!collect_pairs<NH>(a.x, now, hp, t.f[0], t.f[1])) t.dead = 1;
+      turn = next;
+    }
     if (band_tile && more2) {
 #pragma unroll
       for (int k = 0; k < R; k++)
@@ -603,6 +683,9 @@ bool with_width(int w, F&& fn) {
     SWFWI_RES_ON(W8, 5, (k_resident_bwd<P, 5>), 64 * W16)
     SWFWI_RES_ON(W8, 6, (k_resident_bwd<P, 6>), 64 * W16)
     SWFWI_RES_ON(W8, 7, (k_resident_bwd<P, 7>), 64 * W16)
+    SWFWI_RES_ON(W8, 8, (k_resident_bwd<P, 8>), 64 * W16)
+    SWFWI_RES_ON(W8, 9, (k_resident_bwd<P, 9>), 64 * W16)
+    SWFWI_RES_ON(W8, 10, (k_resident_bwd<P, 10>), 64 * W16)
   } else {
     SWFWI_RES_ON(W8, 1, (k_resident_fwd<P, 1, W8>), 64 * W8)
     SWFWI_RES_ON(W8, 2, (k_resident_fwd<P, 2, W8>), 64 * W8)
