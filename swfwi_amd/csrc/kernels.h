@@ -113,6 +113,20 @@ struct BwdStepArgs {
   int split = 0;                  // launch the two fields as separate blocks (small batches)
 };
 
+// Work of the strip-walking forward step: strips of h outputs along z, chunks
+// of `rows` rows along x, and the points of each unit (chunk * nstrip + strip)
+// as (row, z, id, 0), by row and id, at most 64.
+struct UnitPoints {
+  const int* ptr = nullptr;
+  const int4* items = nullptr;
+};
+constexpr int kMarchStrip = 116, kMarchPts = 64;
+struct MarchMap {
+  int nstrip = 0, h = 0, nchunk = 0, rows = 0;
+  int shared = 0;  // entries back to back (they share models) or one after the other
+  UnitPoints src, rec;
+};
+
 // ---- launchers (all asynchronous on `stream`) -------------------------------
 // Tile widths the step kernels are instantiated for, and the tile count along
 // x of a padded grid for one of them.
@@ -123,6 +137,8 @@ int tile_count_x(int nx, int tile_x);
 void launch_fwd_step(const FwdStepArgs& a, int nentries, bool damped, int precision, hipStream_t stream,
                      int chunk = 0);
 void launch_bwd_step(const BwdStepArgs& a, int nentries, int precision, hipStream_t stream, int chunk = 0);
+
+void launch_fwd_march(const FwdStepArgs& a, const MarchMap& m, int nentries, int precision, hipStream_t stream);
 
 void launch_fill(float* p, long long n, float v, hipStream_t s);
 void launch_fill_d(double* p, long long n, double v, hipStream_t s);

@@ -370,6 +370,55 @@ int Propagator::xcorr_range(float dt, int nt, std::vector<float>& weights) {
   return it_min;
 }
 
+const Propagator::MarchLayout* Propagator::march_layout(int E) {
+  const int ux = g_.nxpad - 2 * kHalo, uz = g_.nzpad - 2 * kHalo;
+  if (tile_override_ || g_.npts() >= (1LL << 29)) return nullptr;
+  const int nstrip = (uz + kMarchStrip - 1) / kMarchStrip;
+  const long long strip_rows = (long long)E * nstrip * ux;
+  // Measured (microseconds a step, tiled kernel -> strip walks of 14 / 22 rows,
+  // exact mode): 12 entries of 301x921 (35000 strip rows) 16.1 -> 15.4 / 16.6,
+  // 60 members of 201x301 (41000) 20.8 -> 17.1 / 17.7, 16 of 301x921 (47000)
+  // 19.9 -> 18.5 / 19.4, 8 of 501x1501 (62000) 21.6 -> 21.9 / 20.6, 60 of
+  // 301x921 (177000) 56 -> 47.3 / 46.3 (30 rows 47.1, 10 rows 50.6); below, too
+  // few waves walk too long: 22 entries of 201x301 (15000) 10.1 -> 12.1 (9.8 at
+  // 8 rows), 6 of 301x921 (18000) 10.3 -> 12.1.
+  if (strip_rows < kMarchFrom) return nullptr;
+  const int rows = strip_rows < 2 * kMarchFrom ? 14 : 22;
+  for (const auto& l : march_layouts_)
+    if (l->m.rows == rows) return l->fits ? l.get() : nullptr;
+  auto l = std::make_unique<MarchLayout>();
+  l->m.nstrip = nstrip;
+  l->m.h = 2 * ((uz + 2 * nstrip - 1) / (2 * nstrip));
+  l->m.rows = rows;
+  l->m.nchunk = (ux + rows - 1) / rows;
+  hipStream_t s = stream();
+  l->fits = true;
+  auto bucket = [&](const std::vector<long long>& idx, DBuf<int>& dptr, DBuf<int4>& ditems) {
+    std::vector<std::vector<int4>> lists((size_t)l->m.nstrip * l->m.nchunk);
+    for (size_t i = 0; i < idx.size(); i++) {
+      const int x = (int)(idx[i] / g_.ld), z = (int)(idx[i] % g_.ld);
+      lists[(size_t)((x - kHalo) / rows) * nstrip + (z - kHalo) / l->m.h].push_back(make_int4(x, z, (int)i, 0));
+    }
+    std::vector<int> ptr(1, 0);
+    std::vector<int4> items;
+    for (auto& v : lists) {
+      std::stable_sort(v.begin(), v.end(), [](const int4& p, const int4& q) { return p.x < q.x; });
+      items.insert(items.end(), v.begin(), v.end());
+      ptr.push_back((int)items.size());
+      if ((int)v.size() > kMarchPts) l->fits = false;
+    }
+    dptr.upload(ptr, s);
+    ditems.upload(items, s);
+    SWFWI_HIP(hipStreamSynchronize(s));  // the host vectors end here
+  };
+  bucket(src_idx_, l->sptr, l->sitems);
+  bucket(rec_idx_, l->rptr, l->ritems);
+  l->m.src = UnitPoints{l->sptr.get(), l->sitems.get()};
+  l->m.rec = UnitPoints{l->rptr.get(), l->ritems.get()};
+  march_layouts_.push_back(std::move(l));
+  return march_layouts_.back()->fits ? march_layouts_.back().get() : nullptr;
+}
+
 std::vector<Propagator::FwdLaunch> Propagator::plan_forward(Fields& fw) const {
   // Buffer rotation of a forward run: b holds p(0) (the injected zero field),
   // a holds p(-1) = 0; each step writes next over prev.
@@ -390,7 +439,13 @@ std::vector<Propagator::FwdLaunch> Propagator::plan_forward(Fields& fw) const {
 }
 
 void Propagator::forward_body(int E, const float* rv, long long rvstride, const Sources& src, float* dcal,
-                              float* band, float* fa, float* fb, int rvdiv, int w, hipStream_t s) {
+                              float* band, float* fa, float* fb, int rvdiv, int w, hipStream_t s,
+                              const MarchLayout* march) {
+  MarchMap map;
+  if (march) {
+    map = march->m;
+    map.shared = rvstride == 0 || rvdiv > 1;
+  }
   const long long np = g_.npts();
   const int nt = g_.nt, ng = g_.ng();
   launch_fill(fa, (long long)E * np, 0.f, s);
@@ -427,7 +482,10 @@ void Propagator::forward_body(int E, const float* rv, long long rvstride, const 
     a.inj.t = it + 1 < nt ? it + 1 : -1;
     a.rec.out = dcal ? dcal + (long long)it * ng : nullptr;
     a.band = band ? band + (long long)it * g_.bsize : nullptr;
-    launch_fwd_step(a, E, true, prec_, s, block_chunk(0, E, rvstride, rvdiv));
+    if (march)
+      launch_fwd_march(a, map, E, prec_, s);
+    else
+      launch_fwd_step(a, E, true, prec_, s, block_chunk(0, E, rvstride, rvdiv));
   }
   SWFWI_HIP(hipGetLastError());
 }
@@ -446,12 +504,15 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
     fwd_point_updates += (double)E * (g_.nxpad - 2 * kHalo) * (g_.nzpad - 2 * kHalo) * g_.nt;
     return;
   }
+  const bool lanes = E >= 2 && E <= kLanes && band == nullptr;
   // tile widths for this batch, chosen now while the workspace is free
   // (backward() runs on the state this forward leaves behind)
-  const int tw = tile_choice(0, E, rv, rvstride, rvdiv, w, true);
+  const MarchLayout* march = lanes ? nullptr : march_layout(E);
+  const int tw = tile_choice(0, E, rv, rvstride, rvdiv, w, !march);
   tile_choice(1, E, rv, rvstride, rvdiv, w, true);
   const uintptr_t key[] = {1,
                            (uintptr_t)tw,
+                           (uintptr_t)(march ? march->m.rows : 0),
                            (uintptr_t)E,
                            (uintptr_t)rv,
                            (uintptr_t)rvstride,
@@ -468,12 +529,11 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
                            (uintptr_t)w.c.get(),
                            (uintptr_t)w.d.get(),
                            (uintptr_t)prec_};
-  const bool lanes = E >= 2 && E <= kLanes && band == nullptr;
   if (!lanes) {
     hipStream_t s = stream();
     run_maybe_graph(
         std::vector<uintptr_t>(std::begin(key), std::end(key)), E, 0, g_.nt,
-        [&] { forward_body(E, rv, rvstride, src, dcal, band, w.a.get(), w.b.get(), rvdiv, tw, s); }, s);
+        [&] { forward_body(E, rv, rvstride, src, dcal, band, w.a.get(), w.b.get(), rvdiv, tw, s, march); }, s);
   } else {
     // entry e as a one-entry run on lane e, over its own slice of the batch's
     // buffers (the same rotation, so the batch's final state is unchanged);

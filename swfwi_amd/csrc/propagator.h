@@ -192,6 +192,12 @@ class Propagator {
   Propagator& operator=(const Propagator&) = delete;
 
  private:
+  struct MarchLayout {
+    MarchMap m;
+    DBuf<int> sptr, rptr;
+    DBuf<int4> sitems, ritems;
+    bool fits = false;  // no unit holds more than kMarchPts points
+  };
   // one launch of a forward time loop: step `it` writes next over prev
   struct FwdLaunch {
     int it;
@@ -202,7 +208,7 @@ class Propagator {
   // one forward run of E entries on stream s: p(-1) in fa, p(0) in fb, the
   // two buffers then alternate (the rotation plan_forward describes)
   void forward_body(int E, const float* rv, long long rvstride, const Sources& src, float* dcal, float* band,
-                    float* fa, float* fb, int rvdiv, int w, hipStream_t s);
+                    float* fa, float* fb, int rvdiv, int w, hipStream_t s, const MarchLayout* march = nullptr);
   void backward_body(int E, const float* rv, long long rvstride, const Sources& src, const float* vsrc,
                      long long vstride, const float* band, float* grad, long long gstride, Fields& fw, int rvdiv,
                      int it_min, const std::vector<float>& wts, int w);
@@ -220,6 +226,9 @@ class Propagator {
     ResPoints rec() const { return ResPoints{rptr.get(), ritems.get()}; }
   };
   ResLayout& res_layout(const ResTiles& t);
+  // The strip-walking forward step: whether a batch takes it, and its work
+  // (strips, chunks, points by unit) for a batch of E entries.
+  const MarchLayout* march_layout(int E);
   ResGrid res_grid(const ResTiles& t) const;
   void res_begin(int kind, int E, ResComm& x);  // call with the device's lock held
   bool res_end(int kind, long long steps, hipEvent_t t0);
@@ -235,6 +244,7 @@ class Propagator {
   // the measured width rule (index into kTileWidths) by batch size, or the override
   int fixed_width(int kind, int E) const;
   static constexpr int kGraphMaxEntries = 8;
+  static constexpr long long kMarchFrom = 30000;  // strip rows (strips x rows of x over the batch)
   // A forward batch of 2..kLanes entries without a band (line-search trial
   // runs) runs as one-entry loops side by side, lane e on its own stream:
   // measured on the 301x921 grid, two one-entry loops on two streams take
@@ -286,6 +296,7 @@ class Propagator {
   static constexpr double kResWaitUs = 5e5;
   double ticks_per_us_ = 100;  // of the kernels' wall clock
   std::vector<std::unique_ptr<ResLayout>> res_layouts_;
+  std::vector<std::unique_ptr<MarchLayout>> march_layouts_;  // by chunk length
   std::vector<long long> src_idx_, rec_idx_;  // grid indices of the points
   int res_cap_[2][2] = {{-1, -1}, {-1, -1}};  // [kind][precision] blocks on the chip at once
   DBuf<unsigned long long> xbuf_[2];  // exchange words, forward and backward
