@@ -42,6 +42,9 @@ struct NetGeom {
   const float* r;     // 1 / vel_t of entry e at r + (e / rdiv) * rstride, same layout
   long long rstride;
   int rdiv;
+  // When given (device, entries long): entry e reads field, model and target
+  // pick[e] of their stacks.  What is written stays entry after entry.
+  const int* pick = nullptr;
 };
 
 // Device weights in the layouts the kernels read: every layer's BF16 MFMA
@@ -60,19 +63,24 @@ void net_pack(const float* theta, const NetDev& w, hipStream_t s);
 void net_apply(const float* p, float* y, const NetGeom& g, const NetDev& w, hipStream_t s);
 // p += y over the region
 void net_add(float* p, const float* y, const NetGeom& g, hipStream_t s);
-// Loss of a batch: r = p + y - t over the region, dy = 2 r / count, the sum
-// of r^2 (FP64) into *loss (device), dy zero outside the region.
-void net_loss(const float* p, const float* y, const float* t, float* dy, const NetGeom& g, double* loss_parts,
-              int nparts, hipStream_t s);
-// d loss / d weights: per-block partials reduced in a fixed order into grad.
-// Returns nothing; `parts` must hold net_backward_blocks(g) * kNetParams floats.
-long long net_backward_blocks(const NetGeom& g);
-void net_backward(const float* p, const float* dy, const NetGeom& g, const NetDev& w, float* parts, float* grad,
-                  hipStream_t s);
-// Adam (step >= 1): theta -= lr * mhat / (sqrt(vhat) + eps)
-void net_adam(float* theta, const float* grad, float* m, float* v, int step, float lr, float b1, float b2, float eps,
+// Loss of a batch: r = p + net(p) - t over the region, dy = 2 r / count
+// there (dy elsewhere untouched), the sum of r^2 (FP64) of every block into
+// loss_parts, which must hold net_loss_blocks(g).
+long long net_loss_blocks(const NetGeom& g);
+void net_loss(const float* p, const float* t, float* dy, const NetGeom& g, const NetDev& w, double* loss_parts,
               hipStream_t s);
-void net_reduce_parts(const double* parts, int nparts, double* out, hipStream_t s);
+// d loss / d weights, every block's part of it; `parts` must hold
+// net_backward_blocks(g) * kNetParams floats.
+long long net_backward_blocks(const NetGeom& g);
+void net_backward(const float* p, const float* dy, const NetGeom& g, const NetDev& w, float* parts, hipStream_t s);
+// The parts summed in a fixed order: the gradient and the loss ...
+void net_reduce(const float* parts, long long nblocks, float* grad, const double* loss_parts, long long nloss,
+                double* loss, hipStream_t s);
+// ... or the loss and Adam's step (step >= 1) on the gradient,
+// theta -= lr * mhat / (sqrt(vhat) + eps), with the packed weights renewed
+void net_adam(const float* parts, long long nblocks, const double* loss_parts, long long nloss, double* loss,
+              float* theta, float* m, float* v, const NetDev& w, int step, float lr, float b1, float b2, float eps,
+              hipStream_t s);
 
 // Host handle: weights (FP32 master copy + packed device forms), Adam state
 // and scratch for training on stacks of coarse fields.
@@ -88,8 +96,6 @@ class ConvNet {
   // sum_r r^2 before the step into *loss_dev (device, FP64).
   void train_step(const float* in, const float* target, const NetGeom& g, float lr, double* loss_dev,
                   hipStream_t s);
-  // loss sum into *loss_dev and the weight gradient, without a wait
-  void loss_grad_async(const float* in, const float* target, const NetGeom& g, double* loss_dev, hipStream_t s);
   // loss and gradient without an update (for checks)
   double loss_grad(const float* in, const float* target, const NetGeom& g, float* grad_host, hipStream_t s);
   int steps() const { return step_; }
@@ -102,9 +108,10 @@ class ConvNet {
 
  private:
   void repack(hipStream_t s);
+  void grad_parts(const float* in, const float* target, const NetGeom& g, hipStream_t s);
   DBuf<float> theta_, m_, v_, grad_, w3_;
   DBuf<uint16_t> w1a_, w2b_, w3a_, w2p_;
-  DBuf<float> y_, dy_, parts_, din_, dr_, dtgt_, bin_, br_, btgt_;
+  DBuf<float> dy_, parts_, din_, dr_, dtgt_;
   NetGeom dg_{};
   int dn_ = 0;
   DBuf<double> lparts_, lsum_;

@@ -44,6 +44,9 @@ constexpr int kNH2 = kH2 * kH2;  // 324
 constexpr int kGroups1 = kNH1 / 16;         // 25 groups of 16 layer-1 points
 constexpr int kGroups2 = (kNH2 + 15) / 16;  // 21 groups of 16 layer-2 points
 static_assert(kNH1 % 16 == 0, "layer-1 points fill whole groups");
+constexpr int kB = 512;          // threads of the backward kernel
+constexpr int kH1Pitch = 408;    // channel pitch of the transposed layer 1: 16-byte rows, 12 banks apart
+constexpr int kDz2Pitch = 264;   // and of the transposed dz2: 4 channels 16 banks apart
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -58,9 +61,8 @@ __device__ __host__ __forceinline__ uint16_t bf16_bits(unsigned u) {  // round t
 __device__ __forceinline__ uint16_t bf16_of(float x) { return bf16_bits(__float_as_uint(x)); }
 __device__ __forceinline__ float f32_of(uint16_t h) { return __uint_as_float((unsigned)h << 16); }
 
-// accumulator item v of lane l holds D[row][col]
+// accumulator item v of lane l holds D[row][l % 16]
 __device__ __forceinline__ int d_row(int l, int v) { return 4 * (l >> 4) + v; }
-__device__ __forceinline__ int d_col(int l) { return l & 15; }
 
 // (a, b) rounded to BF16 (nearest even) by the hardware conversion
 // (v_cvt_pk_bf16_f32), a in the low half; the same bits as bf16_of for
@@ -91,6 +93,7 @@ __device__ __forceinline__ float ld_at(const float* base, unsigned i) {
 
 struct TileMap {
   int e, ox, oz;  // entry, tile origin (global padded coords)
+  int in;         // the entry's place in the stacks it reads
 };
 
 // tiles over the region grown by `margin` cells on every side
@@ -102,21 +105,33 @@ __device__ __forceinline__ TileMap tile_of(const NetGeom& g, int margin) {
   const int t = blockIdx.x - m.e * per;
   m.ox = g.x0 - margin + (t / tz) * kTile;
   m.oz = g.z0 - margin + (t % tz) * kTile;
+  m.in = g.pick ? g.pick[m.e] : m.e;
   return m;
 }
 
-// Shared forward work of a tile.  sx[kP*kP]: staged (p, r p) as BF16 pairs
-// (p in the low half); h1[kNH1*16]: layer 1 (BF16).  Layer 2 then goes to
-// h2[kNH2*16] (BF16) when h2 is given and through layer 3 into
-// u[9][kNH2] (FP32) when u is given.  Returns false, with nothing computed,
-// when `skip_zero` is set and the staged input is zero everywhere (the
-// network, ReLU without biases, then gives exactly zero).
-__device__ bool forward_tile(const float* __restrict__ p, const float* __restrict__ r, const NetGeom& g,
-                             const TileMap& m, const NetDev& w, unsigned* sx, uint16_t* h1, uint16_t* h2, float* u,
-                             bool skip_zero) {
+// Layer 2 of the groups of a wave of kNT threads' block: h2[4 (l / 16) + v]
+// of the group's point l % 16
+template <int kNT>
+struct Hidden {
+  static constexpr int kMax = (kGroups2 + kNT / 64 - 1) / (kNT / 64);  // groups per wave, at most
+  bf16x4 h[kMax];
+};
+
+// Shared forward work of a tile, by kNT threads.  sx[kP*kP]: staged (p, r p)
+// as BF16 pairs (p in the low half); h1[kNH1*16]: layer 1 (BF16), with
+// kTrans also channel by channel in h1t[16][kH1Pitch].  Layer 2 is left in
+// `hid` and goes through layer 3 into u[9][kNH2] (FP32) when u is given.
+// Returns false, with nothing computed, when `skip_zero` is set and the
+// staged input is zero everywhere (the network, ReLU without biases, then
+// gives exactly zero).
+template <int kNT, bool kTrans>
+__device__ __forceinline__ bool forward_tile(const float* __restrict__ p, const float* __restrict__ r,
+                                             const NetGeom& g, const TileMap& m, const NetDev& w, unsigned* sx,
+                                             uint16_t* h1, uint16_t* h1t, float* u, bool skip_zero,
+                                             Hidden<kNT>& hid) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int nonzero = 0;
-  for (int q = tid; q < kP * kP; q += kT) {
+  for (int q = tid; q < kP * kP; q += kNT) {
     const int x = m.ox - 3 + q / kP, z = m.oz - 3 + q % kP;
     const bool in = x >= 0 && x < g.nx && z >= 0 && z < g.nz;
     const unsigned o = (unsigned)(x * g.nz + z);
@@ -128,6 +143,15 @@ __device__ bool forward_tile(const float* __restrict__ p, const float* __restric
   const int kq = lane >> 4;  // this lane's K quarter
   const bf16x4 a1a = *reinterpret_cast<const bf16x4*>(w.w1a + lane * 4);
   const bf16x4 a1b = *reinterpret_cast<const bf16x4*>(w.w1a + (64 + lane) * 4);
+  // layer 2's operands (see there): a block that is the only one of its CU
+  // takes them with the others, as no other's work covers their way from L2
+  // (kTrans); many blocks a CU load them late, for the registers
+  hbf16x8 a2p[5];
+  auto load_a2p = [&] {
+#pragma unroll
+    for (int q = 0; q < 5; q++) a2p[q] = *reinterpret_cast<const hbf16x8*>(w.w2p + (q * 64 + lane) * 8);
+  };
+  if constexpr (kTrans) load_a2p();
   if (!__syncthreads_or(nonzero) && skip_zero) return false;  // block-uniform
   // layer 1: lane's B items are (p, r p) at taps 2 kq and 2 kq + 1 (first
   // product) and at tap 8 (second product: k = 16 + 4 kq + v, of which only
@@ -137,10 +161,10 @@ __device__ bool forward_tile(const float* __restrict__ p, const float* __restric
     const int t0 = 2 * kq, t1 = 2 * kq + 1;
     const int o0 = (t0 / 3 - 1) * kP + (t0 % 3 - 1), o1 = (t1 / 3 - 1) * kP + (t1 % 3 - 1);
     const int o8 = kP + 1;
-    constexpr int kMaxG1 = (kGroups1 + kT / 64 - 1) / (kT / 64);  // groups per wavefront, at most
+    constexpr int kMaxG1 = (kGroups1 + kNT / 64 - 1) / (kNT / 64);  // groups per wavefront, at most
 #pragma unroll
     for (int i = 0; i < kMaxG1; i++) {
-      const int grp = wave + i * (kT / 64);
+      const int grp = wave + i * (kNT / 64);
       if (grp >= kGroups1) break;  // wave-uniform
       const int q = grp * 16 + (lane & 15);
       const int s = (q / kH1 + 1) * kP + (q % kH1 + 1);  // staged centre
@@ -152,7 +176,12 @@ __device__ bool forward_tile(const float* __restrict__ p, const float* __restric
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
       acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1a, b0.b, acc, 0, 0, 0);
       acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1b, b1.b, acc, 0, 0, 0);
-      *reinterpret_cast<bf16x4*>(h1 + q * kNetC + 4 * kq) = relu_bf16(acc);  // channels 4 kq .. 4 kq + 3
+      const bf16x4 hv = relu_bf16(acc);
+      *reinterpret_cast<bf16x4*>(h1 + q * kNetC + 4 * kq) = hv;  // channels 4 kq .. 4 kq + 3
+      if constexpr (kTrans) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) h1t[(4 * kq + v) * kH1Pitch + q] = (uint16_t)hv[v];
+      }
     }
   }
   __syncthreads();
@@ -164,9 +193,7 @@ __device__ bool forward_tile(const float* __restrict__ p, const float* __restric
   // chain: a 16x16x16 product that read the accumulator of a 16x16x32 one
   // issued just before it has given wrong sums on gfx950 (no wait states are
   // inserted between the two).
-  hbf16x8 a2p[5];
-#pragma unroll
-  for (int q = 0; q < 5; q++) a2p[q] = *reinterpret_cast<const hbf16x8*>(w.w2p + (q * 64 + lane) * 8);
+  if constexpr (!kTrans) load_a2p();
   const bf16x4 a3 = *reinterpret_cast<const bf16x4*>(w.w3a + lane * 4);
   const int khalf = kq >> 1, kc = 8 * (kq & 1);  // this lane's tap of the pair, first channel
   // B operand of product q < 4: channels kc .. kc + 7 of tap 2q + khalf of
@@ -182,11 +209,11 @@ __device__ bool forward_tile(const float* __restrict__ p, const float* __restric
   // layer 2 per group, its result kept in registers; then (apply) layer 3
   // into u, which may share its memory with h1: every layer-2 read of h1 is
   // done at the barrier between the two
-  constexpr int kMaxG = (kGroups2 + kT / 64 - 1) / (kT / 64);  // groups per wavefront, at most
-  bf16x4 hbs[kMaxG];
+  constexpr int kMaxG = Hidden<kNT>::kMax;
+  bf16x4* const hbs = hid.h;
 #pragma unroll
   for (int i = 0; i < kMaxG; i++) {
-    const int grp = wave + i * (kT / 64);
+    const int grp = wave + i * (kNT / 64);
     if (grp >= kGroups2) break;                // wave-uniform
     const int qa = grp * 16 + (lane & 15);     // this lane's point
     const int qs = qa < kNH2 ? qa : kNH2 - 1;  // points past the region read a valid one
@@ -199,13 +226,12 @@ __device__ bool forward_tile(const float* __restrict__ p, const float* __restric
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2p[q], b, acc, 0, 0, 0);
     }
     hbs[i] = relu_bf16(acc);  // h2[4 kq + v][qa]
-    if (h2 && qa < kNH2) *reinterpret_cast<bf16x4*>(h2 + qa * kNetC + 4 * kq) = hbs[i];
   }
   if (u) {  // uniform over the grid
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kMaxG; i++) {
-      const int grp = wave + i * (kT / 64);
+      const int grp = wave + i * (kNT / 64);
       if (grp >= kGroups2) break;
       const int qa = grp * 16 + (lane & 15);
       f32x4 y3 = {0.f, 0.f, 0.f, 0.f};
@@ -217,47 +243,9 @@ __device__ bool forward_tile(const float* __restrict__ p, const float* __restric
           if (4 * kq + v < 9) ub[v * kNH2] = y3[v];
       }
     }
+    __syncthreads();
   }
-  __syncthreads();
   return true;
-}
-
-// 8 waves per SIMD (63 VGPRs, no spills): 5-6% faster than the 7 the
-// compiler picks by itself (58 VGPRs plus the accumulators)
-__global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(8))) void k_net_apply(const float* __restrict__ p_all, float* __restrict__ y_all,
-                                                  NetGeom g, NetDev w) {
-  __shared__ unsigned sx[kP * kP];
-  // h1 (layer 1) and then u (layer 3): u overwrites h1 after layer 2
-  __shared__ __align__(16) uint16_t h1[kNH1 * kNetC];
-  static_assert(9 * kNH2 * sizeof(float) <= kNH1 * kNetC * sizeof(uint16_t), "u fits in h1");
-  float* u = reinterpret_cast<float*>(h1);
-  const TileMap m = tile_of(g, 0);
-  const float* p = p_all + (long long)m.e * g.stride;
-  const float* r = g.r + (long long)(m.e / g.rdiv) * g.rstride;
-  const int x = threadIdx.x / kTile, z = threadIdx.x % kTile;
-  const int gx = m.ox + x, gz = m.oz + z;
-  float* yo = y_all + (long long)m.e * g.stride + (long long)gx * g.nz + gz;
-  const bool out = gx < g.x1 && gz < g.z1;
-  if (!forward_tile(p, r, g, m, w, sx, h1, nullptr, u, true)) {
-    if (out) *yo = 0.f;
-    return;
-  }
-  if (!out) return;
-  float y = 0.f;
-#pragma unroll
-  for (int t = 0; t < 9; t++) y += u[t * kNH2 + (x + 1 + t / 3 - 1) * kH2 + (z + 1 + t % 3 - 1)];
-  *yo = y;
-}
-
-__global__ void k_net_add(float* p_all, const float* y_all, NetGeom g) {
-  const long long per = (long long)(g.x1 - g.x0) * (g.z1 - g.z0);
-  const long long n = per * g.entries;
-  for (long long i = blockIdx.x * (long long)kT + threadIdx.x; i < n; i += (long long)gridDim.x * kT) {
-    const long long e = i / per, r = i - e * per;
-    const int x = g.x0 + (int)(r / (g.z1 - g.z0)), z = g.z0 + (int)(r % (g.z1 - g.z0));
-    const long long o = e * g.stride + (long long)x * g.nz + z;
-    p_all[o] += y_all[o];
-  }
 }
 
 __device__ __forceinline__ double block_sum_d(double v, double* red) {
@@ -271,160 +259,356 @@ __device__ __forceinline__ double block_sum_d(double v, double* red) {
   return s;
 }
 
-// r = p + y - t over the region; dy = 2 r / count; per-block sum of r^2
-__global__ void k_net_loss(const float* p, const float* y, const float* t, float* dy, NetGeom g, double inv_count,
-                           double* parts) {
-  __shared__ double red[kT / 64];
+// What k_net_apply needs to form the loss in place of the output
+struct LossArgs {
+  const float* t;    // targets
+  double inv_count;  // 1 / (region points x entries)
+  double* parts;     // a block's sum of r^2
+};
+
+// y = net(p) over the region; with kLoss r = p + y - t is formed where y is
+// still in a register: y_all takes dy = 2 r / count and the block's sum of
+// r^2 goes to l.parts.
+// 8 waves per SIMD (63 VGPRs, no spills): 5-6% faster than the 7 the
+// compiler picks by itself (58 VGPRs plus the accumulators)
+template <bool kLoss>
+__global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(8))) void k_net_apply(
+    const float* __restrict__ p_all, float* __restrict__ y_all, NetGeom g, NetDev w, LossArgs l) {
+  __shared__ unsigned sx[kP * kP];
+  // h1 (layer 1) and then u (layer 3): u overwrites h1 after layer 2
+  __shared__ __align__(16) uint16_t h1[kNH1 * kNetC];
+  static_assert(9 * kNH2 * sizeof(float) <= kNH1 * kNetC * sizeof(uint16_t), "u fits in h1");
+  float* u = reinterpret_cast<float*>(h1);
+  const TileMap m = tile_of(g, 0);
+  const float* p = p_all + (long long)m.in * g.stride;
+  const float* r = g.r + (long long)(m.in / g.rdiv) * g.rstride;
+  const int x = threadIdx.x / kTile, z = threadIdx.x % kTile;
+  const int gx = m.ox + x, gz = m.oz + z;
+  const long long at = (long long)gx * g.nz + gz;
+  float* yo = y_all + (long long)m.e * g.stride + at;
+  const bool out = gx < g.x1 && gz < g.z1;
+  Hidden<kT> hid;
+  const bool some = forward_tile<kT, false>(p, r, g, m, w, sx, h1, nullptr, u, true, hid);
+  float y = 0.f;
+  if (some && out) {
+#pragma unroll
+    for (int t = 0; t < 9; t++) y += u[t * kNH2 + (x + 1 + t / 3 - 1) * kH2 + (z + 1 + t % 3 - 1)];
+  }
+  if constexpr (kLoss) {
+    __shared__ double red[kT / 64];
+    double acc = 0;
+    if (out) {
+      const float res = p[at] + y - l.t[(long long)m.in * g.stride + at];
+      *yo = (float)(2.0 * res * l.inv_count);
+      acc = (double)res * res;
+    }
+    const double sum = block_sum_d(acc, red);
+    if (threadIdx.x == 0) l.parts[blockIdx.x] = sum;
+  } else if (out) {
+    *yo = y;
+  }
+}
+
+__global__ void k_net_add(float* p_all, const float* y_all, NetGeom g) {
   const long long per = (long long)(g.x1 - g.x0) * (g.z1 - g.z0);
   const long long n = per * g.entries;
-  double acc = 0;
   for (long long i = blockIdx.x * (long long)kT + threadIdx.x; i < n; i += (long long)gridDim.x * kT) {
     const long long e = i / per, r = i - e * per;
     const int x = g.x0 + (int)(r / (g.z1 - g.z0)), z = g.z0 + (int)(r % (g.z1 - g.z0));
     const long long o = e * g.stride + (long long)x * g.nz + z;
-    const float res = p[o] + y[o] - t[o];
-    dy[o] = (float)(2.0 * res * inv_count);
-    acc += (double)res * res;
+    p_all[o] += y_all[o];
   }
-  const double s = block_sum_d(acc, red);
-  if (threadIdx.x == 0) parts[blockIdx.x] = s;
+}
+
+// A chain of FP32 products D += fa(a(k, i)) fb(b(k, i)), batches k = kFrom ..
+// kTo - 1 of kLen, in order: a batch's operands are read (a, b) while the one
+// before it is multiplied, and made floats (fa, fb) where they are used.  The
+// compiler by itself reads each where it is used: 170 cycles a product in
+// place of the 32 that it takes.
+template <int kFrom, int kTo, int kLen, class A, class B, class FA, class FB>
+__device__ __forceinline__ f32x4 mfma_chain(f32x4 acc, A a, B b, FA fa, FB fb) {
+  decltype(a(0, 0)) va[2][kLen];
+  decltype(b(0, 0)) vb[2][kLen];
+#pragma unroll
+  for (int i = 0; i < kLen; i++) va[0][i] = a(kFrom, i), vb[0][i] = b(kFrom, i);
+#pragma unroll
+  for (int k = kFrom; k < kTo; k++) {
+    const int c = (k - kFrom) & 1, n = c ^ 1;
+    __builtin_amdgcn_sched_barrier(0);
+    if (k + 1 < kTo) {
+#pragma unroll
+      for (int i = 0; i < kLen; i++) va[n][i] = a(k + 1, i), vb[n][i] = b(k + 1, i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kLen; i++)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fa(va[c][i]), fb(vb[c][i]), acc, 0, 0, 0);
+  }
+  return acc;
 }
 
 // d loss / d weights of one tile: recompute the forward pieces, then
-//   dW3[t][c] = sum_tile dy(x) h2[c](x + o_t)
+//   dW3[t][c] = sum_tile dy(x) h2[c](x + o_t)                   (FP32 MFMA)
 //   dz2[c](x') = relu'(z2) sum_t W3[t][c] dy(x' - o_t)        (tile + 1)
-//   dW2[t][ci][co] = sum_tile h1[ci](x + o_t) dz2[co](x)        (MFMA, K = tile points)
-//   dz1[ci](x) = relu'(z1) sum_t sum_co W2[t][ci][co] dz2[co](x - o_t)   (MFMA)
-//   dW1[t][k][c] = sum_tile in_k(x + o_t) dz1[c](x), in_0 = p, in_1 = r p
+//   dW2[t][ci][co] = sum_tile h1[ci](x + o_t) dz2[co](x)        (BF16 MFMA, K = tile points)
+//   dz1[ci](x) = relu'(z1) sum_t sum_co W2[t][ci][co] dz2[co](x - o_t)   (BF16 MFMA)
+//   dW1[t][k][c] = sum_tile in_k(x + o_t) dz1[c](x), in_0 = p, in_1 = r p  (FP32 MFMA)
 // into parts[block][kNetParams].  The forward values enter as the forward
-// products saw them: inputs, h1, h2 and W3 rounded to BF16.
-__global__ __launch_bounds__(kT) void k_net_backward(const float* __restrict__ p_all, const float* __restrict__ dy_all,
+// products saw them: inputs, h1, h2 and W3 rounded to BF16; dy and dz1 are
+// FP32 and stay so (v_mfma_f32_16x16x4_f32: lane l supplies A[l % 16][l / 16]
+// and B[l / 16][l % 16], D as the others).
+//
+// A minibatch is about one tile per CU, so a block's serial chain is the
+// kernel's time: 8 waves share every stage, and what was a serial sum over
+// the tile's points in each of a few threads (dW1, dW3) is a product on the
+// matrix cores.  An FP32 product of K = 4 adds its four terms to the
+// accumulator one by one in order, each a fused multiply-add (measured: the
+// same bits, subnormals included), so a wave that walks the points in order
+// gives the bits of the serial sum; for that order each of these sums stays
+// with one wave, and the two of dW1 and that of dW3 run at the same time on
+// SIMDs of their own.  dW2's operands come channel by channel from
+// transposed copies (three taps from two 8-byte reads, where point by point
+// they took 12 two-byte reads); h2's sign comes from the forward's
+// registers.
+// Measured on 16 samples of 83 x 42 points (288 tiles): 26.7 us with the
+// serial sums on 4 waves, 16.6 us so.
+__global__ __launch_bounds__(kB) void k_net_backward(const float* __restrict__ p_all, const float* __restrict__ dy_all,
                                                      NetGeom g, NetDev w, float* __restrict__ parts) {
+  constexpr int kW = kB / 64;
   __shared__ unsigned sx[kP * kP];
-  __shared__ __align__(16) uint16_t h1[kNH1 * kNetC];
-  __shared__ uint16_t h2[kNH2 * kNetC];
-  __shared__ float sdy[kNH1];                 // dy over the tile + 2
-  __shared__ uint16_t dz2[kNH2 * kNetC];      // BF16 (MFMA operand)
-  __shared__ float dz1[kTile * kTile * kNetC];
+  __shared__ float sdy[kNH1];                                 // dy over the tile + 2
+  // dy over the tile on layer 2's 18-point rows, zero around (a row and a
+  // point before and after), so that every tap's shift is one offset
+  __shared__ float tdy[(kH2 + 2) * kH2 + 2];
+  __shared__ __align__(16) uint16_t h2[kNH2 * kNetC];
+  __shared__ __align__(16) uint16_t dz2[kNH2 * kNetC];        // BF16 (MFMA operand)
+  __shared__ __align__(16) uint16_t dz2t[kNetC * kDz2Pitch];  // the tile's own, channel by channel
+  __shared__ __align__(16) uint16_t h1t[kNetC * kH1Pitch];    // layer 1, channel by channel
+  __shared__ union __align__(16) {
+    uint16_t h1[kNH1 * kNetC];           // layer 1 for layer 2 ...
+    float dz1[kTile * kTile * kNetC];    // ... and then this
+  } mem;
   // tiles cover the region grown by 2: dz2 is non-zero up to 1 and dz1 up
   // to 2 cells outside the region, and every point's terms belong to the
   // one tile that owns it
   const TileMap m = tile_of(g, 2);
-  const long long eo = (long long)m.e * g.stride;
-  forward_tile(p_all + eo, g.r + (long long)(m.e / g.rdiv) * g.rstride, g, m, w, sx, h1, h2, nullptr, false);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int q = tid; q < kNH1; q += kT) {
+  const float* dy = dy_all + (long long)m.e * g.stride;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kq = lane >> 4, ln = lane & 15;
+  for (int q = tid; q < kNH1; q += kB) {
     const int x = m.ox - 2 + q / kH1, z = m.oz - 2 + q % kH1;
     const bool in = x >= g.x0 && x < g.x1 && z >= g.z0 && z < g.z1;  // dy is zero outside the region
-    sdy[q] = in ? dy_all[eo + (long long)x * g.nz + z] : 0.f;
+    const float d = in ? dy[(long long)x * g.nz + z] : 0.f;
+    sdy[q] = d;
+    const int tx = q / kH1 - 2, tz = q % kH1 - 2;
+    if ((unsigned)tx < (unsigned)kTile && (unsigned)tz < (unsigned)kTile) tdy[(tx + 2) * kH2 + tz + 2] = d;
+  }
+  for (int i = tid; i < (kH2 + 2) * kH2 + 2; i += kB) {
+    const int tx = (i - 1 + kH2) / kH2 - 3, tz = (i - 1 + kH2) % kH2 - 1;
+    if ((unsigned)tx >= (unsigned)kTile || (unsigned)tz >= (unsigned)kTile) tdy[i] = 0.f;
+  }
+  // the weights' operands on their way during the forward
+  f32x4 w3[9];
+  bf16x4 w2[9];
+#pragma unroll
+  for (int t = 0; t < 9; t++) {
+    w3[t] = *reinterpret_cast<const f32x4*>(w.w3 + t * kNetC + 4 * kq);
+    w2[t] = *reinterpret_cast<const bf16x4*>(w.w2b + (t * 64 + lane) * 4);
+  }
+  Hidden<kB> hid;
+  forward_tile<kB, true>(p_all + (long long)m.in * g.stride, g.r + (long long)(m.in / g.rdiv) * g.rstride, g, m, w, sx,
+                         mem.h1, h1t, nullptr, false, hid);
+  // dz2 over the tile + 1, lane for lane as the layer-2 result lies
+  {
+#pragma unroll
+    for (int i = 0; i < Hidden<kB>::kMax; i++) {
+      const int grp = wave + i * kW;
+      const int q = grp * 16 + ln;
+      if (q < kNH2) {
+        const int x = q / kH2, z = q % kH2;  // layer-2 coords; sdy coords = +1
+        f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 9; t++) {
+          const float d = sdy[(x + 1 - (t / 3 - 1)) * kH1 + (z + 1 - (t % 3 - 1))];
+#pragma unroll
+          for (int v = 0; v < 4; v++) a[v] = fmaf(w3[t][v], d, a[v]);
+        }
+        bf16x4 o;
+#pragma unroll
+        for (int v = 0; v < 4; v++) o[v] = (short)bf16_of(f32_of((uint16_t)hid.h[i][v]) > 0.f ? a[v] : 0.f);
+        *reinterpret_cast<bf16x4*>(h2 + q * kNetC + 4 * kq) = hid.h[i];
+        *reinterpret_cast<bf16x4*>(dz2 + q * kNetC + 4 * kq) = o;
+        if (x >= 1 && x <= kTile && z >= 1 && z <= kTile) {
+#pragma unroll
+          for (int v = 0; v < 4; v++) dz2t[(4 * kq + v) * kDz2Pitch + (x - 1) * kTile + z - 1] = (uint16_t)o[v];
+        }
+      }
+    }
   }
   __syncthreads();
   float* out = parts + (long long)blockIdx.x * kNetParams;
-  // dz2 over the tile + 1
-  for (int q = tid; q < kNH2; q += kT) {
-    const int x = q / kH2, z = q % kH2;  // layer-2 coords; sdy coords = +1
-#pragma unroll
-    for (int c = 0; c < kNetC; c++) {
-      float a = 0.f;
-#pragma unroll
-      for (int t = 0; t < 9; t++) {
-        const int dx = t / 3 - 1, dz = t % 3 - 1;
-        a = fmaf(w.w3[t * kNetC + c], sdy[(x + 1 - dx) * kH1 + (z + 1 - dz)], a);
-      }
-      dz2[q * kNetC + c] = bf16_of(f32_of(h2[q * kNetC + c]) > 0.f ? a : 0.f);
-    }
-  }
-  // dW3: 144 sums over the tile's 256 points, one per thread
-  if (tid < kNetW3) {
-    const int t = tid / kNetC, c = tid % kNetC;
-    const int dx = t / 3 - 1, dz = t % 3 - 1;
-    float a = 0.f;
-    for (int x = 0; x < kTile; x++)
-      for (int z = 0; z < kTile; z++)
-        a = fmaf(sdy[(x + 2) * kH1 + (z + 2)], f32_of(h2[((x + 1 + dx) * kH2 + (z + 1 + dz)) * kNetC + c]), a);
-    out[kNetW1 + kNetW2 + tid] = a;
-  }
-  __syncthreads();
-  // dW2 on MFMA: per tap, D[ci][co] = sum over the 256 tile points (16 K-steps)
-  for (int t = wave; t < 9; t += kT / 64) {
-    const int dx = t / 3 - 1, dz = t % 3 - 1;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int kc = 0; kc < kTile * kTile / 16; kc++) {
-      bf16x4 a, b;
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int pt = kc * 16 + 4 * (lane >> 4) + v;  // tile point of this K item
-        const int x = pt / kTile, z = pt % kTile;
-        a[v] = (short)h1[((x + 2 + dx) * kH1 + (z + 2 + dz)) * kNetC + (lane & 15)];
-        b[v] = (short)dz2[((x + 1) * kH2 + (z + 1)) * kNetC + (lane & 15)];
-      }
-      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int v = 0; v < 4; v++) out[kNetW1 + (t * kNetC + d_row(lane, v)) * kNetC + d_col(lane)] = acc[v];
-  }
-  // dz1 on MFMA: per group of 16 tile points, D[pt][ci] = sum_t A_t[pt][co] B_t[co][ci]
-  {
-    bf16x4 b[9];
-#pragma unroll
-    for (int t = 0; t < 9; t++) b[t] = *reinterpret_cast<const bf16x4*>(w.w2b + (t * 64 + lane) * 4);
-    for (int grp = wave; grp < kTile * kTile / 16; grp += kT / 64) {
-      const int pt = grp * 16 + (lane & 15);
-      const int x = pt / kTile, z = pt % kTile;
-      const int kofs = 4 * (lane >> 4);
+  // this lane's tap as a row of dW1 and dW3; the products' rows past the
+  // ninth are not kept
+  const int tl = ln < 9 ? ln : 8, dx = tl / 3 - 1, dz = tl % 3 - 1;
+  // dW3: D[t][c] = sum over the points x' of the tile + 1 of dy(x' - o_t)
+  // h2[c](x'), dy taken where x' - o_t is in the tile; four points a product
+  f32x4 a3 = {0.f, 0.f, 0.f, 0.f};
+  const float* t3 = tdy + kH2 + 1 - dx * kH2 - dz + kq;
+  const uint16_t* b3 = h2 + kq * kNetC + ln;
+  static_assert(kNH2 == 4 * 9 * 9, "whole batches of K-steps");
+  constexpr int kFirst3 = 4;  // batches before the barrier
+  const auto same = [](float v) { return v; };
+  const auto at3 = [&](int k, int i) { return t3[4 * (9 * k + i)]; };
+  const auto bt3 = [&](int k, int i) { return b3[4 * (9 * k + i) * kNetC]; };
+  // dz1 by waves 0 .. 6 (a row of the tile each: D[pt][ci]), in whose time
+  // wave 7 has done the first part of dW3
+  if (wave == kW - 1) {
+    a3 = mfma_chain<0, kFirst3, 9>(a3, at3, bt3, same, f32_of);
+  } else {
+    for (int x = wave; x < kTile; x += kW - 1) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int t = 0; t < 9; t++) {
-        const int dx = t / 3 - 1, dz = t % 3 - 1;
-        const int q2 = (x + 1 - dx) * kH2 + (z + 1 - dz);
-        const bf16x4 a = *reinterpret_cast<const bf16x4*>(dz2 + q2 * kNetC + kofs);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[t], acc, 0, 0, 0);
+        const int q2 = (x + 1 - (t / 3 - 1)) * kH2 + (ln + 1 - (t % 3 - 1));
+        const bf16x4 a = *reinterpret_cast<const bf16x4*>(dz2 + q2 * kNetC + 4 * kq);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, w2[t], acc, 0, 0, 0);
       }
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        const int pr = grp * 16 + d_row(lane, v), c = d_col(lane);
-        const int xr = pr / kTile, zr = pr % kTile;
-        const bool on = f32_of(h1[((xr + 2) * kH1 + (zr + 2)) * kNetC + c]) > 0.f;
-        dz1[pr * kNetC + c] = on ? acc[v] : 0.f;
+        const int z = d_row(lane, v);
+        const bool on = f32_of(h1t[ln * kH1Pitch + (x + 2) * kH1 + z + 2]) > 0.f;
+        mem.dz1[(x * kTile + z) * kNetC + ln] = on ? acc[v] : 0.f;
       }
     }
   }
   __syncthreads();
-  // dW1: 288 sums over the tile
-  for (int j = tid; j < kNetW1; j += kT) {
-    const int t = j / (kNetIn * kNetC), k = (j / kNetC) % kNetIn, c = j % kNetC;
-    const int dx = t / 3 - 1, dz = t % 3 - 1;
-    const int sh = 16 * k;  // p in the low half, r p in the high half
-    float a = 0.f;
-    for (int x = 0; x < kTile; x++)
-      for (int z = 0; z < kTile; z++) {
-        const float in = f32_of((uint16_t)(sx[(x + 3 + dx) * kP + (z + 3 + dz)] >> sh));
-        a = fmaf(in, dz1[(x * kTile + z) * kNetC + c], a);
-      }
-    out[j] = a;
+  if (wave == kW - 1) {
+    a3 = mfma_chain<kFirst3, 9, 9>(a3, at3, bt3, same, f32_of);
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      if (d_row(lane, v) < 9) out[kNetW1 + kNetW2 + d_row(lane, v) * kNetC + ln] = a3[v];
+  } else if (wave < 2) {
+    // dW1: D[t][c] = sum over the tile's points of in_k(x + o_t) dz1[c](x),
+    // wave k its input
+    f32x4 a1 = {0.f, 0.f, 0.f, 0.f};
+    const int sh = wave ? 0 : 16;  // p in the low half, r p in the high half
+    const unsigned* in = sx + (3 + dx) * kP + 3 + dz + kq;
+    const float* d1 = mem.dz1 + kq * kNetC + ln;
+    a1 = mfma_chain<0, kTile / 2, kTile / 2>(
+        a1, [&](int k, int i) { return in[(2 * k + i / (kTile / 4)) * kP + 4 * (i % (kTile / 4))]; },
+        [&](int k, int i) { return d1[(k * (kTile / 2) + i) * 4 * kNetC]; },
+        [&](unsigned pr) { return __uint_as_float((pr << sh) & 0xffff0000u); }, same);
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      if (d_row(lane, v) < 9) out[(d_row(lane, v) * kNetIn + wave) * kNetC + ln] = a1[v];
+  } else if (wave >= 4) {
+    // dW2: waves 4, 5, 6 take a column of taps each; a K-step is a row of the tile
+    const int cx = wave - 5;
+    f32x4 a2[3] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 4
+    for (int x = 0; x < kTile; x++) {
+      // h1 at z + 2 + dz = 4 kq + (1 .. 3) + v: out of the eight from 4 kq on
+      const uint2* ap = reinterpret_cast<const uint2*>(h1t + ln * kH1Pitch + (x + 2 + cx) * kH1 + 4 * kq);
+      const uint2 d01 = ap[0], d23 = ap[1];
+      const bf16x4 b = *reinterpret_cast<const bf16x4*>(dz2t + ln * kDz2Pitch + x * kTile + 4 * kq);
+      union { unsigned u[2]; bf16x4 b; } lo, mid, hi;
+      lo.u[0] = __builtin_amdgcn_alignbyte(d01.y, d01.x, 2);
+      lo.u[1] = __builtin_amdgcn_alignbyte(d23.x, d01.y, 2);
+      mid.u[0] = d01.y;
+      mid.u[1] = d23.x;
+      hi.u[0] = lo.u[1];
+      hi.u[1] = __builtin_amdgcn_alignbyte(d23.y, d23.x, 2);
+      a2[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(lo.b, b, a2[0], 0, 0, 0);
+      a2[1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(mid.b, b, a2[1], 0, 0, 0);
+      a2[2] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(hi.b, b, a2[2], 0, 0, 0);
+    }
+#pragma unroll
+    for (int z = 0; z < 3; z++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        out[kNetW1 + (((cx + 1) * 3 + z) * kNetC + d_row(lane, v)) * kNetC + ln] = a2[z][v];
+  }
+}
+
+// What k_net_reduce needs to move the weights on as well
+struct AdamArgs {
+  float *theta, *m, *v;  // theta null: the gradient only
+  float c1, c2, lr, b1, b2, eps;
+  NetDev w;
+};
+
+// weight j's new value into every packed form that holds it (the padding in
+// those is zero from k_net_pack on)
+__device__ __forceinline__ void pack_weight(const NetDev& w, int j, float th) {
+  uint16_t* w1a = const_cast<uint16_t*>(w.w1a);
+  uint16_t* w2b = const_cast<uint16_t*>(w.w2b);
+  uint16_t* w3a = const_cast<uint16_t*>(w.w3a);
+  uint16_t* w2p = const_cast<uint16_t*>(w.w2p);
+  const uint16_t b = bf16_of(th);
+  if (j < kNetW1) {
+    const int k = j / kNetC, c = j % kNetC;
+    w1a[(k / 16) * 256 + (((k % 16) / 4) * 16 + c) * 4 + k % 4] = b;
+  } else if (j < kNetW1 + kNetW2) {
+    const int i = j - kNetW1, t = i / (kNetC * kNetC), ci = (i / kNetC) % kNetC, co = i % kNetC;
+    const int k = (t & 1) * 16 + ci;
+    w2p[(t / 2) * 512 + ((k / 8) * 16 + co) * 8 + k % 8] = b;
+    w2b[t * 256 + ((co / 4) * 16 + ci) * 4 + co % 4] = b;
+  } else {
+    const int i = j - kNetW1 - kNetW2, t = i / kNetC, c = i % kNetC;
+    w3a[((c / 4) * 16 + t) * 4 + c % 4] = b;
+    const_cast<float*>(w.w3)[i] = f32_of(b);
   }
 }
 
 // grad[j] = sum over blocks of parts[b][j] in FP64, in a fixed order: each
 // block takes 16 weights; its 16 thread groups sum consecutive runs of the
-// partials in block order, then the 16 run sums are added in run order
-constexpr int kRedJ = 16, kRedRuns = kT / kRedJ;
-__global__ void k_net_reduce(const float* parts, long long nblocks, float* grad) {
-  __shared__ double run[kRedRuns][kRedJ];
+// partials in block order, then the 16 run sums are added in run order.  The
+// weight's Adam step and its packed forms follow where its gradient is in a
+// register, and one more block sums the loss's partials: one launch for what
+// four did (288 blocks' partials: 4.8 us in place of 7.0 + 2.4 + 4.2 + 3.1).
+constexpr int kRedT = 256, kRedJ = 16, kRedRuns = kRedT / kRedJ;
+constexpr int kRedBlocks = (kNetParams + kRedJ - 1) / kRedJ;
+__global__ __launch_bounds__(kRedT) void k_net_reduce(const float* __restrict__ parts, long long nblocks,
+                                                      float* __restrict__ grad, const double* __restrict__ lparts,
+                                                      long long nl, double* __restrict__ loss, AdamArgs a) {
+  __shared__ double run[kRedT];
+  if (blockIdx.x == kRedBlocks) {  // the loss: strided sums, then a fixed tree
+    double s = 0;
+#pragma unroll 4
+    for (long long i = threadIdx.x; i < nl; i += kRedT) s += lparts[i];
+    run[threadIdx.x] = s;
+    __syncthreads();
+    for (int h = kRedT / 2; h > 0; h >>= 1) {
+      if (threadIdx.x < h) run[threadIdx.x] += run[threadIdx.x + h];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *loss = run[0];
+    return;
+  }
   const int jl = threadIdx.x % kRedJ, r = threadIdx.x / kRedJ;
   const int j = blockIdx.x * kRedJ + jl;
   const long long per = (nblocks + kRedRuns - 1) / kRedRuns;
   const long long b0 = r * per, b1 = b0 + per < nblocks ? b0 + per : nblocks;
   double s = 0;
-  if (j < kNetParams)
+  if (j < kNetParams) {
+#pragma unroll 8
     for (long long b = b0; b < b1; b++) s += parts[b * kNetParams + j];
-  run[r][jl] = s;
-  __syncthreads();
-  if (r == 0 && j < kNetParams) {
-    double t = 0;
-    for (int q = 0; q < kRedRuns; q++) t += run[q][jl];
-    grad[j] = (float)t;
   }
+  run[threadIdx.x] = s;
+  __syncthreads();
+  if (r != 0 || j >= kNetParams) return;
+  double t = 0;
+#pragma unroll
+  for (int q = 0; q < kRedRuns; q++) t += run[q * kRedJ + jl];
+  const float gr = (float)t;
+  if (grad) grad[j] = gr;
+  if (!a.theta) return;
+  const float mi = a.b1 * a.m[j] + (1.f - a.b1) * gr;
+  const float vi = a.b2 * a.v[j] + (1.f - a.b2) * gr * gr;
+  a.m[j] = mi;
+  a.v[j] = vi;
+  const float th = a.theta[j] - a.lr * (mi * a.c1) / (sqrtf(vi * a.c2) + a.eps);
+  a.theta[j] = th;
+  pack_weight(a.w, j, th);
 }
 
 __global__ void k_net_pack(const float* theta, uint16_t* w1a, uint16_t* w2b, uint16_t* w3a,
@@ -459,48 +643,6 @@ __global__ void k_net_pack(const float* theta, uint16_t* w1a, uint16_t* w2b, uin
   }
 }
 
-__global__ void k_net_adam(float* theta, const float* grad, float* m, float* v, float c1, float c2, float lr,
-                           float b1, float b2, float eps) {
-  const int i = blockIdx.x * kT + threadIdx.x;
-  if (i >= kNetParams) return;
-  const float gr = grad[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gr;
-  const float vi = b2 * v[i] + (1.f - b2) * gr * gr;
-  m[i] = mi;
-  v[i] = vi;
-  theta[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
-}
-
-// *out = sum of parts[0..n) in FP64 in a fixed order: consecutive runs per
-// thread, then the run sums pairwise in a fixed tree
-__global__ void k_sum_parts(const double* parts, int n, double* out) {
-  __shared__ double red[kT];
-  const int per = (n + kT - 1) / kT, i0 = threadIdx.x * per;
-  double s = 0;
-  for (int i = i0; i < i0 + per && i < n; i++) s += parts[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int h = kT / 2; h > 0; h >>= 1) {
-    if (threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = red[0];
-}
-
-// the minibatch: sample idx[b] of the training set into slot b, for the
-// inputs, models and targets at once
-__global__ void k_gather3(float* din, float* dr, float* dt, const float* sin, const float* sr, const float* st,
-                          const int* idx, int batch, long long stride) {
-  const long long n = (long long)batch * stride;
-  for (long long i = blockIdx.x * (long long)kT + threadIdx.x; i < n; i += (long long)gridDim.x * kT) {
-    const long long b = i / stride, o = i - b * stride;
-    const long long src = (long long)idx[b] * stride + o;
-    din[i] = sin[src];
-    dr[i] = sr[src];
-    dt[i] = st[src];
-  }
-}
-
 long long tiles_of(const NetGeom& g, int margin) {
   const long long tz = (g.z1 - g.z0 + 2 * margin + kTile - 1) / kTile,
                   tx = (g.x1 - g.x0 + 2 * margin + kTile - 1) / kTile;
@@ -528,38 +670,42 @@ void net_pack(const float* theta, const NetDev& w, hipStream_t s) {
 
 void net_apply(const float* p, float* y, const NetGeom& g, const NetDev& w, hipStream_t s) {
   check_geom(g, 2);
-  hipLaunchKernelGGL(k_net_apply, dim3((unsigned)tiles_of(g, 0)), dim3(kT), 0, s, p, y, g, w);
+  hipLaunchKernelGGL(k_net_apply<false>, dim3((unsigned)tiles_of(g, 0)), dim3(kT), 0, s, p, y, g, w, LossArgs{});
 }
 
 void net_add(float* p, const float* y, const NetGeom& g, hipStream_t s) {
   hipLaunchKernelGGL(k_net_add, dim3(2048), dim3(kT), 0, s, p, y, g);
 }
 
-void net_loss(const float* p, const float* y, const float* t, float* dy, const NetGeom& g, double* loss_parts,
-              int nparts, hipStream_t s) {
+long long net_loss_blocks(const NetGeom& g) { return tiles_of(g, 0); }
+
+void net_loss(const float* p, const float* t, float* dy, const NetGeom& g, const NetDev& w, double* loss_parts,
+              hipStream_t s) {
+  check_geom(g, 2);
   const double count = (double)(g.x1 - g.x0) * (g.z1 - g.z0) * g.entries;
-  hipLaunchKernelGGL(k_net_loss, dim3(nparts), dim3(kT), 0, s, p, y, t, dy, g, 1.0 / count, loss_parts);
+  hipLaunchKernelGGL(k_net_apply<true>, dim3((unsigned)tiles_of(g, 0)), dim3(kT), 0, s, p, dy, g, w,
+                     LossArgs{t, 1.0 / count, loss_parts});
 }
 
 long long net_backward_blocks(const NetGeom& g) { return tiles_of(g, 2); }
 
-void net_backward(const float* p, const float* dy, const NetGeom& g, const NetDev& w, float* parts, float* grad,
-                  hipStream_t s) {
+void net_backward(const float* p, const float* dy, const NetGeom& g, const NetDev& w, float* parts, hipStream_t s) {
   check_geom(g, 2);
-  const long long nb = tiles_of(g, 2);
-  hipLaunchKernelGGL(k_net_backward, dim3((unsigned)nb), dim3(kT), 0, s, p, dy, g, w, parts);
-  hipLaunchKernelGGL(k_net_reduce, dim3((kNetParams + kRedJ - 1) / kRedJ), dim3(kT), 0, s, parts, nb, grad);
+  hipLaunchKernelGGL(k_net_backward, dim3((unsigned)tiles_of(g, 2)), dim3(kB), 0, s, p, dy, g, w, parts);
 }
 
-void net_adam(float* theta, const float* grad, float* m, float* v, int step, float lr, float b1, float b2, float eps,
+void net_reduce(const float* parts, long long nblocks, float* grad, const double* loss_parts, long long nloss,
+                double* loss, hipStream_t s) {
+  hipLaunchKernelGGL(k_net_reduce, dim3(kRedBlocks + 1), dim3(kRedT), 0, s, parts, nblocks, grad, loss_parts, nloss,
+                     loss, AdamArgs{});
+}
+
+void net_adam(const float* parts, long long nblocks, const double* loss_parts, long long nloss, double* loss,
+              float* theta, float* m, float* v, const NetDev& w, int step, float lr, float b1, float b2, float eps,
               hipStream_t s) {
   const float c1 = 1.f / (1.f - std::pow(b1, (float)step)), c2 = 1.f / (1.f - std::pow(b2, (float)step));
-  hipLaunchKernelGGL(k_net_adam, dim3((kNetParams + kT - 1) / kT), dim3(kT), 0, s, theta, grad, m, v, c1, c2, lr, b1,
-                     b2, eps);
-}
-
-void net_reduce_parts(const double* parts, int nparts, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(kT), 0, s, parts, nparts, out);
+  hipLaunchKernelGGL(k_net_reduce, dim3(kRedBlocks + 1), dim3(kRedT), 0, s, parts, nblocks, (float*)nullptr,
+                     loss_parts, nloss, loss, AdamArgs{theta, m, v, c1, c2, lr, b1, b2, eps, w});
 }
 
 // ---- host handle -------------------------------------------------------------
@@ -574,7 +720,6 @@ ConvNet::ConvNet() {
   w2b_.resize(9 * 64 * 4);
   w3a_.resize(64 * 4);
   w2p_.resize(5 * 64 * 8);
-  lparts_.resize(1024);
   lsum_.resize(1);
 }
 
@@ -598,22 +743,18 @@ void ConvNet::correct(float* p, const NetGeom& g, float* yscratch, hipStream_t s
   net_add(p, yscratch, g, s);
 }
 
-// loss into *loss_dev (sum of r^2, FP64) and the weight gradient into grad_
-void ConvNet::loss_grad_async(const float* in, const float* target, const NetGeom& g, double* loss_dev,
-                              hipStream_t s) {
-  const size_t n = (size_t)g.stride * g.entries;
-  y_.resize(n);
-  dy_.resize(n);
+// dy, the per-block gradients and the per-block losses
+void ConvNet::grad_parts(const float* in, const float* target, const NetGeom& g, hipStream_t s) {
+  dy_.resize((size_t)g.stride * g.entries);
   parts_.resize((size_t)net_backward_blocks(g) * kNetParams);
-  net_apply(in, y_.get(), g, dev(), s);
-  const int np = 1024;
-  net_loss(in, y_.get(), target, dy_.get(), g, lparts_.get(), np, s);
-  net_reduce_parts(lparts_.get(), np, loss_dev, s);
-  net_backward(in, dy_.get(), g, dev(), parts_.get(), grad_.get(), s);
+  lparts_.resize((size_t)net_loss_blocks(g));
+  net_loss(in, target, dy_.get(), g, dev(), lparts_.get(), s);
+  net_backward(in, dy_.get(), g, dev(), parts_.get(), s);
 }
 
 double ConvNet::loss_grad(const float* in, const float* target, const NetGeom& g, float* grad_host, hipStream_t s) {
-  loss_grad_async(in, target, g, lsum_.get(), s);
+  grad_parts(in, target, g, s);
+  net_reduce(parts_.get(), net_backward_blocks(g), grad_.get(), lparts_.get(), net_loss_blocks(g), lsum_.get(), s);
   double loss = 0;
   SWFWI_HIP(hipMemcpyAsync(&loss, lsum_.get(), sizeof(double), hipMemcpyDeviceToHost, s));
   if (grad_host) SWFWI_HIP(hipMemcpyAsync(grad_host, grad_.get(), sizeof(float) * kNetParams, hipMemcpyDeviceToHost, s));
@@ -624,10 +765,10 @@ double ConvNet::loss_grad(const float* in, const float* target, const NetGeom& g
 
 void ConvNet::train_step(const float* in, const float* target, const NetGeom& g, float lr, double* loss_dev,
                          hipStream_t s) {
-  loss_grad_async(in, target, g, loss_dev, s);
+  grad_parts(in, target, g, s);
   step_++;
-  net_adam(theta_.get(), grad_.get(), m_.get(), v_.get(), step_, lr, 0.9f, 0.999f, 1e-8f, s);
-  repack(s);
+  net_adam(parts_.get(), net_backward_blocks(g), lparts_.get(), net_loss_blocks(g), loss_dev, theta_.get(), m_.get(),
+           v_.get(), dev(), step_, lr, 0.9f, 0.999f, 1e-8f, s);
 }
 
 void ConvNet::set_data(const float* in_host, const float* r_host, const float* target_host, int n,
@@ -652,10 +793,7 @@ void ConvNet::train(int batch, int steps, float lr, unsigned long long seed, dou
   if (steps < 0) fail(kErrArg, "negative step count");
   NetGeom g = dg_;
   g.entries = batch;
-  bin_.resize((size_t)batch * g.stride);
-  br_.resize((size_t)batch * g.stride);
-  btgt_.resize((size_t)batch * g.stride);
-  g.r = br_.get();
+  g.r = dr_.get();
   g.rstride = g.stride;
   g.rdiv = 1;
   // seeded shuffle of the sample order (splitmix64 + Fisher-Yates), refreshed
@@ -683,12 +821,9 @@ void ConvNet::train(int batch, int steps, float lr, unsigned long long seed, dou
   DBuf<double> dloss;
   didx.upload(idx.data(), idx.size(), s);
   dloss.resize((size_t)steps);
-  const long long total = (long long)batch * g.stride;
-  const unsigned gblocks = (unsigned)std::min<long long>((total + kT - 1) / kT, 2048);
   for (int k = 0; k < steps; k++) {
-    hipLaunchKernelGGL(k_gather3, dim3(gblocks), dim3(kT), 0, s, bin_.get(), br_.get(), btgt_.get(), din_.get(),
-                       dr_.get(), dtgt_.get(), didx.get() + (size_t)k * batch, batch, g.stride);
-    train_step(bin_.get(), btgt_.get(), g, lr, dloss.get() + k, s);
+    g.pick = didx.get() + (size_t)k * batch;
+    train_step(din_.get(), dtgt_.get(), g, lr, dloss.get() + k, s);
   }
   std::vector<double> l((size_t)steps);
   dloss.download(l.data(), l.size(), s);
