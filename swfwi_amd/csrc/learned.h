@@ -63,24 +63,20 @@ void net_pack(const float* theta, const NetDev& w, hipStream_t s);
 void net_apply(const float* p, float* y, const NetGeom& g, const NetDev& w, hipStream_t s);
 // p += y over the region
 void net_add(float* p, const float* y, const NetGeom& g, hipStream_t s);
-// Loss of a batch: r = p + net(p) - t over the region, dy = 2 r / count
-// there (dy elsewhere untouched), the sum of r^2 (FP64) of every block into
-// loss_parts, which must hold net_loss_blocks(g).
-long long net_loss_blocks(const NetGeom& g);
-void net_loss(const float* p, const float* t, float* dy, const NetGeom& g, const NetDev& w, double* loss_parts,
+// Loss of a batch, the sum of r^2 with r = p + net(p) - t over the region
+// (FP64), and the gradient of its mean with respect to every weight: each
+// block's part; `parts` must hold net_grad_blocks(g) * kNetParams floats,
+// `loss_parts` net_grad_blocks(g) doubles.
+long long net_grad_blocks(const NetGeom& g);
+void net_grad(const float* p, const float* t, const NetGeom& g, const NetDev& w, float* parts, double* loss_parts,
               hipStream_t s);
-// d loss / d weights, every block's part of it; `parts` must hold
-// net_backward_blocks(g) * kNetParams floats.
-long long net_backward_blocks(const NetGeom& g);
-void net_backward(const float* p, const float* dy, const NetGeom& g, const NetDev& w, float* parts, hipStream_t s);
 // The parts summed in a fixed order: the gradient and the loss ...
-void net_reduce(const float* parts, long long nblocks, float* grad, const double* loss_parts, long long nloss,
-                double* loss, hipStream_t s);
+void net_reduce(const float* parts, const double* loss_parts, long long nblocks, float* grad, double* loss,
+                hipStream_t s);
 // ... or the loss and Adam's step (step >= 1) on the gradient,
 // theta -= lr * mhat / (sqrt(vhat) + eps), with the packed weights renewed
-void net_adam(const float* parts, long long nblocks, const double* loss_parts, long long nloss, double* loss,
-              float* theta, float* m, float* v, const NetDev& w, int step, float lr, float b1, float b2, float eps,
-              hipStream_t s);
+void net_adam(const float* parts, const double* loss_parts, long long nblocks, double* loss, float* theta, float* m,
+              float* v, const NetDev& w, int step, float lr, float b1, float b2, float eps, hipStream_t s);
 
 // Host handle: weights (FP32 master copy + packed device forms), Adam state
 // and scratch for training on stacks of coarse fields.
@@ -111,7 +107,7 @@ class ConvNet {
   void grad_parts(const float* in, const float* target, const NetGeom& g, hipStream_t s);
   DBuf<float> theta_, m_, v_, grad_, w3_;
   DBuf<uint16_t> w1a_, w2b_, w3a_, w2p_;
-  DBuf<float> dy_, parts_, din_, dr_, dtgt_;
+  DBuf<float> parts_, din_, dr_, dtgt_;
   NetGeom dg_{};
   int dn_ = 0;
   DBuf<double> lparts_, lsum_;

@@ -1,5 +1,5 @@
 """The training step's kernels at the sizes where their tiles end, and its
-three launches against the parts they stand for.
+two launches against the parts they stand for.
 
 * the weight gradient (sums over the tile's points on the matrix cores) for
   regions of one point, of exactly one tile and two tiles with their 2-cell
