@@ -535,6 +535,24 @@ static void timed(hipStream_t s, double& ms_out, const std::function<void()>& bo
   (void)hipEventDestroy(e1);
 }
 
+// the runs' traces, one after the other at `host`, and their places on the device
+std::vector<HostSpan> Batch::traces(float* host, float* dev) const {
+  std::vector<HostSpan> v;
+  v.reserve(lay_.size());
+  for (const Layout& L : lay_) {
+    const size_t m = (size_t)L.nt * L.ng;
+    v.push_back({host, dev + L.dcal, sizeof(float) * m});
+    host += m;
+  }
+  return v;
+}
+
+size_t Batch::traces_bytes() const {
+  size_t n = 0;
+  for (const Layout& L : lay_) n += sizeof(float) * (size_t)L.nt * L.ng;
+  return n;
+}
+
 void Batch::forward(float* dcal_host) {
   hipStream_t s = stream_.get();
   if (tune_ && !tuned_ && !fixed_x_) tune();
@@ -553,27 +571,21 @@ void Batch::forward(float* dcal_host) {
     }
     SWFWI_HIP(hipGraphLaunch(graph_[0], s));
   };
+  PageIn pages(dcal_host, traces_bytes());
   timed(s, last_ms[0], body);
   SWFWI_HIP(hipGetLastError());
   if (dcal_host) {
-    long long o = 0;
-    for (const Layout& L : lay_) {
-      const long long m = (long long)L.nt * L.ng;
-      SWFWI_HIP(hipMemcpyAsync(dcal_host + o, dcal_.get() + L.dcal, sizeof(float) * m, hipMemcpyDeviceToHost, s));
-      o += m;
-    }
+    pages.wait();
+    lane_.down(traces(dcal_host, dcal_.get()), s);
   }
   SWFWI_HIP(hipStreamSynchronize(s));
 }
 
 void Batch::adjoint_from_observed(const float* dobs_host, float* vsrc_host) {
   hipStream_t s = stream_.get();
-  long long o = 0;
-  for (const Layout& L : lay_) {  // observed data into vsrc_, then the residual in place
-    const long long m = (long long)L.nt * L.ng;
-    SWFWI_HIP(hipMemcpyAsync(vsrc_.get() + L.dcal, dobs_host + o, sizeof(float) * m, hipMemcpyHostToDevice, s));
-    o += m;
-  }
+  PageIn pages(vsrc_host, traces_bytes());
+  // observed data into vsrc_, then the residual in place
+  lane_.up(traces(const_cast<float*>(dobs_host), vsrc_.get()), s);
   // the residual dobs - dcal replaces the recording, then transVsrc into vsrc_
   launch_sub(vsrc_.get(), dcal_.get(), dcal_.get(), dcal_len_, s);
   // transVsrc per group: a group's entries are contiguous in constructor order
@@ -592,26 +604,15 @@ void Batch::adjoint_from_observed(const float* dobs_host, float* vsrc_host) {
     i = j;
   }
   if (vsrc_host) {
-    o = 0;
-    for (const Layout& L : lay_) {
-      const long long m = (long long)L.nt * L.ng;
-      SWFWI_HIP(hipMemcpyAsync(vsrc_host + o, vsrc_.get() + L.dcal, sizeof(float) * m, hipMemcpyDeviceToHost, s));
-      o += m;
-    }
+    pages.wait();
+    lane_.down(traces(vsrc_host, vsrc_.get()), s);
   }
   SWFWI_HIP(hipStreamSynchronize(s));
 }
 
 void Batch::backward(const float* vsrc_host, float* grad_host, float* model_grad_host) {
   hipStream_t s = stream_.get();
-  if (vsrc_host) {
-    long long o = 0;
-    for (const Layout& L : lay_) {
-      const long long m = (long long)L.nt * L.ng;
-      SWFWI_HIP(hipMemcpyAsync(vsrc_.get() + L.dcal, vsrc_host + o, sizeof(float) * m, hipMemcpyHostToDevice, s));
-      o += m;
-    }
-  }
+  if (vsrc_host) lane_.up(traces(const_cast<float*>(vsrc_host), vsrc_.get()), s);
   auto body = [&] {
     if (!graphs_) {
       run_loop(false);

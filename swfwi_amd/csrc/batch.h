@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "device.h"
+#include "hostcopy.h"
 
 namespace swfwi {
 
@@ -214,6 +215,9 @@ class Batch {
   std::vector<BatchEntry> ent_;      // run order (nt descending)
   std::vector<int> run_of_;          // constructor order -> run index
   std::vector<Layout> lay_;
+  std::vector<HostSpan> traces(float* host, float* dev) const;
+  size_t traces_bytes() const;
+  HostLane lane_;
   std::vector<int> tile0_;           // per run index, prefix of tiles
   int strip_count(int uz) const;     // strips of an update region uz high
   long long strip_rows_ = 0;         // strips x rows of x over all entries

@@ -90,12 +90,14 @@ Enkf::Enkf(Solver& s, const float* wlt_host, const float* dobs_host, float sigfa
 }
 
 void Enkf::set_members(const float* host) {
-  mem_.upload(host, (size_t)N_ * s_.npts(), s_.stream());
+  const size_t n = (size_t)N_ * s_.npts();
+  mem_.resize(n);
+  s_.lane().up({{const_cast<float*>(host), mem_.get(), n * sizeof(float)}}, s_.stream());
   s_.prop().sync();
 }
 
 void Enkf::get_members(float* host) {
-  mem_.download(host, (size_t)N_ * s_.npts(), s_.stream());
+  s_.lane().down({{host, mem_.get(), sizeof(float) * N_ * s_.npts()}}, s_.stream());
   s_.prop().sync();
 }
 

@@ -170,8 +170,11 @@ void Solver::forward_shots(const float* wlt_host, float* dobs_host) {
   upload_now(hi, h, s);
   Propagator::Sources src{wtab_.get(), ns, 0, lo.get(), hi.get()};
   dcal.resize((size_t)ns * m);
+  const size_t bytes = sizeof(float) * ns * m;
+  PageIn pages(dobs_host, bytes);
   prop_.forward(ns, rv_.get(), 0, src, dcal.get(), nullptr, w);
-  dcal.download(dobs_host, (size_t)ns * m, s);
+  pages.wait();
+  lane_.down({{dobs_host, dcal.get(), bytes}}, s);
   prop_.sync();
 }
 

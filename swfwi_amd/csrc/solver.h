@@ -8,6 +8,7 @@
 #include <cstdint>
 #include <vector>
 
+#include "hostcopy.h"
 #include "linesearch.h"
 #include "propagator.h"
 
@@ -37,6 +38,7 @@ class Solver {
   Solver(const Geometry& g, int precision);
 
   Propagator& prop() { return prop_; }
+  HostLane& lane() { return lane_; }
   const Geometry& geo() const { return prop_.geo(); }
   hipStream_t stream() const { return prop_.stream(); }
   long long npts() const { return prop_.geo().npts(); }
@@ -89,6 +91,7 @@ class Solver {
 
  private:
   Propagator prop_;
+  HostLane lane_;
   DBuf<float> vel_, rv_, wlt_, wtab_;
   bool bound_ = false;
 };
