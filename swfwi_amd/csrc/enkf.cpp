@@ -151,9 +151,9 @@ void Enkf::analyze(const double* e_host, uint64_t seed) {
   G_.resize((size_t)N * N);
   P_.resize((size_t)N * N);
   Q_.resize((size_t)N * N);
-  op_gram_f64(band_.get(), band_.get(), N, nd, G_.get(), st);
-  op_gram_f64(hap_.get(), band_.get(), N, nd, P_.get(), st);
-  op_gram_f64(band_.get(), t0_.get(), N, nd, Q_.get(), st);
+  op_gram_f64(band_.get(), band_.get(), N, nd, G_.get(), part_, st);
+  op_gram_f64(hap_.get(), band_.get(), N, nd, P_.get(), part_, st);
+  op_gram_f64(band_.get(), t0_.get(), N, nd, Q_.get(), part_, st);
   std::vector<double> G((size_t)N * N), P((size_t)N * N), Q((size_t)N * N);
   G_.download(G.data(), G.size(), st);
   P_.download(P.data(), P.size(), st);
@@ -193,9 +193,13 @@ void Enkf::analyze(const double* e_host, uint64_t seed) {
     }
 
   // model space: A' t4 and the velTrans(velRecover(v) + t5) update
-  T_.upload(t4_, st);
+  const int ld = (N + kUpdateChunk - 1) / kUpdateChunk * kUpdateChunk;
+  std::vector<double> rows((size_t)N * ld, 0.0);
+  for (int j = 0; j < N; j++)
+    for (int i = 0; i < N; i++) rows[(size_t)j * ld + i] = t4_[(size_t)j + (size_t)N * i];
+  T_.upload(rows, st);
   const Geometry& gg = s_.geo();
-  enkf_model_update(mem_.get(), mem_out_.get(), n, N, T_.get(), gg.dx, gg.dt, st);
+  enkf_model_update(mem_.get(), mem_out_.get(), n, N, T_.get(), ld, gg.dx, gg.dt, st);
   std::swap(mem_, mem_out_);
   SWFWI_HIP(hipStreamSynchronize(st));
 }

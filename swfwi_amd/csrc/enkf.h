@@ -15,7 +15,10 @@ constexpr int kMaxMembers = 1024;
 void enkf_ha_perturb(const float* ha, int N, long long nd, double* hap, double* max_abs_value, hipStream_t s);
 void enkf_band(const float* ha, const double* hap, const float* d, const double* e_in, uint64_t seed, double sigma,
                int N, long long nd, double* band, double* t0, hipStream_t s);
-void enkf_model_update(const float* vels, float* out, long long n, int N, const double* T, float dx, float dt,
+// T: [N][ld] with T[j][i] = t4[j + N i], ld = N up to the next multiple of
+// kUpdateChunk, zero past N
+constexpr int kUpdateChunk = 16;
+void enkf_model_update(const float* vels, float* out, long long n, int N, const double* T, int ld, float dx, float dt,
                        hipStream_t s);
 void enkf_member_mean(const float* vels, long long n, int N, float* mean, hipStream_t s);
 
@@ -53,7 +56,7 @@ class Enkf {
   float sigfac_;
   DBuf<float> dobs_, mem_, mem_out_, rv_, ha_, d_, encsrc_, mean_;
   DBuf<int> code_;
-  DBuf<double> hap_, band_, t0_, e_, G_, P_, Q_, T_;
+  DBuf<double> hap_, band_, t0_, e_, G_, P_, Q_, T_, part_;
   CodeStream codes_{2};  // ENKF_SEED (enkfanalyze.h:44)
   bool sigma_init_ = false;
   double sigma_ = 0;

@@ -83,59 +83,84 @@ __global__ void k_ha_perturb(const float* ha, int N, long long nd, double* hap, 
 
 // Perturbation E (generated N(0, sigma) or given), D = d + E, gamma = E -
 // rowmean(E), band = HA' + gamma, t0 = D - HA (enkfanalyze.cpp:430-460).
-__global__ void k_band(const float* ha, const double* hap, const float* d, const double* e_in, uint64_t seed,
-                       double sigma, int N, long long nd, double* band, double* t0) {
-  for (long long r = blockIdx.x * (long long)kB + threadIdx.x; r < nd; r += (long long)gridDim.x * kB) {
-    double s = 0.0;
-    for (int i = 0; i < N; i++) {
-      const double e = e_in ? e_in[(long long)i * nd + r] : sigma * normal_at(seed, (uint64_t)i * nd + r);
-      s += e;
-      band[(long long)i * nd + r] = e;  // E parked in band until its row mean is known
+// A block takes 64 data rows; four waves share their members (the generator's
+// FP64 logarithms and cosines are most of the time), one adds up a row's E in
+// member order.  60 members of 150500 data: 177 us with a row's members one
+// after the other in a thread -> 116.
+constexpr int kBandRows = 64, kBandShare = kB / kBandRows;
+
+__global__ __launch_bounds__(kB) void k_band(const float* __restrict__ ha, const double* __restrict__ hap,
+                                             const float* __restrict__ d, const double* __restrict__ e_in,
+                                             uint64_t seed, double sigma, int N, long long nd, double* band,
+                                             double* __restrict__ t0) {
+  __shared__ double mean[kBandRows];
+  const int rl = threadIdx.x % kBandRows, part = threadIdx.x / kBandRows;
+  for (long long base = blockIdx.x * (long long)kBandRows; base < nd; base += (long long)gridDim.x * kBandRows) {
+    const long long r = base + rl;
+    if (r < nd) {
+      for (int i = part; i < N; i += kBandShare) {
+        // E parked in band until its row mean is known
+        band[(long long)i * nd + r] =
+            e_in ? e_in[(long long)i * nd + r] : sigma * normal_at(seed, (uint64_t)i * nd + r);
+      }
     }
-    const double avg = s / N;
-    const double dr = d[r];
-    for (int i = 0; i < N; i++) {
-      const long long q = (long long)i * nd + r;
-      const double e = band[q];
-      t0[q] = (dr + e) - (double)ha[q];
-      band[q] = hap[q] + (e - avg);
+    __syncthreads();
+    if (part == 0 && r < nd) {
+      double s = 0.0;
+#pragma unroll 8
+      for (int i = 0; i < N; i++) s += band[(long long)i * nd + r];
+      mean[rl] = s / N;
     }
+    __syncthreads();
+    if (r < nd) {
+      const double avg = mean[rl], dr = d[r];
+      for (int i = part; i < N; i += kBandShare) {
+        const long long q = (long long)i * nd + r;
+        const double e = band[q];
+        t0[q] = (dr + e) - (double)ha[q];
+        band[q] = hap[q] + (e - avg);
+      }
+    }
+    __syncthreads();
   }
 }
 
 // Per point of the model: pCreateAMean (FP32 member-order sum / N), A' = A -
 // mean in FP64, t5 = A' * T, then vel = velTrans(velRecover(vel) + t5) in the
 // reference's float/double mix (enkfanalyze.cpp:113-183,578-597, common.h:21-30).
-constexpr int kChunk = 16;  // members updated per pass (register accumulators)
-
-__global__ void k_model_update(const float* vels, float* out, long long n, int N, const double* __restrict__ sT,
-                               float dx, float dt) {
-  // sT (N x N) is read with wave-uniform indices: served from the scalar cache
+// A thread takes a point and kUpdateChunk members (blockIdx.y): T's row of a
+// member j is kUpdateChunk consecutive doubles at a wave-uniform address, two
+// wide scalar loads next to 16 FMAs, and the members' chunks run as blocks of
+// their own, since the points alone leave about one wave a SIMD.  60 members
+// of a 301 x 201 model: 258 us (column-wise T, the chunks one after the other)
+// -> 42.
+__global__ void k_model_update(const float* __restrict__ vels, float* __restrict__ out, long long n, int N,
+                               const double* __restrict__ T, int ld, float dx, float dt) {
+  const int i0 = blockIdx.y * kUpdateChunk;
   for (long long p = blockIdx.x * (long long)kB + threadIdx.x; p < n; p += (long long)gridDim.x * kB) {
     float sum = 0.f;
+#pragma unroll 8
     for (int j = 0; j < N; j++) sum += vels[(long long)j * n + p];
     const float mean = sum / N;
-    for (int i0 = 0; i0 < N; i0 += kChunk) {
-      double acc[kChunk];
+    double acc[kUpdateChunk];
 #pragma unroll
-      for (int k = 0; k < kChunk; k++) acc[k] = 0.0;
-      for (int j = 0; j < N; j++) {
-        const double ap = (double)vels[(long long)j * n + p] - (double)mean;
+    for (int k = 0; k < kUpdateChunk; k++) acc[k] = 0.0;
+#pragma unroll 2
+    for (int j = 0; j < N; j++) {
+      const double ap = (double)vels[(long long)j * n + p] - (double)mean;
 #pragma unroll
-        for (int k = 0; k < kChunk; k++)
-          if (i0 + k < N) acc[k] = __builtin_fma(ap, sT[j + N * (i0 + k)], acc[k]);
-      }
+      for (int k = 0; k < kUpdateChunk; k++) acc[k] = __builtin_fma(ap, T[(long long)j * ld + i0 + k], acc[k]);
+    }
 #pragma unroll
-      for (int k = 0; k < kChunk; k++) {
-        const int i = i0 + k;
-        if (i >= N) break;
-        float v = vels[(long long)i * n + p];
-        float t = dx * dx / (dt * dt * v);  // velRecover
-        v = sqrtf(t);
-        v = (float)((double)v + acc[k]);
-        v = dx * dx / (dt * dt * v * v);    // velTrans
-        out[(long long)i * n + p] = v;
-      }
+    for (int k = 0; k < kUpdateChunk; k++) {
+      const int i = i0 + k;
+      if (i >= N) break;
+      float v = vels[(long long)i * n + p];
+      float t = dx * dx / (dt * dt * v);  // velRecover
+      v = sqrtf(t);
+      v = (float)((double)v + acc[k]);
+      v = dx * dx / (dt * dt * v * v);    // velTrans
+      out[(long long)i * n + p] = v;
     }
   }
 }
@@ -144,6 +169,7 @@ __global__ void k_model_update(const float* vels, float* out, long long n, int N
 __global__ void k_member_mean(const float* vels, long long n, int N, float* mean) {
   for (long long p = blockIdx.x * (long long)kB + threadIdx.x; p < n; p += (long long)gridDim.x * kB) {
     float sum = 0.f;
+#pragma unroll 8
     for (int j = 0; j < N; j++) sum += vels[(long long)j * n + p];
     mean[p] = sum / N;
   }
@@ -182,13 +208,14 @@ void enkf_ha_perturb(const float* ha, int N, long long nd, double* hap, double* 
 
 void enkf_band(const float* ha, const double* hap, const float* d, const double* e_in, uint64_t seed, double sigma,
                int N, long long nd, double* band, double* t0, hipStream_t s) {
-  hipLaunchKernelGGL(k_band, dim3(nblocks(nd)), dim3(kB), 0, s, ha, hap, d, e_in, seed, sigma, N, nd, band, t0);
+  hipLaunchKernelGGL(k_band, dim3(nblocks(nd * kBandShare)), dim3(kB), 0, s, ha, hap, d, e_in, seed, sigma, N, nd, band, t0);
 }
 
-void enkf_model_update(const float* vels, float* out, long long n, int N, const double* T, float dx, float dt,
+void enkf_model_update(const float* vels, float* out, long long n, int N, const double* T, int ld, float dx, float dt,
                        hipStream_t s) {
   if (N > kMaxMembers) fail(kErrRange, "ensemble larger than the supported maximum");
-  hipLaunchKernelGGL(k_model_update, dim3(nblocks(n, 2048)), dim3(kB), 0, s, vels, out, n, N, T, dx, dt);
+  hipLaunchKernelGGL(k_model_update, dim3(nblocks(n, 2048), ld / kUpdateChunk), dim3(kB), 0, s, vels, out, n, N, T, ld, dx,
+                     dt);
 }
 
 void enkf_member_mean(const float* vels, long long n, int N, float* mean, hipStream_t s) {

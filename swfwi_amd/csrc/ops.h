@@ -87,8 +87,8 @@ void op_axpy1(const float* src, float* dst, long long n, hipStream_t s);
 // C[N][N] (column-major, C[i + N*j]) += sum_r A[i][r] * B[j][r] over rows r,
 // where A and B are E x m matrices stored entry-major (A[i][r] = A + i*m + r,
 // FP32 or FP64 inputs promoted to FP64).  Used for the data-space Gram
-// products of the analysis (enkfanalyze.cpp:420-476).
-void op_gram_f64(const double* A, const double* B, int N, long long m, double* C, hipStream_t s);
+// products of the analysis (enkfanalyze.cpp:420-476).  `part`: workspace.
+void op_gram_f64(const double* A, const double* B, int N, long long m, double* C, DBuf<double>& part, hipStream_t s);
 // model update t5 = A' * T (A' = members - mean, modelSize x N, T N x N).
 void op_apply_nxn(const double* Ap, const double* T, int N, long long n, double* out, hipStream_t s);
 

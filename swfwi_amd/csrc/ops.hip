@@ -438,25 +438,35 @@ __global__ __launch_bounds__(kG2Threads, 4) void k_gram_rows(const double* __res
   }
 }
 
-// sum of the per-block partials in block order; for a symmetric product only
-// the upper-triangle tiles were formed, the lower ones are mirrored
-__global__ void k_gram_mfma_finish(const double* part, int nchunk, int N, bool sym, double* C) {
-  const int NN = N * N;
-  for (int q = blockIdx.x * kB + threadIdx.x; q < NN; q += gridDim.x * kB) {
-    const int i = q % N, j = q / N;
-    const int src = (sym && i / 16 > j / 16) ? j + N * i : q;
-    double s = 0;
-    for (int c = 0; c < nchunk; c++) s += part[(long long)c * NN + src];
-    C[q] = s;
-  }
-}
+// C = the sum of the at most kGramParts partials in their order; for a
+// symmetric product of which only the tiles J >= I were formed the lower ones
+// are mirrored.  A block takes 16 outputs: its 256 threads read all of their
+// partials at once (32 loads in flight a thread) and 16 of them add up from
+// LDS, where one thread an output read and added one by one (60 members, 512
+// partials: 149 us -> 11).
+constexpr int kGramParts = 512;
+constexpr int kFinQ = 16, kFinC = kB / kFinQ;
 
-__global__ void k_gram_finish(const double* part, int nchunk, int NN, double* C) {
-  for (int q = blockIdx.x * kB + threadIdx.x; q < NN; q += gridDim.x * kB) {
-    double s = 0;
-    for (int c = 0; c < nchunk; c++) s += part[(long long)c * NN + q];
-    C[q] = s;
+__global__ void k_gram_finish(const double* __restrict__ part, int nparts, int N, bool sym, double* __restrict__ C) {
+  __shared__ double v[kGramParts][kFinQ];
+  const int NN = N * N, ql = threadIdx.x % kFinQ, c0 = threadIdx.x / kFinQ;
+  const int q = blockIdx.x * kFinQ + ql;
+  const int i = q % N, j = q / N;
+  const int src = (sym && i / 16 > j / 16) ? j + N * i : q;
+  double t[kGramParts / kFinC];
+#pragma unroll
+  for (int k = 0; k < kGramParts / kFinC; k++) {
+    const int c = c0 + k * kFinC;
+    t[k] = q < NN && c < nparts ? part[(long long)c * NN + src] : 0.0;
   }
+#pragma unroll
+  for (int k = 0; k < kGramParts / kFinC; k++) v[c0 + k * kFinC][ql] = t[k];
+  __syncthreads();
+  if (c0 != 0 || q >= NN) return;
+  double s = 0;
+#pragma unroll 16
+  for (int c = 0; c < nparts; c++) s += v[c][ql];
+  C[q] = s;
 }
 
 // out[r][e] ... out is (n x N) entry-major: out[e*n + r] = sum_j Ap[j*n + r] * T[j + N*e]
@@ -627,16 +637,16 @@ double op_launch_latency(int blocks, int reps, bool graph, hipStream_t s) {
   return 1e3 * ms / reps;
 }
 
-void op_gram_f64(const double* A, const double* B, int N, long long m, double* C, hipStream_t s) {
+void op_gram_f64(const double* A, const double* B, int N, long long m, double* C, DBuf<double>& part, hipStream_t s) {
   if (N >= 1 && N <= kGMaxN) {
     // one block per run of rows, two blocks per CU; partials summed in order
-    long long nblk = 512;
+    long long nblk = kGramParts;
     long long rows = (m + nblk - 1) / nblk;
     rows = ((rows + kG2KC - 1) / kG2KC) * kG2KC;
     if (rows < kG2KC) rows = kG2KC;
     nblk = (m + rows - 1) / rows;
     if (nblk < 1) nblk = 1;
-    DBuf<double> part((size_t)nblk * N * N);
+    part.resize((size_t)nblk * N * N);
     const bool sym = A == B;
     if (sym)
       hipLaunchKernelGGL(k_gram_rows<true>, dim3((unsigned)nblk), dim3(kG2Threads), 0, s, A, B, N, m, rows,
@@ -644,9 +654,8 @@ void op_gram_f64(const double* A, const double* B, int N, long long m, double* C
     else
       hipLaunchKernelGGL(k_gram_rows<false>, dim3((unsigned)nblk), dim3(kG2Threads), 0, s, A, B, N, m, rows,
                          part.get());
-    hipLaunchKernelGGL(k_gram_mfma_finish, dim3(nblocks((long long)N * N)), dim3(kB), 0, s, part.get(), (int)nblk, N,
-                       sym, C);
-    SWFWI_HIP(hipStreamSynchronize(s));
+    hipLaunchKernelGGL(k_gram_finish, dim3((N * N + kFinQ - 1) / kFinQ), dim3(kB), 0, s, part.get(), (int)nblk, N, sym,
+                       C);
     return;
   }
   const int nt = (N + kGT - 1) / kGT;
@@ -655,10 +664,10 @@ void op_gram_f64(const double* A, const double* B, int N, long long m, double* C
   chunk = ((chunk + kGK - 1) / kGK) * kGK;
   nchunk = (m + chunk - 1) / chunk;
   if (nchunk < 1) nchunk = 1;
-  DBuf<double> part((size_t)nchunk * N * N);
+  part.resize((size_t)nchunk * N * N);
   hipLaunchKernelGGL(k_gram, dim3(nt, nt, (unsigned)nchunk), dim3(kGT * kGT), 0, s, A, B, N, m, chunk, part.get());
-  hipLaunchKernelGGL(k_gram_finish, dim3(nblocks((long long)N * N)), dim3(kB), 0, s, part.get(), (int)nchunk, N * N, C);
-  SWFWI_HIP(hipStreamSynchronize(s));
+  hipLaunchKernelGGL(k_gram_finish, dim3((N * N + kFinQ - 1) / kFinQ), dim3(kB), 0, s, part.get(), (int)nchunk, N,
+                     false, C);
 }
 void op_apply_nxn(const double* Ap, const double* T, int N, long long n, double* out, hipStream_t s) {
   hipLaunchKernelGGL(k_apply_nxn, dim3(nblocks(n, 2048)), dim3(kB), (size_t)N * N * sizeof(double), s, Ap, T, N, n,
