@@ -298,7 +298,9 @@ class Propagator {
   std::vector<std::unique_ptr<ResLayout>> res_layouts_;
   std::vector<std::unique_ptr<MarchLayout>> march_layouts_;  // by chunk length
   std::vector<long long> src_idx_, rec_idx_;  // grid indices of the points
-  int res_cap_[2][2] = {{-1, -1}, {-1, -1}};  // [kind][precision] blocks on the chip at once
+  int res_cap_[2][2] = {{-1, -1}, {-1, -1}};  // [kind][precision] blocks on the chip at once, one a CU
+  int res_twice_[2][kResTwiceRows + 1] = {};   // [precision][rows a wave] two forward blocks fit a CU: 1, -1, 0 not asked
+  bool res_twice(int rows);
   DBuf<unsigned long long> xbuf_[2];  // exchange words, forward and backward
   unsigned xbase_ = 0;
   DBuf<int> abort_dev_;

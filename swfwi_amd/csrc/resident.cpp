@@ -52,13 +52,21 @@ void Propagator::set_resident(int mode, double wait_us) {
   res_gave_up_ = false;
 }
 
+bool Propagator::res_twice(int rows) {
+  if (rows > kResTwiceRows) return false;
+  int& known = res_twice_[prec_][rows];
+  if (!known) known = resident_per_cu(false, prec_, rows * kResWaves) >= 2 ? 1 : -1;
+  return known == 1;
+}
+
 bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   if (resident_ == 0 || tile_override_ || (kind == 1 && bwd_split_ >= 0) || g_.nt < 2) return false;
   const int most = kind == 1 ? kResMaxWidthBwd : kResMaxWidthFwd;
   int& cap = res_cap_[kind][prec_];
   if (cap < 0) {  // every width's kernel fits at least one block a CU
-    cap = resident_capacity(kind == 1, prec_, 1);
-    for (int w = kResWaves; w <= most; w += kResWaves) cap = std::min(cap, resident_capacity(kind == 1, prec_, w));
+    cap = resident_cus();
+    for (int w = kResWaves; w <= most; w += kResWaves)
+      if (resident_per_cu(kind == 1, prec_, w) < 1) cap = 0;
   }
   const int ux = g_.nxpad - 2 * kHalo, uz = g_.nzpad - 2 * kHalo;
   t.ntz = (uz + kResTileZ - 1) / kResTileZ;
@@ -67,17 +75,29 @@ bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   const int cols = cap / E / t.ntz;  // tile columns of an entry
   if (cols < 1) return false;
   t.w = std::max(kResWaves, (ux + cols - 1) / cols);
+  if (kind == 0) {
+    // Two blocks a CU, one computing while the other waits for its halos,
+    // where that makes no more rows a CU (11 run as 12): 201x301 E=2 2.26 -> 2.05, E=8 3.7 ->
+    // 3.2, E=11 5.3 -> 3.4, E=13 6.1 -> 4.7, E=16 6.2 -> 5.15; 301x921 E=2
+    // 4.1 -> 3.15, E=4 7.1 -> 5.2; 90x120 E=24 3.1 -> 2.6; with a row more
+    // 501x1501 E=1 3.9 -> 4.7, 301x921 E=3 5.1 -> 5.3.  In FP32, where a row
+    // takes less, two tiles of 2 rows for one of 4 lose (201x301 E=5 2.83 ->
+    // 2.93, 250x400 E=3 2.80 -> 2.99; exact 3.02 -> 2.83, 2.94 -> 2.76).
+    const int w2 = std::max(kResWaves, (ux + 2 * cap / E / t.ntz - 1) / (2 * cap / E / t.ntz));
+    const int rows = (t.w + kResWaves - 1) / kResWaves, rows2 = (w2 + kResWaves - 1) / kResWaves;
+    if (2 * rows2 <= rows + (rows == 11) && (prec_ == kExact || rows2 != 2) && res_twice(rows2)) t.w = w2;
+  }
   t.ntx = (ux + t.w - 1) / t.w;
   if (t.w > most) return false;
   if (resident_ == 1) return true;
   if (res_gave_up_) return false;  // the chip is shared: a run of this handle has waited in vain
   // Measured over E (forward / backward microseconds a step, per-step kernels
   // -> resident): 201x301 E=1 4.7 -> 1.74, E=4 4.7 -> 2.7 / 8.1 -> 3.4, E=8
-  // 6.2 -> 3.6 / 10.4 -> 5.2, E=11 6.9 -> 5.3 / 11.4 -> 9.1, E=16 7.9 -> 6.1,
-  // E=21 9.8 -> 8.1; 301x921 E=1 5.2 -> 2.7 / 6.6 -> 3.4; 501x1501 E=1 6.8 ->
-  // 4.0 / 10.4 -> 6.2.  Side by side on streams, 2 to 4 entries of wide tiles
-  // are better left to the per-step kernels (301x921 E=4 5.4 against 7.1,
-  // 501x1501 E=2 7.0 against 7.3).
+  // 6.2 -> 3.2 / 10.4 -> 5.2, E=11 6.9 -> 3.4 / 11.4 -> 9.1, E=16 7.9 -> 5.2,
+  // E=21 9.8 -> 8.1; 301x921 E=1 5.2 -> 2.7 / 6.6 -> 3.4, E=4 5.4 -> 5.2;
+  // 501x1501 E=1 6.8 -> 4.0 / 10.4 -> 6.2.  2 to 4 entries of wide tiles run
+  // faster side by side on streams with a launch a step (501x1501 E=2 7.0
+  // against 7.3).
   return kind == 1 || E == 1 || E > kLanes || t.w <= kResLanesWidth;
 }
 

@@ -39,6 +39,7 @@ constexpr int kResMaxPts = 512;             // sources or receivers of one tile,
 constexpr int kResMaxWidthFwd = 128;        // widest tile (x)
 constexpr int kResMaxWidthBwd = 80;          // (spills from 57 columns on; 69 columns still 9.1 against 11.4 us per step)
 constexpr int kResLanesWidth = 80;           // widest for 2 to 4 forward entries
+constexpr int kResTwiceRows = 6;             // most rows a wave of which two forward blocks fit a CU
 
 // Tiles of one entry: w x h outputs each (the last column and row may be smaller).
 struct ResTiles {
@@ -117,8 +118,9 @@ struct ResBwdArgs {
   long long gstride = 0;
 };
 
-// Blocks of the resident kernel for tile width w that fit the device at once (0: none).
-int resident_capacity(bool backward, int precision, int w);
+// CUs of the device, and blocks of the kernel for tile width w that fit one at once (0: none).
+int resident_cus();
+int resident_per_cu(bool backward, int precision, int w);
 void launch_resident_fwd(const ResFwdArgs& a, int precision, hipStream_t s);
 void launch_resident_bwd(const ResBwdArgs& a, int precision, hipStream_t s);
 

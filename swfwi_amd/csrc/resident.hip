@@ -377,8 +377,10 @@ constexpr int edge_share(int w, int NT) {
   return ((w <= 12 ? w * kResTileZ : 12 * kResTileZ + (w - 12) * 12) + NT - 1) / NT;
 }
 
+// (tiles of up to kResTwiceRows rows a wave in 128 registers, so that two
+// blocks fit a CU; 5 and 6 rows spill 3 and 23 of them)
 template <int P, int R, int NW>
-__global__ __launch_bounds__(64 * NW) void k_resident_fwd(ResFwdArgs a) {
+__global__ __launch_bounds__(64 * NW, R <= kResTwiceRows ? 4 : 2) void k_resident_fwd(ResFwdArgs a) {
   constexpr int NX = NW * R + 12;
   __shared__ float cur[NX * LZ];
   __shared__ float ub[2 * NW * 64];
@@ -710,16 +712,21 @@ bool with_kernel(int precision, int w, F&& fn) {
 
 }  // namespace
 
-int resident_capacity(bool backward, int precision, int w) {
-  int dev = 0, cus = 0, per = 0;
+int resident_cus() {
+  int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return 0;
+  return cus;
+}
+
+int resident_per_cu(bool backward, int precision, int w) {
+  int per = 0;
   auto ask = [&](auto k, int threads) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, threads, 0) != hipSuccess) per = 0;
   };
   const bool ok = backward ? with_kernel<true>(precision, w, ask) : with_kernel<false>(precision, w, ask);
-  return ok && per > 0 ? cus : 0;  // one block per CU: more would share its SIMDs
+  return ok ? per : 0;
 }
 
 void launch_resident_fwd(const ResFwdArgs& a, int precision, hipStream_t s) {
