@@ -494,6 +494,9 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
                          Fields& w, int rvdiv) {
   const long long np = g_.npts();
   w.ensure(E, np, true);
+  ResTiles rt;
+  if (band && plan_parts(0, E, rt) && !plan_parts(1, E, rt))
+    tile_choice(1, E, rv, rvstride, rvdiv, w, true);  // for the backward, while the workspace is free
   if (resident_forward(E, rv, rvstride, src, dcal, band, w, rvdiv)) {
     // (the widths a run of this size would fall back to, untimed)
     tile_choice(0, E, rv, rvstride, rvdiv, w, false);

@@ -230,7 +230,9 @@ class Propagator {
   // (strips, chunks, points by unit) for a batch of E entries.
   const MarchLayout* march_layout(int E);
   ResGrid res_grid(const ResTiles& t) const;
-  void res_begin(int kind, int E, ResComm& x);  // call with the device's lock held
+  int plan_parts(int kind, int E, ResTiles& t);  // the launches a run takes, one after the other (0: not resident), and their tiles
+  void res_begin(int kind, int E, int parts, ResComm& x);  // call with the device's lock held; E: most entries of a launch
+  void res_part(int kind, int E, ResComm& x);  // before each launch
   bool res_end(int kind, long long steps, hipEvent_t t0);
   bool resident_forward(int E, const float* rv, long long rvstride, const Sources& src, float* dcal, float* band,
                         Fields& w, int rvdiv);

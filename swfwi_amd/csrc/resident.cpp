@@ -59,6 +59,35 @@ bool Propagator::res_twice(int rows) {
   return known == 1;
 }
 
+// A batch too large for the chip, or one whose tiles would be very wide, is
+// faster as two or three resident launches one after the other, each with
+// tiles of a size that costs least a row.  Measured, microseconds a step.
+// Forward, a launch a step -> in parts: 201x301 E=22 10.0 -> 6.7, E=26 10.7 ->
+// 9.1, E=33 12.1 -> 10.1, 301x921 E=8 11.9 -> 10.1, 90x120 E=80 10.4 -> 7.9,
+// E=100 11.0 -> 6.8; E=20 as one launch of 16 rows 8.65 -> 7.6 (of 14 rows, 10
+// entries of 250x500, 7.07 -> 7.3).  Parts of 9 rows a wave lose: 301x921 E=5
+// 9.4 -> 10.0 (in three of 3 rows 8.35).  Three parts pay at 4 rows, in exact
+// mode also at 3 (250x500 E=12 10.0 -> 9.7, in FP32 9.35 -> 10.15); 301x921
+// E=12 in FP32, 6 rows, 13.6 -> 14.3.  Backward: 201x301 E=13 12.6 -> 9.2,
+// E=16 13.7 -> 10.4, E=22 17.9 -> 15.5, 301x921 E=6 19.1 -> 15.5, 90x120
+// E=100 20.6 -> 18.4; one launch of 10 rows 12.4 -> 9.2 (90x120 E=60), of 9
+// rows the same, of 8 rows 7.8 -> 8.1 (201x301 E=10).
+int Propagator::plan_parts(int kind, int E, ResTiles& t) {
+  const auto rows = [](const ResTiles& r) { return (r.w + kResWaves - 1) / kResWaves; };
+  const bool one = plan_resident(kind, E, t);
+  if (resident_ == 1) return one ? 1 : 0;
+  if (one && rows(t) < (kind == 1 ? kResWideBwd : kResWideFwd)) return 1;
+  for (int n = 2; n <= kResMaxParts && n < E; n++) {
+    ResTiles p;
+    if (!plan_resident(kind, (E + n - 1) / n, p)) continue;
+    const int r = rows(p);
+    if (kind == 1 || n == 2 ? r > kResPartRows : r != 4 && (prec_ != kExact || r != 3)) continue;
+    t = p;
+    return n;
+  }
+  return one ? 1 : 0;
+}
+
 bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   if (resident_ == 0 || tile_override_ || (kind == 1 && bwd_split_ >= 0) || g_.nt < 2) return false;
   const int most = kind == 1 ? kResMaxWidthBwd : kResMaxWidthFwd;
@@ -136,7 +165,7 @@ ResGrid Propagator::res_grid(const ResTiles& t) const {
   return g;
 }
 
-void Propagator::res_begin(int kind, int E, ResComm& x) {
+void Propagator::res_begin(int kind, int E, int parts, ResComm& x) {
   hipStream_t s = stream();
   if (!abort_host_) {
     SWFWI_HIP(hipHostMalloc(reinterpret_cast<void**>(&abort_host_), sizeof(int), hipHostMallocMapped));
@@ -151,8 +180,7 @@ void Propagator::res_begin(int kind, int E, ResComm& x) {
   const size_t words = (size_t)(kind == 1 ? 3 : 2) * E * (size_t)g_.npts();
   if (kind == 1) {
     buf.resize(std::max(words, buf.size()));
-    launch_fill_u32(reinterpret_cast<unsigned*>(buf.get()), 2 * (long long)words, 0xffffffffu, s);  // empty
-  } else if (words > buf.size() || xbase_ > 0xffffffffu - (unsigned)g_.nt - 2) {
+  } else if (words > buf.size() || (unsigned long long)xbase_ + (g_.nt + 1ull) * parts > 0xffffffffull) {
     // no word of the buffer carries a stamp of this run: stamps grow, and the
     // words are cleared when the buffer is new or the stamps would wrap
     buf.resize(std::max(words, buf.size()));
@@ -164,13 +192,20 @@ void Propagator::res_begin(int kind, int E, ResComm& x) {
     *abort_host_ = 0;
   }
   x.buf = buf.get();
-  x.base = xbase_;
-  if (kind == 0) xbase_ += (unsigned)g_.nt + 1;
   x.abort_dev = abort_dev_.get();
   void* mapped = nullptr;
   SWFWI_HIP(hipHostGetDevicePointer(&mapped, abort_host_, 0));
   x.abort_host = static_cast<int*>(mapped);
   x.limit = (long long)(res_wait_us_ * ticks_per_us_);
+}
+
+void Propagator::res_part(int kind, int E, ResComm& x) {
+  if (kind == 1) {
+    launch_fill_u32(reinterpret_cast<unsigned*>(x.buf), 2 * 3 * E * g_.npts(), 0xffffffffu, stream());  // empty
+  } else {
+    x.base = xbase_;
+    xbase_ += (unsigned)g_.nt + 1;
+  }
 }
 
 bool Propagator::res_end(int kind, long long steps, hipEvent_t t0) {
@@ -197,14 +232,16 @@ bool Propagator::res_end(int kind, long long steps, hipEvent_t t0) {
 bool Propagator::resident_forward(int E, const float* rv, long long rvstride, const Sources& src, float* dcal,
                                   float* band, Fields& w, int rvdiv) {
   ResTiles t;
-  if (!plan_resident(0, E, t)) return false;
+  const int parts = plan_parts(0, E, t);
+  if (parts < 1) return false;
   ResLayout& l = res_layout(t);
   if (!l.fits) return false;
   hipStream_t s = stream();
   const long long np = g_.npts();
   std::lock_guard<std::mutex> lock(device_lock(dev_));
   ResFwdArgs a;
-  res_begin(0, E, a.x);
+  const int part = (E + parts - 1) / parts;
+  res_begin(0, part, parts, a.x);
   hipEvent_t t0 = nullptr;
   if (timing_) {
     t0 = pooled_event();
@@ -222,7 +259,6 @@ bool Propagator::resident_forward(int E, const float* rv, long long rvstride, co
   inj.t = 0;
   launch_point_inject(w.b.get(), np, inj, g_.ns(), E, s);
   a.g = res_grid(t);
-  a.E = E;
   a.nt = g_.nt;
   a.fstride = np;
   a.fa = w.a.get();
@@ -241,7 +277,12 @@ bool Propagator::resident_forward(int E, const float* rv, long long rvstride, co
   a.ng = g_.ng();
   a.band = band;
   a.bsize = g_.bsize;
-  launch_resident_fwd(a, prec_, s);
+  for (int e = 0; e < E; e += part) {
+    a.g.e0 = e;
+    a.E = std::min(part, E - e);
+    res_part(0, a.E, a.x);
+    launch_resident_fwd(a, prec_, s);
+  }
   return res_end(0, g_.nt, t0);
 }
 
@@ -249,7 +290,8 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
                                    long long vstride, const float* band, float* grad, long long gstride, Fields& w,
                                    int rvdiv, int it_min, const std::vector<float>& wts) {
   ResTiles t;
-  if (!plan_resident(1, E, t)) return false;
+  const int parts = plan_parts(1, E, t);
+  if (parts < 1) return false;
   ResLayout& l = res_layout(t);
   if (!l.fits) return false;
   hipStream_t s = stream();
@@ -261,7 +303,8 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
   }
   std::lock_guard<std::mutex> lock(device_lock(dev_));
   ResBwdArgs a;
-  res_begin(1, E, a.x);
+  const int part = (E + parts - 1) / parts;
+  res_begin(1, part, parts, a.x);
   hipEvent_t t0 = nullptr;
   if (timing_) {
     t0 = pooled_event();
@@ -277,7 +320,6 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
   ginj.t = nt - 1;
   launch_point_inject(w.spare0, np, ginj, ng, E, s);
   a.g = res_grid(t);
-  a.E = E;
   a.nt = nt;
   a.it_min = it_min;
   a.fstride = np;
@@ -302,7 +344,12 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
   a.weights = res_wts_.get();
   a.grad = grad;
   a.gstride = gstride;
-  launch_resident_bwd(a, prec_, s);
+  for (int e = 0; e < E; e += part) {
+    a.g.e0 = e;
+    a.E = std::min(part, E - e);
+    res_part(1, a.E, a.x);
+    launch_resident_bwd(a, prec_, s);
+  }
   return res_end(1, nt - it_min, t0);
 }
 

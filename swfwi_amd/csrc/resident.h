@@ -23,7 +23,8 @@
 // flag that every waiting block polls, all blocks then leave, and the caller
 // runs the per-step kernels instead.  The launch needs every block on the chip
 // at once; the host checks the blocks against the device's capacity and lets
-// one resident run at a time onto a device.
+// one resident run at a time onto a device.  A batch that does not fit goes as
+// two or three launches of a part of its entries each, over one buffer.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -40,6 +41,10 @@ constexpr int kResMaxWidthFwd = 128;        // widest tile (x)
 constexpr int kResMaxWidthBwd = 80;          // (spills from 57 columns on; 69 columns still 9.1 against 11.4 us per step)
 constexpr int kResLanesWidth = 80;           // widest for 2 to 4 forward entries
 constexpr int kResTwiceRows = 6;             // most rows a wave of which two forward blocks fit a CU
+
+constexpr int kResMaxParts = 3;               // most launches of one run
+constexpr int kResWideFwd = 15, kResWideBwd = 10;  // rows a wave from which parts are faster than one launch
+constexpr int kResPartRows = 7;               // most rows a wave of a part
 
 // Tiles of one entry: w x h outputs each (the last column and row may be smaller).
 struct ResTiles {
@@ -69,12 +74,13 @@ struct ResGrid {
   const float* delta_x = nullptr;
   const float* delta_z = nullptr;
   ResTiles t;
+  int e0 = 0;  // the launch takes the entries from here on; the exchange counts from it
 };
 
 struct ResFwdArgs {
   ResGrid g;
   ResComm x;
-  int E = 1, nt = 0;
+  int E = 1, nt = 0;  // (E: entries of this launch)
   long long fstride = 0;
   float* fa = nullptr;  // in: p(-1); the two then hold p(nt-1) and p(nt) as the per-step loop leaves them
   float* fb = nullptr;  // in: p(0)

@@ -72,8 +72,9 @@ template <int NW>
 __device__ __forceinline__ Place place(const ResGrid& g, int rows) {
   Place p;
   const int nt = g.t.ntx * g.t.ntz;
-  p.e = blockIdx.x / nt;
-  p.tile = blockIdx.x - p.e * nt;
+  const int e = blockIdx.x / nt;
+  p.e = g.e0 + e;
+  p.tile = blockIdx.x - e * nt;
   const int tx = p.tile / g.t.ntz, tz = p.tile - tx * g.t.ntz;
   p.x0 = kHalo + tx * g.t.w;
   p.z0 = kHalo + tz * g.t.h;
@@ -434,6 +435,7 @@ __global__ __launch_bounds__(64 * NW, R <= kResTwiceRows ? 4 : 2) void k_residen
   Halo<NH> hp;
   halo_points<64 * NW, NH>(g, p, hp);
   const long long words = (long long)a.E * a.fstride;  // of one parity
+  const long long xo = (long long)(p.e - g.e0) * a.fstride;
   __syncthreads();
   const bool chains = shared != 0;
 
@@ -460,7 +462,7 @@ __global__ __launch_bounds__(64 * NW, R <= kResTwiceRows ? 4 : 2) void k_residen
     __syncthreads();
     ring_rows<NW, R>(p, u, ub);
     const unsigned stamp = a.x.base + (unsigned)it + 1;
-    u64* words_now = a.x.buf + ((it + 1) & 1) * words + fo;
+    u64* words_now = a.x.buf + ((it + 1) & 1) * words + xo;
     const bool more = it + 1 < a.nt;
 #pragma unroll
     for (int k = 0; k < R; k++) {
@@ -575,7 +577,7 @@ __device__ __forceinline__ void bwd_half(const ResBwdArgs& a, BwdTile<P, R>& t) 
   halo_points<NT, NH>(g, p, hp);
   edge_points<NT, NE>(g, p, ep);
   const long long copy = (long long)a.E * a.fstride;  // words of one of the three copies
-  u64* words = a.x.buf + fo;
+  u64* words = a.x.buf + (long long)(p.e - g.e0) * a.fstride;
   int turn = 0;  // the copy that the field being formed goes to
   __syncthreads();
   const bool chains = t.shared[F] != 0;
