@@ -153,8 +153,8 @@ int swfwi_solver_set_bwd_split(swfwi_solver h, int mode);
  * larger ones as two or three, a part of the batch each), 0 never,
  * 1 wherever the tiles fit.  wait_us bounds how long a block of that launch
  * waits for its neighbours (5e5 by default) before the run is done again with
- * one launch per step (and, by rule, so are the handle's later runs).  A fixed tile width or backward form also means one
- * launch per step.  Same results. */
+ * one launch per step (and, by rule, so are the handle's later runs).  A fixed
+ * tile width or backward form also means one launch per step.  Same results. */
 int swfwi_solver_set_resident(swfwi_solver h, int mode, double wait_us);
 /* Record a HIP event pair around every forward / backward time loop on the
  * handle's stream (graph replays included); swfwi_solver_kernel_times waits
