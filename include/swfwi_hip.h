@@ -150,7 +150,7 @@ int swfwi_solver_get_tile_x(swfwi_solver h, int kind, int entries, int *tile_x);
 int swfwi_solver_set_bwd_split(swfwi_solver h, int mode);
 /* The resident time loop: -1 by rule (the default: batches small enough to
  * keep their tiles on the chip run a whole time loop as one launch, somewhat
- * larger ones as two or three, a part of the batch each), 0 never,
+ * larger ones as a few, a part of the batch each), 0 never,
  * 1 wherever the tiles fit.  wait_us bounds how long a block of that launch
  * waits for its neighbours (5e5 by default) before the run is done again with
  * one launch per step (and, by rule, so are the handle's later runs).  A fixed

@@ -130,8 +130,8 @@ class Propagator {
   static int xcorr_range(float dt, int nt, std::vector<float>& weights);
 
   // The resident time loop (resident.h): -1 by rule (the default: batches
-  // whose tiles fit the chip, as a whole or in two or three parts), 0 never, 1 wherever it fits.  wait_us bounds
-  // one wait of a block for its neighbours, after which the run is done again
+  // whose tiles fit the chip, as a whole or in parts), 0 never, 1 wherever
+  // it fits.  wait_us bounds one wait of a block for its neighbours, after which the run is done again
   // by the per-step kernels.  A fixed tile width or backward form also
   // means the per-step kernels.
   void set_resident(int mode, double wait_us);

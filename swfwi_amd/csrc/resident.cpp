@@ -60,7 +60,7 @@ bool Propagator::res_twice(int rows) {
 }
 
 // A batch too large for the chip, or one whose tiles would be very wide, is
-// faster as two or three resident launches one after the other, each with
+// faster as a few resident launches one after the other, each with
 // tiles of a size that costs least a row.  Measured, microseconds a step.
 // Forward, a launch a step -> in parts: 201x301 E=22 10.0 -> 6.7, E=26 10.7 ->
 // 9.1, E=33 12.1 -> 10.1, 301x921 E=8 11.9 -> 10.1, 90x120 E=80 10.4 -> 7.9,
@@ -72,12 +72,15 @@ bool Propagator::res_twice(int rows) {
 // E=16 13.7 -> 10.4, E=22 17.9 -> 15.5, 301x921 E=6 19.1 -> 15.5, 90x120
 // E=100 20.6 -> 18.4; one launch of 10 rows 12.4 -> 9.2 (90x120 E=60), of 9
 // rows the same, of 8 rows 7.8 -> 8.1 (201x301 E=10).
+// More parts pay backward only: 201x301 E=32 24.8 -> 20.9, E=60 46.9 -> 43.5,
+// 301x921 E=8 23.7 -> 20.3, E=13 35.2 -> 35.3, E=16 43.6 -> 40.6, 90x120 E=200
+// 41.9 -> 31.3; forward the strip walk has caught up (201x301 E=40: 14.0).
 int Propagator::plan_parts(int kind, int E, ResTiles& t) {
   const auto rows = [](const ResTiles& r) { return (r.w + kResWaves - 1) / kResWaves; };
   const bool one = plan_resident(kind, E, t);
   if (resident_ == 1) return one ? 1 : 0;
   if (one && rows(t) < (kind == 1 ? kResWideBwd : kResWideFwd)) return 1;
-  for (int n = 2; n <= kResMaxParts && n < E; n++) {
+  for (int n = 2; n <= (kind == 1 ? kResMaxPartsBwd : kResMaxPartsFwd) && n < E; n++) {
     ResTiles p;
     if (!plan_resident(kind, (E + n - 1) / n, p)) continue;
     const int r = rows(p);

@@ -24,7 +24,7 @@
 // runs the per-step kernels instead.  The launch needs every block on the chip
 // at once; the host checks the blocks against the device's capacity and lets
 // one resident run at a time onto a device.  A batch that does not fit goes as
-// two or three launches of a part of its entries each, over one buffer.
+// a few launches of a part of its entries each, over one buffer.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -42,7 +42,7 @@ constexpr int kResMaxWidthBwd = 80;          // (spills from 57 columns on; 69 c
 constexpr int kResLanesWidth = 80;           // widest for 2 to 4 forward entries
 constexpr int kResTwiceRows = 6;             // most rows a wave of which two forward blocks fit a CU
 
-constexpr int kResMaxParts = 3;               // most launches of one run
+constexpr int kResMaxPartsFwd = 3, kResMaxPartsBwd = 8;  // most launches of one run
 constexpr int kResWideFwd = 15, kResWideBwd = 10;  // rows a wave from which parts are faster than one launch
 constexpr int kResPartRows = 7;               // most rows a wave of a part
 

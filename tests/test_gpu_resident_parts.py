@@ -1,4 +1,4 @@
-"""Batches that run as two or three resident launches, one after the other: the
+"""Batches that run as several resident launches, one after the other: the
 same bits as one launch per step, also where the last part is smaller, where a
 part spans two models and where the backward's parts are not the forward's."""
 import numpy as np
@@ -20,7 +20,8 @@ def need_gpu():
 
 @pytest.mark.parametrize("precision", [capi.PREC_EXACT, capi.PREC_FP32])
 @pytest.mark.parametrize("ns,nx,nz", [(13, 301, 201), (17, 301, 201), (33, 301, 201), (5, 921, 301), (8, 921, 301),
-                                      (60, 120, 90), (79, 120, 90)])
+                                      (60, 120, 90), (79, 120, 90),
+                                      (39, 301, 201), (63, 301, 201)])
 def test_parts_match_the_per_step_kernels(ns, nx, nz, precision):
     case = acquisition(nx, nz, 20)
     sx = np.linspace(1, nx - 2, ns).astype(np.int32)
