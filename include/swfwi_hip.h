@@ -156,6 +156,13 @@ int swfwi_solver_set_bwd_split(swfwi_solver h, int mode);
  * one launch per step (and, by rule, so are the handle's later runs).  A fixed
  * tile width or backward form also means one launch per step.  Same results. */
 int swfwi_solver_set_resident(swfwi_solver h, int mode, double wait_us);
+/* How the last run of a kind (0 forward, 1 backward) went: route 0 none yet, 1
+ * one tiled launch per step, 2 the entries side by side on streams of their
+ * own, 3 one strip-walking launch per step, 4 resident; its step or resident
+ * launches; and the tile width, the rows a strip walk takes or the width of a
+ * resident tile.  gave_up: resident runs of this handle whose wait ran out.
+ * Any pointer may be null. */
+int swfwi_solver_last_run(swfwi_solver h, int kind, int *route, int *launches, int *width, long long *gave_up);
 /* Record a HIP event pair around every forward / backward time loop on the
  * handle's stream (graph replays included); swfwi_solver_kernel_times waits
  * for them and returns the accumulated milliseconds and step-kernel launch

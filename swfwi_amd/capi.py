@@ -61,6 +61,7 @@ SIGNATURES = {
     "swfwi_solver_time_steps": (_I, [_VP, _I, _I, _I, _I, C.POINTER(_F)]),
     "swfwi_solver_set_bwd_split": (_I, [_VP, _I]),
     "swfwi_solver_set_resident": (_I, [_VP, _I, C.c_double]),
+    "swfwi_solver_last_run": (_I, [_VP, _I, C.POINTER(_I), C.POINTER(_I), C.POINTER(_I), C.POINTER(C.c_longlong)]),
     "swfwi_enkf_create": (_I, [C.POINTER(_VP), _VP, _f32, _f32, _F, _I]),
     "swfwi_enkf_destroy": (_I, [_VP]),
     "swfwi_enkf_set_members": (_I, [_VP, _f32]),
@@ -301,6 +302,15 @@ class Solver:
         """The resident time loop: -1 by rule, 0 never, 1 wherever it fits;
         wait_us bounds one wait of a block before the per-step launches take over."""
         check(load().swfwi_solver_set_resident(self.h, int(mode), float(wait_us)))
+
+    ROUTES = ("none", "per step", "side by side", "strips", "resident")
+
+    def last_run(self, kind):
+        """(route, launches, tile width or rows, waits that ran out so far) of
+        the last forward (0) or backward (1) run."""
+        r, n, w, g = _I(0), _I(0), _I(0), C.c_longlong(0)
+        check(load().swfwi_solver_last_run(self.h, kind, C.byref(r), C.byref(n), C.byref(w), C.byref(g)))
+        return self.ROUTES[r.value], n.value, w.value, g.value
 
     def time_steps(self, kind, entries, tile_x, reps=100):
         """Microseconds per launch of back-to-back step kernels on scratch fields."""

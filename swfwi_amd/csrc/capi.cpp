@@ -427,6 +427,18 @@ int swfwi_solver_set_resident(swfwi_solver h, int mode, double wait_us) {
   });
 }
 
+int swfwi_solver_last_run(swfwi_solver h, int kind, int* route, int* launches, int* width, long long* gave_up) {
+  return guarded([&] {
+    NEED(h);
+    if (kind != 0 && kind != 1) fail(kErrArg, "kind must be 0 (forward) or 1 (backward)");
+    const Propagator& p = h->s->prop();
+    if (route) *route = p.last_run[kind].route;
+    if (launches) *launches = p.last_run[kind].launches;
+    if (width) *width = p.last_run[kind].width;
+    if (gave_up) *gave_up = p.gave_up;
+  });
+}
+
 int swfwi_solver_set_bwd_split(swfwi_solver h, int mode) {
   return guarded([&] {
     NEED(h);

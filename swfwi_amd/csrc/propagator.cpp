@@ -507,6 +507,7 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
     fwd_point_updates += (double)E * (g_.nxpad - 2 * kHalo) * (g_.nzpad - 2 * kHalo) * g_.nt;
     return;
   }
+  int tw1 = 0;  // the lanes' tile width
   const bool lanes = E >= 2 && E <= kLanes && band == nullptr;
   // tile widths for this batch, chosen now while the workspace is free
   // (backward() runs on the state this forward leaves behind)
@@ -542,7 +543,7 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
     // buffers (the same rotation, so the batch's final state is unchanged);
     // the lanes start after the work queued so far and the main stream
     // continues after all of them
-    const int tw1 = tile_choice(0, 1, rv, rvstride, rvdiv, w, false);
+    tw1 = tile_choice(0, 1, rv, rvstride, rvdiv, w, false);
     hipStream_t main = stream();
     SWFWI_HIP(hipEventRecord(lane_events_[0], main));
     for (int e = 0; e < E; e++) {
@@ -569,12 +570,16 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
   }
   const std::vector<FwdLaunch> plan = plan_forward(w);  // sets the final state
   flush_timing_if_full();
+  last_run[0] = lanes   ? LastRun{kSideBySide, E * g_.nt, kTileWidths[tw1]}
+                : march ? LastRun{kStripWalk, g_.nt, march->m.rows}
+                        : LastRun{kPerStep, g_.nt, kTileWidths[tw]};
   fwd_launches += (long long)plan.size() * (lanes ? E : 1);
   fwd_point_updates += (double)E * (g_.nxpad - 2 * kHalo) * (g_.nzpad - 2 * kHalo) * g_.nt;
 }
 
 void Propagator::forward_external(const float* rv, const Sources& src, float* dcal, float* fa, float* fb) {
   forward_body(1, rv, 0, src, dcal, nullptr, fa, fb, 1, fixed_width(0, 1), stream());
+  last_run[0] = LastRun{kPerStep, g_.nt, kTileWidths[fixed_width(0, 1)]};
   fwd_launches += g_.nt;
   fwd_point_updates += (double)(g_.nxpad - 2 * kHalo) * (g_.nzpad - 2 * kHalo) * g_.nt;
 }
@@ -724,6 +729,7 @@ int Propagator::backward(int E, const float* rv, long long rvstride, const Sourc
     backward_body(E, rv, rvstride, src, vsrc, vstride, band, grad, gstride, w, rvdiv, it_min, wts, tw);
   }, stream());
   flush_timing_if_full();
+  last_run[1] = LastRun{kPerStep, iters, kTileWidths[tw]};
   bwd_launches += iters;
   bwd_point_updates += 2.0 * E * (g_.nxpad - 2 * kHalo) * (g_.nzpad - 2 * kHalo) * iters;
   return iters;

@@ -136,6 +136,17 @@ class Propagator {
   // means the per-step kernels.
   void set_resident(int mode, double wait_us);
 
+  // How the last run of a kind (0 forward, 1 backward) went: its launches of
+  // the step (or resident) kernel and the tile width, rows of a strip walk's
+  // chunk or width of a resident tile.  gave_up: resident runs of this handle
+  // whose wait ran out.
+  enum Route { kNoRun = 0, kPerStep = 1, kSideBySide = 2, kStripWalk = 3, kResident = 4 };
+  struct LastRun {
+    int route = kNoRun, launches = 0, width = 0;
+  };
+  LastRun last_run[2];
+  long long gave_up = 0;
+
   // step counters for throughput accounting (a resident loop counts its steps)
   long long fwd_launches = 0, bwd_launches = 0;
   double fwd_point_updates = 0, bwd_point_updates = 0;

@@ -220,7 +220,10 @@ bool Propagator::res_end(int kind, long long steps, hipEvent_t t0) {
   SWFWI_HIP(hipGetLastError());
   SWFWI_HIP(hipStreamSynchronize(stream()));
   const bool ok = *static_cast<volatile int*>(abort_host_) == 0;
-  if (!ok) res_gave_up_ = true;
+  if (!ok) {
+    res_gave_up_ = true;
+    gave_up++;
+  }
   if (timing_) {
     if (ok) {
       pending_.push_back(TimedLoop{t0, t1, kind, steps});
@@ -286,7 +289,9 @@ bool Propagator::resident_forward(int E, const float* rv, long long rvstride, co
     res_part(0, a.E, a.x);
     launch_resident_fwd(a, prec_, s);
   }
-  return res_end(0, g_.nt, t0);
+  if (!res_end(0, g_.nt, t0)) return false;
+  last_run[0] = LastRun{kResident, (E + part - 1) / part, t.w};
+  return true;
 }
 
 bool Propagator::resident_backward(int E, const float* rv, long long rvstride, const Sources& src, const float* vsrc,
@@ -353,7 +358,9 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
     res_part(1, a.E, a.x);
     launch_resident_bwd(a, prec_, s);
   }
-  return res_end(1, nt - it_min, t0);
+  if (!res_end(1, nt - it_min, t0)) return false;
+  last_run[1] = LastRun{kResident, (E + part - 1) / part, t.w};
+  return true;
 }
 
 }  // namespace swfwi
