@@ -370,19 +370,39 @@ int Propagator::xcorr_range(float dt, int nt, std::vector<float>& weights) {
   return it_min;
 }
 
-const Propagator::MarchLayout* Propagator::march_layout(int E) {
+// Measured, microseconds a step, tiled kernel -> strip walks of 14 / 22 rows,
+// exact mode: 12 entries of 301x921 (35000 strip rows) 16.1 -> 15.4 / 16.6, 60
+// members of 201x301 (41000) 20.8 -> 17.1 / 17.7, 16 of 301x921 (47000) 19.9 ->
+// 18.5 / 19.4, 8 of 501x1501 (62000) 21.6 -> 21.9 / 20.6, 60 of 301x921 (177000,
+// runs of 400 steps) 56 -> 47.3 / 46.3 (30 rows 47.1, 10 rows 50.6); below, too
+// few waves walk too long: 22 entries of 201x301 (15000) 10.1 -> 12.1 (9.8 at 8
+// rows), 6 of 301x921 (18000) 10.3 -> 12.1.
+// A strip's row costs the same however few of its 116 z are outputs, a column
+// of tiles by its number of 64-z tiles, so what counts is tiles per strip.
+// Speedup over the tiled kernel (update regions of 400 and 1100 columns, both
+// modes) at 31000 / 62000 / 110000 / 200000 strip rows: 2 tiles a strip 0.97-1.10
+// / 1.04-1.30 / 1.00-1.25 / 1.00-1.37, 1.8 tiles 0.94-0.99 / 1.02-1.07 / 0.98-1.02 /
+// 0.98-1.08, 1.75 tiles 0.92-1.00 / 0.99-1.10 / 0.95-1.02 / 0.98-1.10, 1.5 tiles
+// 0.80-0.94 / 0.91-1.06 / 0.90-1.00 / 0.90-1.11, one tile 0.70-0.82 / 0.78-0.91 /
+// 0.77-0.88 / 0.82-0.92.
+// Entries with models of their own stream a third array, and the tiled kernel's
+// order (chunks of tile columns, entry by entry) keeps more of it in L2: 2 tiles
+// a strip 1.02-1.09 / 0.99-1.12 at 31000 / 62000 strip rows, then 0.95-1.09 at
+// 80000, 0.89-1.08 at 110000, 0.92-1.00 at 200000; 1.8 tiles 0.96-0.97 at 45000.
+bool Propagator::strips_pay(int E, int per_model) const {
   const int ux = g_.nxpad - 2 * kHalo, uz = g_.nzpad - 2 * kHalo;
-  if (tile_override_ || g_.npts() >= (1LL << 29)) return nullptr;
   const int nstrip = (uz + kMarchStrip - 1) / kMarchStrip;
   const long long strip_rows = (long long)E * nstrip * ux;
-  // Measured (microseconds a step, tiled kernel -> strip walks of 14 / 22 rows,
-  // exact mode): 12 entries of 301x921 (35000 strip rows) 16.1 -> 15.4 / 16.6,
-  // 60 members of 201x301 (41000) 20.8 -> 17.1 / 17.7, 16 of 301x921 (47000)
-  // 19.9 -> 18.5 / 19.4, 8 of 501x1501 (62000) 21.6 -> 21.9 / 20.6, 60 of
-  // 301x921 (177000) 56 -> 47.3 / 46.3 (30 rows 47.1, 10 rows 50.6); below, too
-  // few waves walk too long: 22 entries of 201x301 (15000) 10.1 -> 12.1 (9.8 at
-  // 8 rows), 6 of 301x921 (18000) 10.3 -> 12.1.
-  if (strip_rows < kMarchFrom) return nullptr;
+  if (per_model < kMarchShared) return g_.ntz >= 2 * nstrip && strip_rows >= kMarchFrom && strip_rows <= kMarchOwnTo;
+  if (g_.ntz >= 2 * nstrip) return strip_rows >= kMarchFrom;
+  return 5 * g_.ntz >= 9 * nstrip && strip_rows >= 2 * kMarchFrom;
+}
+
+const Propagator::MarchLayout* Propagator::march_layout(int E, int per_model) {
+  const int ux = g_.nxpad - 2 * kHalo, uz = g_.nzpad - 2 * kHalo;
+  if (tile_override_ || g_.npts() >= (1LL << 29) || !strips_pay(E, per_model)) return nullptr;
+  const int nstrip = (uz + kMarchStrip - 1) / kMarchStrip;
+  const long long strip_rows = (long long)E * nstrip * ux;
   const int rows = strip_rows < 2 * kMarchFrom ? 14 : 22;
   for (const auto& l : march_layouts_)
     if (l->m.rows == rows) return l->fits ? l.get() : nullptr;
@@ -511,7 +531,7 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
   const bool lanes = E >= 2 && E <= kLanes && band == nullptr;
   // tile widths for this batch, chosen now while the workspace is free
   // (backward() runs on the state this forward leaves behind)
-  const MarchLayout* march = lanes ? nullptr : march_layout(E);
+  const MarchLayout* march = lanes ? nullptr : march_layout(E, rvstride == 0 ? E : rvdiv);
   const int tw = tile_choice(0, E, rv, rvstride, rvdiv, w, !march);
   tile_choice(1, E, rv, rvstride, rvdiv, w, true);
   const uintptr_t key[] = {1,

@@ -237,9 +237,11 @@ class Propagator {
     ResPoints rec() const { return ResPoints{rptr.get(), ritems.get()}; }
   };
   ResLayout& res_layout(const ResTiles& t);
-  // The strip-walking forward step: whether a batch takes it, and its work
-  // (strips, chunks, points by unit) for a batch of E entries.
-  const MarchLayout* march_layout(int E);
+  // The strip-walking forward step: whether a batch of E entries takes it
+  // (per_model: entries of each model), and its work (strips, chunks, points by
+  // unit).
+  bool strips_pay(int E, int per_model) const;
+  const MarchLayout* march_layout(int E, int per_model);
   ResGrid res_grid(const ResTiles& t) const;
   int plan_parts(int kind, int E, ResTiles& t);  // the launches a run takes, one after the other (0: not resident), and their tiles
   void res_begin(int kind, int E, int parts, ResComm& x);  // call with the device's lock held; E: most entries of a launch
@@ -257,7 +259,10 @@ class Propagator {
   // the measured width rule (index into kTileWidths) by batch size, or the override
   int fixed_width(int kind, int E) const;
   static constexpr int kGraphMaxEntries = 8;
-  static constexpr long long kMarchFrom = 30000;  // strip rows (strips x rows of x over the batch)
+  // strip rows (strips x rows of x over the batch) from which strips are walked, and
+  // to which where fewer than kMarchShared entries share a model (measured: one, and five or more)
+  static constexpr long long kMarchFrom = 30000, kMarchOwnTo = 70000;
+  static constexpr int kMarchShared = 4;
   // A forward batch of 2..kLanes entries without a band (line-search trial
   // runs) runs as one-entry loops side by side, lane e on its own stream:
   // measured on the 301x921 grid, two one-entry loops on two streams take

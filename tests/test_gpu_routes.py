@@ -121,6 +121,42 @@ def test_strip_walks(oracle, nx, nz, nb, ns, rows):
     s.close()
 
 
+@pytest.mark.parametrize("precision", [capi.PREC_EXACT, capi.PREC_FP32])
+@pytest.mark.parametrize("nx,nz,nb,ns,rows", [(360, 24, 20, 160, 0), (360, 96, 20, 160, 22), (360, 108, 20, 80, 0),
+                                              (360, 172, 20, 80, 0), (360, 213, 20, 54, 0), (360, 380, 20, 80, 0),
+                                              (360, 511, 20, 16, 0), (360, 511, 20, 31, 22)])
+def test_strips_only_where_they_are_filled(nx, nz, nb, ns, rows, precision):
+    """Strips hold up to 116 z and tiles 64: the walk takes 2 tiles a strip from
+    30000 strip rows, 1.8 from 60000, and never less (one strip of 44, two of 64,
+    of 96 and of 100, three of 78, four of 100: tiled)."""
+    case, s, wlt, start = survey(nx, nz, nb, ns, nt=12, precision=precision)
+    s.set_resident(0)
+    strips = -(-(nz + nb) // 116) * (nx + 2 * nb) * ns
+    assert strips >= 30000
+    print(f"{ns} shots of {nx}x{nz}: {strips} strip rows", flush=True)
+    a = s.forward_shots(wlt)
+    route = s.last_run(0)
+    assert route[:3] == ("strips", 12, rows) if rows else route[:2] == ("per step", 12)
+    s.set_tile_x(16)
+    assert np.count_nonzero(a) > 0 and np.array_equal(bits(a), bits(s.forward_shots(wlt)))
+    s.close()
+
+
+@pytest.mark.parametrize("members,route", [(60, "strips"), (102, "strips"), (104, "per step")])
+def test_strips_of_entries_with_their_own_models(members, route):
+    """Members of 201x301: 682 strip rows each, tiled past 70000."""
+    from swfwi_amd.enkf import Enkf
+    case, s, wlt, start = survey(301, 201, 20, 4, nt=80)
+    s.set_resident(0)
+    e = Enkf(s, wlt, s.forward_shots(wlt), 0.2, members)
+    e.set_members(np.stack([start * np.float32(1 + 0.002 * k) for k in range(members)]))
+    print(f"{members} members", flush=True)
+    e.analyze(None, 3)
+    assert s.last_run(0)[0] == route
+    e.close()
+    s.close()
+
+
 @pytest.mark.parametrize("ns,rows", [(60, 14), (92, 22)])
 def test_strip_walks_in_fp32(ns, rows):
     case, s, wlt, start = survey(301, 201, 20, ns, precision=capi.PREC_FP32)
