@@ -8,6 +8,17 @@
 
 namespace swfwi {
 
+namespace {
+// Memory the runtime knows (pinned, managed or a device's): it copies that
+// directly, and the host may not be able to touch it at all.
+bool known_to_runtime(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();  // ordinary memory
+  return false;
+}
+}  // namespace
+
 HostLane::~HostLane() {
   for (hipEvent_t e : done_)
     if (e) (void)hipEventDestroy(e);
@@ -17,14 +28,15 @@ HostLane::~HostLane() {
 void HostLane::run(const std::vector<HostSpan>& spans, hipStream_t s, bool down) {
   size_t total = 0;
   for (const HostSpan& p : spans) total += p.bytes;
-  if (total < kHostCopyFrom) {
+  const bool direct = total > 0 && known_to_runtime(spans.front().host);
+  if (total < kHostCopyFrom || direct) {
     for (const HostSpan& p : spans) {
       if (down)
         SWFWI_HIP(hipMemcpyAsync(p.host, p.dev, p.bytes, hipMemcpyDeviceToHost, s));
       else
         SWFWI_HIP(hipMemcpyAsync(p.dev, p.host, p.bytes, hipMemcpyHostToDevice, s));
     }
-    if (down) SWFWI_HIP(hipStreamSynchronize(s));
+    if (down || direct) SWFWI_HIP(hipStreamSynchronize(s));
     return;
   }
   if (!pin_) SWFWI_HIP(hipHostMalloc((void**)&pin_, 2 * kWorkers * kPiece, hipHostMallocDefault));
@@ -102,7 +114,7 @@ void HostLane::run(const std::vector<HostSpan>& spans, hipStream_t s, bool down)
 }
 
 PageIn::PageIn(void* p, size_t bytes) {
-  if (!p || bytes < kHostCopyFrom) return;
+  if (!p || bytes < kHostCopyFrom || known_to_runtime(p)) return;
   constexpr size_t kPage = 4096;
   const int n = std::min<int>(4, std::max(1u, std::thread::hardware_concurrency()));
   threads_.reserve(n);
