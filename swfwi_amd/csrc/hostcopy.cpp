@@ -4,7 +4,6 @@
 #include <cstring>
 #include <exception>
 #include <mutex>
-#include <system_error>
 
 namespace swfwi {
 
@@ -25,21 +24,29 @@ HostLane::~HostLane() {
   if (pin_) (void)hipHostFree(pin_);
 }
 
+// whether the pinned slots are there; without them the runtime copies
+bool HostLane::slots() {
+  if (!pin_ && hipHostMalloc((void**)&pin_, 2 * kWorkers * kPiece, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    pin_ = nullptr;
+  }
+  return pin_ != nullptr;
+}
+
 void HostLane::run(const std::vector<HostSpan>& spans, hipStream_t s, bool down) {
   size_t total = 0;
   for (const HostSpan& p : spans) total += p.bytes;
-  const bool direct = total > 0 && known_to_runtime(spans.front().host);
-  if (total < kHostCopyFrom || direct) {
+  const bool known = total > 0 && known_to_runtime(spans.front().host);
+  if (total < kHostCopyFrom || known || !slots()) {
     for (const HostSpan& p : spans) {
       if (down)
         SWFWI_HIP(hipMemcpyAsync(p.host, p.dev, p.bytes, hipMemcpyDeviceToHost, s));
       else
         SWFWI_HIP(hipMemcpyAsync(p.dev, p.host, p.bytes, hipMemcpyHostToDevice, s));
     }
-    if (down || direct) SWFWI_HIP(hipStreamSynchronize(s));
+    if (down || known) SWFWI_HIP(hipStreamSynchronize(s));
     return;
   }
-  if (!pin_) SWFWI_HIP(hipHostMalloc((void**)&pin_, 2 * kWorkers * kPiece, hipHostMallocDefault));
   for (hipEvent_t& e : done_)
     if (!e) SWFWI_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   int device = 0;
@@ -101,7 +108,7 @@ void HostLane::run(const std::vector<HostSpan>& spans, hipStream_t s, bool down)
   for (int k = 1; k <= extra; k++) {
     try {
       threads.emplace_back(worker, k);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {
       break;  // no more threads to be had: those there are do it
     }
   }
@@ -117,18 +124,18 @@ PageIn::PageIn(void* p, size_t bytes) {
   if (!p || bytes < kHostCopyFrom || known_to_runtime(p)) return;
   constexpr size_t kPage = 4096;
   const int n = std::min<int>(4, std::max(1u, std::thread::hardware_concurrency()));
-  threads_.reserve(n);
   char* base = (char*)p;
-  for (int k = 0; k < n; k++) {
-    char *a = base + bytes / n * k, *b = k + 1 < n ? base + bytes / n * (k + 1) : base + bytes;
-    try {
+  try {
+    threads_.reserve(n);
+    for (int k = 0; k < n; k++) {
+      char *a = base + bytes / n * k, *b = k + 1 < n ? base + bytes / n * (k + 1) : base + bytes;
       threads_.emplace_back([this, a, b] {
         for (char* q = a; q < b && !stop_.load(std::memory_order_relaxed); q += kPage)
           __atomic_fetch_or(q, (char)0, __ATOMIC_RELAXED);
       });
-    } catch (const std::system_error&) {
-      return;  // the copy touches the rest
     }
+  } catch (const std::exception&) {
+    // no more threads to be had: the copy touches the rest
   }
 }
 

@@ -27,7 +27,7 @@ struct HostSpan {
 // runtime knows goes to it as well: it transfers pinned memory without a copy
 // (77 MB 1.43 ms up and 1.44 down, in pieces 2.13 and 2.13).
 // 16 MB of pinned memory, allocated on the first large copy (0.5 ms) and
-// given back with the handle.
+// given back with the handle; where they cannot be had the runtime copies.
 constexpr size_t kHostCopyFrom = 16u << 20;
 class HostLane {
  public:
@@ -44,6 +44,7 @@ class HostLane {
  private:
   static constexpr int kWorkers = 4;
   static constexpr size_t kPiece = 2u << 20;
+  bool slots();
   void run(const std::vector<HostSpan>& spans, hipStream_t s, bool down);
   char* pin_ = nullptr;
   hipEvent_t done_[2 * kWorkers] = {};

@@ -23,8 +23,10 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["pageable", "known"])
+@pytest.mark.parametrize("what", ["pageable", "known", "no_pin", "no_memory"])
 def test_copies(driver, what):
     """Ordinary memory goes through pinned pieces; memory that the runtime knows
-    goes to it whole, and the host does not touch it."""
+    goes to it whole, and the host does not touch it.  Without pinned memory the
+    runtime copies; an allocation that fails on the way (each in turn, the
+    threads' own among them) ends in an exception at most."""
     subprocess.run([driver, what], check=True, timeout=60)
