@@ -230,8 +230,8 @@ long long Propagator::tile_key(int kind, int E) const {
 int Propagator::tile_choice_cached(int kind, int E) const {
   if (tile_override_) return tile_override_;
   const long long key = tile_key(kind, E);
-  for (const auto& kv : tile_cache_)
-    if (kv.first == key) return kTileWidths[kv.second];
+  for (const TileChoice& c : tile_cache_)
+    if (c.key == key) return kTileWidths[c.width];
   return 0;
 }
 
@@ -325,11 +325,14 @@ int Propagator::tile_choice(int kind, int E, const float* rv, long long rvstride
                             bool may_time) {
   if (tile_override_) return fixed_width(kind, E);
   const long long key = tile_key(kind, E);
-  for (const auto& kv : tile_cache_)
-    if (kv.first == key) return kv.second;
+  const bool timed = tune_ && may_time;
+  TileChoice* known = nullptr;
+  for (TileChoice& c : tile_cache_)
+    if (c.key == key) known = &c;
+  if (known && (known->timed || !timed)) return known->width;
   const int rule = fixed_width(kind, E);  // the measured rule is the incumbent
   int best = rule;
-  if (tune_ && may_time) {
+  if (timed) {
     // timed trial on scratch wavefields (the caller's workspace is free at
     // this point: forward() tunes before it zeroes and runs); three
     // interleaved rounds, the first warming clocks and caches; a width
@@ -348,7 +351,10 @@ int Propagator::tile_choice(int kind, int E, const float* rv, long long rvstride
       if (faster && std::max(t[0][i], t[1][i]) < std::max(t[0][best], t[1][best])) best = i;
     }
   }
-  tile_cache_.push_back({key, best});
+  if (known)
+    *known = TileChoice{key, best, timed};
+  else
+    tile_cache_.push_back(TileChoice{key, best, timed});
   return best;
 }
 

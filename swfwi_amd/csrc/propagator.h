@@ -253,8 +253,8 @@ class Propagator {
                          long long vstride, const float* band, float* grad, long long gstride, Fields& w, int rvdiv,
                          int it_min, const std::vector<float>& wts);
   // Tile width (index into kTileWidths) for a kernel kind (0 forward,
-  // 1 backward) and batch size: fixed override, cached choice, or a timed
-  // trial of every width on scratch wavefields (the tile tuner).
+  // 1 backward) and batch size: fixed override, cached choice, or, when the run
+  // may time, a timed trial of every width on scratch wavefields (the tile tuner).
   int tile_choice(int kind, int E, const float* rv, long long rvstride, int rvdiv, Fields& w, bool may_time);
   // the measured width rule (index into kTileWidths) by batch size, or the override
   int fixed_width(int kind, int E) const;
@@ -305,7 +305,12 @@ class Propagator {
   bool tune_ = true;
   DBuf<float> tune_grad_;  // scratch gradient of the tuner's backward trials
   int bwd_split_ = -1;
-  std::vector<std::pair<long long, int>> tile_cache_;  // (kind*2^32 + E) -> width index
+  struct TileChoice {
+    long long key;  // tile_key
+    int width;      // index into kTileWidths
+    bool timed;     // else the rule's, until a run of the size may time
+  };
+  std::vector<TileChoice> tile_cache_;
   DBuf<int> sxp_, szp_, gxp_, gzp_;
 
   int resident_ = -1;

@@ -1,0 +1,123 @@
+// The propagator's host side against a runtime and launchers of this file's
+// own: nothing runs, what is launched is counted, a resident run can be told to
+// find the chip shared, and allocations can be made to fail.
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <string>
+
+#include "propagator.h"
+
+using namespace swfwi;
+
+static int g_fwd = 0, g_bwd = 0, g_march = 0, g_resident[2] = {0, 0};
+static bool g_shared[2] = {false, false}, g_no_memory = false, g_no_pinned = false;
+static long long g_limit = 0;
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+  if (g_no_memory) return hipErrorOutOfMemory;
+  return (*p = std::calloc(n, 1)) ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (g_no_pinned) return hipErrorOutOfMemory;
+  return (*p = std::calloc(n, 1)) ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { *d = h; return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "test"; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 100000; return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)std::malloc(1); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { std::free((void*)s); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)std::malloc(1); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t e) { std::free((void*)e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 1; return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = nullptr; return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) { *e = nullptr; return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+}
+
+namespace swfwi {
+int tile_count_x(int nx, int tile_x) { return (nx - 2 * kHalo + tile_x - 1) / tile_x; }
+void launch_fill(float*, long long, float, hipStream_t) {}
+void launch_fill_u32(unsigned*, long long, unsigned, hipStream_t) {}
+void launch_point_inject(float*, long long, const Inject&, int, int, hipStream_t) {}
+void launch_fwd_step(const FwdStepArgs&, int, bool, int, hipStream_t, int) { g_fwd++; }
+void launch_bwd_step(const BwdStepArgs&, int, int, hipStream_t, int) { g_bwd++; }
+void launch_fwd_march(const FwdStepArgs&, const MarchMap&, int, int, hipStream_t) { g_march++; }
+int resident_cus() { return 256; }
+int resident_per_cu(bool backward, int, int) { return backward ? 1 : 2; }
+static void resident(int kind, const ResComm& x) {
+  g_resident[kind]++;
+  g_limit = x.limit;
+  if (g_shared[kind]) *x.abort_host = 1;
+}
+void launch_resident_fwd(const ResFwdArgs& a, int, hipStream_t) { resident(0, a.x); }
+void launch_resident_bwd(const ResBwdArgs& a, int, hipStream_t) { resident(1, a.x); }
+}  // namespace swfwi
+
+struct Run {
+  Propagator p;
+  Fields w;
+  std::vector<float> v;  // stands in for every array of the caller's
+  int nt;
+  static Geometry geometry(int nt) {
+    Geometry g;
+    g.nx = 301, g.nz = 201, g.nb = 20, g.dt = 0.002f, g.dx = 20, g.fm = 12, g.nt = nt;
+    g.sx = {3}, g.sz = {1}, g.gx = {9}, g.gz = {1};
+    return g;
+  }
+  explicit Run(int nt_) : p(geometry(nt_), kExact), v(64), nt(nt_) {}
+  Propagator::Sources src() { return Propagator::Sources{v.data(), 1, 0, nullptr, nullptr}; }
+  // launches of the per-step kernels (trials included), resident launches; the run's route
+  int forward(int E, bool band) {
+    g_fwd = g_bwd = g_march = g_resident[0] = g_resident[1] = 0;
+    p.forward(E, v.data(), 0, src(), nullptr, band ? v.data() : nullptr, w);
+    return p.last_run[0].route;
+  }
+  int backward(int E) {
+    g_fwd = g_bwd = g_resident[0] = g_resident[1] = 0;
+    p.backward(E, v.data(), 0, src(), v.data(), 0, v.data(), v.data(), p.geo().npts(), w);
+    return p.last_run[1].route;
+  }
+};
+
+#define EXPECT(c) do { if (!(c)) { std::printf("line %d: %s (fwd %d bwd %d)\n", __LINE__, #c, g_fwd, g_bwd); return 1; } } while (0)
+constexpr int kTrial = 3 * kNumWidths * 8;  // launches of one kernel's width trials
+
+static int tuner() {
+  const int nt = 170;
+  Run fresh(nt), used(nt);
+  fresh.p.set_resident(0, 5e5);
+  EXPECT(fresh.forward(8, true) == Propagator::kPerStep);
+  EXPECT(g_fwd == nt + kTrial && g_bwd == kTrial);
+  EXPECT(used.forward(8, true) == Propagator::kResident);
+  EXPECT(g_fwd == 0 && g_bwd == 0 && g_resident[0] == 1);
+  EXPECT(used.p.tile_choice_cached(0, 8) > 0 && used.p.tile_choice_cached(1, 8) > 0);
+  used.p.set_resident(0, 5e5);
+  EXPECT(used.forward(8, true) == Propagator::kPerStep);
+  EXPECT(g_fwd == nt + kTrial && g_bwd == kTrial);  // as a new handle's
+  EXPECT(used.forward(8, true) == Propagator::kPerStep);
+  EXPECT(g_fwd == nt && g_bwd == 0);
+  used.p.set_tuning(false);
+  EXPECT(used.forward(8, true) == Propagator::kPerStep && g_fwd == nt && g_bwd == 0);
+  return 0;
+}
+
+int main(int, char** argv) {
+  const std::string what = argv[1];
+  if (what == "tuner") return tuner();
+  return 2;
+}

@@ -1,0 +1,35 @@
+"""What the propagator decides on the host, on the CPU: its own sources over
+launchers that count (propagator_driver.cpp)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(HERE, "..", "swfwi_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    cxx = shutil.which("g++")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    if not cxx or not os.path.exists(os.path.join(rocm, "include", "hip", "hip_runtime.h")):
+        pytest.skip("no host compiler or HIP headers")
+    exe = str(tmp_path_factory.mktemp("prop") / "propagator_driver")
+    subprocess.run([cxx, "-O1", "-g", "-std=c++17", "-w", "-D__HIP_PLATFORM_AMD__", "-I", CSRC, "-I",
+                    os.path.join(rocm, "include"), os.path.join(HERE, "propagator_driver.cpp"),
+                    os.path.join(CSRC, "propagator.cpp"), os.path.join(CSRC, "resident.cpp"), "-o", exe, "-pthread"],
+                   check=True)
+    return exe
+
+
+def run(driver, what):
+    r = subprocess.run([driver, what], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_widths_are_timed_after_a_resident_run(driver):
+    """A run that takes the resident loop keeps the rule's widths as they are,
+    and the first per-step run of the size still times them."""
+    run(driver, "tuner")
