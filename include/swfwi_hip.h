@@ -136,9 +136,10 @@ int swfwi_solver_set_graphs(swfwi_solver h, int on);
  * by batch size (the default). */
 int swfwi_solver_set_tile_x(swfwi_solver h, int tile_x);
 /* The tile tuner (1, the default) or the measured rule alone (0): with
- * tile_x 0, the first forward run of each batch size times every width on
- * scratch wavefields and keeps the rule's width unless another is faster by
- * 3% in both timed rounds.  Every width gives the same results bit for bit. */
+ * tile_x 0, the first run of each batch size that launches a step kernel times
+ * every width on scratch wavefields (the forward run before a gradient times
+ * the backward kernel's) and keeps the rule's width unless another is faster
+ * by 3% in both timed rounds.  Every width gives the same results bit for bit. */
 int swfwi_solver_set_tuning(swfwi_solver h, int on);
 /* Tile width in use for a kernel kind (0 forward, 1 backward) and batch
  * size, 0 when that batch size has not run yet. */

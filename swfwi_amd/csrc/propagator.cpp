@@ -520,9 +520,11 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
                          Fields& w, int rvdiv) {
   const long long np = g_.npts();
   w.ensure(E, np, true);
-  ResTiles rt;
-  if (band && plan_parts(0, E, rt) && !plan_parts(1, E, rt))
-    tile_choice(1, E, rv, rvstride, rvdiv, w, true);  // for the backward, while the workspace is free
+  // the backward's tile width is timed now, while the workspace is free
+  // (backward() runs on the state this forward leaves behind), if a backward
+  // run can follow and will not be resident
+  const bool time_bwd = band && !runs_resident(1, E);
+  if (time_bwd && runs_resident(0, E)) tile_choice(1, E, rv, rvstride, rvdiv, w, true);
   if (resident_forward(E, rv, rvstride, src, dcal, band, w, rvdiv)) {
     // (the widths a run of this size would fall back to, untimed)
     tile_choice(0, E, rv, rvstride, rvdiv, w, false);
@@ -535,11 +537,9 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
   }
   int tw1 = 0;  // the lanes' tile width
   const bool lanes = E >= 2 && E <= kLanes && band == nullptr;
-  // tile widths for this batch, chosen now while the workspace is free
-  // (backward() runs on the state this forward leaves behind)
   const MarchLayout* march = lanes ? nullptr : march_layout(E, rvstride == 0 ? E : rvdiv);
   const int tw = tile_choice(0, E, rv, rvstride, rvdiv, w, !march);
-  tile_choice(1, E, rv, rvstride, rvdiv, w, true);
+  tile_choice(1, E, rv, rvstride, rvdiv, w, time_bwd);
   const uintptr_t key[] = {1,
                            (uintptr_t)tw,
                            (uintptr_t)(march ? march->m.rows : 0),

@@ -161,8 +161,9 @@ class Propagator {
   // Tile width override (8, 16, 32) or 0 for the tuner; tuning off falls back
   // to the measured rule by batch size.
   void set_tile_x(int tx);
-  // The tile tuner (on by default): the first forward() of a batch size
-  // times every width on scratch wavefields and keeps the measured rule's
+  // The tile tuner (on by default): the first forward() of a batch size that
+  // launches step kernels (for the backward kernel: that a per-step backward()
+  // can follow) times every width on scratch wavefields and keeps the measured rule's
   // width unless another is faster by kTuneMargin in both timed rounds.
   void set_tuning(bool on) {
     tune_ = on;
@@ -244,6 +245,7 @@ class Propagator {
   const MarchLayout* march_layout(int E, int per_model);
   ResGrid res_grid(const ResTiles& t) const;
   int plan_parts(int kind, int E, ResTiles& t);  // the launches a run takes, one after the other (0: not resident), and their tiles
+  bool runs_resident(int kind, int E);  // whether a run starts as resident launches
   void res_begin(int kind, int E, int parts, ResComm& x);  // call with the device's lock held; E: most entries of a launch
   void res_part(int kind, int E, ResComm& x);  // before each launch
   bool res_end(int kind, long long steps, hipEvent_t t0);

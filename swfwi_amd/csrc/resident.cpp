@@ -91,6 +91,11 @@ int Propagator::plan_parts(int kind, int E, ResTiles& t) {
   return one ? 1 : 0;
 }
 
+bool Propagator::runs_resident(int kind, int E) {
+  ResTiles t;
+  return plan_parts(kind, E, t) > 0 && res_layout(t).fits;
+}
+
 bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   if (resident_ == 0 || tile_override_ || (kind == 1 && bwd_split_ >= 0) || g_.nt < 2) return false;
   const int most = kind == 1 ? kResMaxWidthBwd : kResMaxWidthFwd;

@@ -73,13 +73,13 @@ struct Run {
   Fields w;
   std::vector<float> v;  // stands in for every array of the caller's
   int nt;
-  static Geometry geometry(int nt) {
+  static Geometry geometry(int nt, bool crowded) {
     Geometry g;
     g.nx = 301, g.nz = 201, g.nb = 20, g.dt = 0.002f, g.dx = 20, g.fm = 12, g.nt = nt;
-    g.sx = {3}, g.sz = {1}, g.gx = {9}, g.gz = {1};
+    g.sx = {3}, g.sz = {1}, g.gx.assign(crowded ? 700 : 1, 9), g.gz.assign(crowded ? 700 : 1, 1);
     return g;
   }
-  explicit Run(int nt_) : p(geometry(nt_), kExact), v(64), nt(nt_) {}
+  explicit Run(int nt_, bool crowded = false) : p(geometry(nt_, crowded), kExact), v(64), nt(nt_) {}
   Propagator::Sources src() { return Propagator::Sources{v.data(), 1, 0, nullptr, nullptr}; }
   // launches of the per-step kernels (trials included), resident launches; the run's route
   int forward(int E, bool band) {
@@ -116,8 +116,26 @@ static int tuner() {
   return 0;
 }
 
+static int backward_trials() {
+  const int nt = 170;
+  Run r(nt);
+  r.p.set_resident(0, 5e5);
+  EXPECT(r.forward(30, false) == Propagator::kPerStep && g_fwd == nt + kTrial && g_bwd == 0);  // nothing follows
+  EXPECT(r.p.tile_choice_cached(1, 30) > 0);
+  EXPECT(r.forward(30, true) == Propagator::kPerStep && g_fwd == nt && g_bwd == kTrial);
+  EXPECT(r.backward(30) == Propagator::kPerStep && r.p.last_run[1].width == r.p.tile_choice_cached(1, 30));
+  Run s(nt);  // 40 entries: the forward a launch a step, the backward resident in parts
+  EXPECT(s.forward(40, true) == Propagator::kPerStep && g_fwd == nt + kTrial && g_bwd == 0);
+  EXPECT(s.backward(40) == Propagator::kResident && g_resident[1] >= 2 && g_bwd == 0);
+  Run c(nt, true);  // more receivers at a place than a resident tile takes
+  EXPECT(c.forward(8, true) == Propagator::kPerStep && g_bwd == kTrial && g_resident[0] == 0);
+  EXPECT(c.backward(8) == Propagator::kPerStep);
+  return 0;
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "tuner") return tuner();
+  if (what == "backward_trials") return backward_trials();
   return 2;
 }

@@ -33,3 +33,9 @@ def test_widths_are_timed_after_a_resident_run(driver):
     """A run that takes the resident loop keeps the rule's widths as they are,
     and the first per-step run of the size still times them."""
     run(driver, "tuner")
+
+
+def test_backward_widths_are_timed_for_a_backward_run(driver):
+    """No trials of the backward kernel where no backward run follows, or where
+    it takes the resident loop."""
+    run(driver, "backward_trials")
