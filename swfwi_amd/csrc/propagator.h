@@ -237,7 +237,7 @@ class Propagator {
     ResPoints src() const { return ResPoints{sptr.get(), sitems.get()}; }
     ResPoints rec() const { return ResPoints{rptr.get(), ritems.get()}; }
   };
-  ResLayout& res_layout(const ResTiles& t);
+  ResLayout* res_layout(const ResTiles& t);  // null: no memory for it
   // The strip-walking forward step: whether a batch of E entries takes it
   // (per_model: entries of each model), and its work (strips, chunks, points by
   // unit).

@@ -19,6 +19,20 @@ std::mutex& device_lock(int dev) {
   return mu[dev >= 0 && dev < kMaxDevices ? dev : 0];
 }
 
+// Whether the buffers that `get` asks for could be had: without them the
+// per-step kernels run.
+template <class F>
+bool had(F&& get) {
+  try {
+    get();
+    return true;
+  } catch (const Error& e) {
+    if (e.code != kErrHip) throw;
+    (void)hipGetLastError();
+    return false;
+  }
+}
+
 struct HostPoints {
   std::vector<int> ptr;
   std::vector<int2> items;
@@ -93,7 +107,9 @@ int Propagator::plan_parts(int kind, int E, ResTiles& t) {
 
 bool Propagator::runs_resident(int kind, int E) {
   ResTiles t;
-  return plan_parts(kind, E, t) > 0 && res_layout(t).fits;
+  if (plan_parts(kind, E, t) < 1) return false;
+  const ResLayout* l = res_layout(t);
+  return l && l->fits;
 }
 
 bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
@@ -138,22 +154,25 @@ bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   return kind == 1 || E == 1 || E > kLanes || t.w <= kResLanesWidth;
 }
 
-Propagator::ResLayout& Propagator::res_layout(const ResTiles& t) {
+Propagator::ResLayout* Propagator::res_layout(const ResTiles& t) {
   for (auto& l : res_layouts_)
-    if (l->t.w == t.w && l->t.h == t.h) return *l;
+    if (l->t.w == t.w && l->t.h == t.h) return l.get();
   hipStream_t s = stream();
   auto l = std::make_unique<ResLayout>();
   l->t = t;
   const HostPoints src = bucket(src_idx_, g_.ld, t), rec = bucket(rec_idx_, g_.ld, t);
   l->fits = src.most <= kResMaxPts && rec.most <= kResMaxPts;
-  l->sptr.upload(src.ptr, s);
-  l->sitems.upload(src.items, s);
-  l->rptr.upload(rec.ptr, s);
-  l->ritems.upload(rec.items, s);
+  const bool ok = had([&] {
+    l->sptr.upload(src.ptr, s);
+    l->sitems.upload(src.items, s);
+    l->rptr.upload(rec.ptr, s);
+    l->ritems.upload(rec.items, s);
+  });
   SWFWI_HIP(hipStreamSynchronize(s));  // the host vectors end here
+  if (!ok) return nullptr;
   if (res_layouts_.size() >= 16) res_layouts_.erase(res_layouts_.begin());
   res_layouts_.push_back(std::move(l));
-  return *res_layouts_.back();
+  return res_layouts_.back().get();
 }
 
 ResGrid Propagator::res_grid(const ResTiles& t) const {
@@ -176,12 +195,14 @@ ResGrid Propagator::res_grid(const ResTiles& t) const {
 void Propagator::res_begin(int kind, int E, int parts, ResComm& x) {
   hipStream_t s = stream();
   if (!abort_host_) {
-    SWFWI_HIP(hipHostMalloc(reinterpret_cast<void**>(&abort_host_), sizeof(int), hipHostMallocMapped));
+    abort_dev_.resize(1);
+    void* flag = nullptr;
+    SWFWI_HIP(hipHostMalloc(&flag, sizeof(int), hipHostMallocMapped));
+    abort_host_ = static_cast<int*>(flag);
     int dev = 0, khz = 0;
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0)
       ticks_per_us_ = khz * 1e-3;
-    abort_dev_.resize(1);
     *abort_host_ = 1;  // cleared below
   }
   DBuf<unsigned long long>& buf = xbuf_[kind];
@@ -245,14 +266,14 @@ bool Propagator::resident_forward(int E, const float* rv, long long rvstride, co
   ResTiles t;
   const int parts = plan_parts(0, E, t);
   if (parts < 1) return false;
-  ResLayout& l = res_layout(t);
-  if (!l.fits) return false;
+  const ResLayout* l = res_layout(t);
+  if (!l || !l->fits) return false;
   hipStream_t s = stream();
   const long long np = g_.npts();
   std::lock_guard<std::mutex> lock(device_lock(dev_));
   ResFwdArgs a;
   const int part = (E + parts - 1) / parts;
-  res_begin(0, part, parts, a.x);
+  if (!had([&] { res_begin(0, part, parts, a.x); })) return false;
   hipEvent_t t0 = nullptr;
   if (timing_) {
     t0 = pooled_event();
@@ -277,8 +298,8 @@ bool Propagator::resident_forward(int E, const float* rv, long long rvstride, co
   a.rv = rv;
   a.rvstride = rvstride;
   a.rvdiv = rvdiv;
-  a.src = l.src();
-  a.rec = l.rec();
+  a.src = l->src();
+  a.rec = l->rec();
   a.amp = src.amp;
   a.amp_ld = src.ld;
   a.amp_estride = src.estride;
@@ -305,19 +326,19 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
   ResTiles t;
   const int parts = plan_parts(1, E, t);
   if (parts < 1) return false;
-  ResLayout& l = res_layout(t);
-  if (!l.fits) return false;
+  const ResLayout* l = res_layout(t);
+  if (!l || !l->fits) return false;
   hipStream_t s = stream();
   const long long np = g_.npts();
   const int nt = g_.nt, ng = g_.ng();
   if (res_wts_.size() != wts.size()) {  // the taper weights follow from dt and nt alone
-    res_wts_.upload(wts, s);
+    if (!had([&] { res_wts_.upload(wts, s); })) return false;
     SWFWI_HIP(hipStreamSynchronize(s));
   }
   std::lock_guard<std::mutex> lock(device_lock(dev_));
   ResBwdArgs a;
   const int part = (E + parts - 1) / parts;
-  res_begin(1, part, parts, a.x);
+  if (!had([&] { res_begin(1, part, parts, a.x); })) return false;
   hipEvent_t t0 = nullptr;
   if (timing_) {
     t0 = pooled_event();
@@ -342,8 +363,8 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
   a.rv = rv;
   a.rvstride = rvstride;
   a.rvdiv = rvdiv;
-  a.src = l.src();
-  a.rec = l.rec();
+  a.src = l->src();
+  a.rec = l->rec();
   a.amp = src.amp;
   a.amp_ld = src.ld;
   a.amp_estride = src.estride;

@@ -11,12 +11,13 @@
 using namespace swfwi;
 
 static int g_fwd = 0, g_bwd = 0, g_march = 0, g_resident[2] = {0, 0};
-static bool g_shared[2] = {false, false}, g_no_memory = false, g_no_pinned = false;
+static bool g_shared[2] = {false, false}, g_no_pinned = false;
+static int g_memory = 1 << 30;  // allocations that succeed
 static long long g_limit = 0;
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
-  if (g_no_memory) return hipErrorOutOfMemory;
+  if (g_memory-- <= 0) return hipErrorOutOfMemory;
   return (*p = std::calloc(n, 1)) ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
@@ -62,6 +63,7 @@ int resident_per_cu(bool backward, int, int) { return backward ? 1 : 2; }
 static void resident(int kind, const ResComm& x) {
   g_resident[kind]++;
   g_limit = x.limit;
+  if (!x.buf || !x.abort_dev || !x.abort_host) std::abort();
   if (g_shared[kind]) *x.abort_host = 1;
 }
 void launch_resident_fwd(const ResFwdArgs& a, int, hipStream_t) { resident(0, a.x); }
@@ -133,9 +135,30 @@ static int backward_trials() {
   return 0;
 }
 
+static int no_memory() {
+  for (int left = -1; left < 16; left++) {  // the allocation that fails (-1: pinned memory)
+    Run r(170);
+    r.p.set_resident(0, 5e5);
+    r.forward(8, true);  // the fields and lists exist
+    r.backward(8);
+    r.p.set_resident(-1, 5e5);
+    if (left >= 0) g_memory = left;
+    g_no_pinned = left < 0;
+    const int f = r.forward(8, true), b = r.backward(8);
+    if (left <= 0) EXPECT(f == Propagator::kPerStep && b == Propagator::kPerStep);
+    if (left == 15) EXPECT(f == Propagator::kResident && b == Propagator::kResident && g_memory > 0);
+    EXPECT(r.p.gave_up == 0);
+    g_memory = 1 << 30;
+    g_no_pinned = false;
+    EXPECT(r.forward(8, true) == Propagator::kResident && r.backward(8) == Propagator::kResident);
+  }
+  return 0;
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "tuner") return tuner();
   if (what == "backward_trials") return backward_trials();
+  if (what == "no_memory") return no_memory();
   return 2;
 }

@@ -39,3 +39,9 @@ def test_backward_widths_are_timed_for_a_backward_run(driver):
     """No trials of the backward kernel where no backward run follows, or where
     it takes the resident loop."""
     run(driver, "backward_trials")
+
+
+def test_no_memory_for_the_resident_loop(driver):
+    """Where its buffers cannot be had the per-step kernels run, and the resident
+    loop again once there is memory."""
+    run(driver, "no_memory")
