@@ -154,8 +154,10 @@ int swfwi_solver_set_bwd_split(swfwi_solver h, int mode);
  * larger ones as a few, a part of the batch each), 0 never,
  * 1 wherever the tiles fit.  wait_us bounds how long a block of that launch
  * waits for its neighbours (5e5 by default) before the run is done again with
- * one launch per step (and, by rule, so are the handle's later runs).  A fixed
- * tile width or backward form also means one launch per step.  Same results. */
+ * one launch per step (and, by rule, so are the handle's next runs: up to the
+ * 64th forward run from there, twice as many each time a wait runs out again,
+ * 4096 at most).  A fixed tile width or backward form also means one launch per
+ * step.  Same results. */
 int swfwi_solver_set_resident(swfwi_solver h, int mode, double wait_us);
 /* How the last run of a kind (0 forward, 1 backward) went: route 0 none yet, 1
  * one tiled launch per step, 2 the entries side by side on streams of their

@@ -520,6 +520,7 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
                          Fields& w, int rvdiv) {
   const long long np = g_.npts();
   w.ensure(E, np, true);
+  if (res_rest_ > 0) res_rest_--;
   // the backward's tile width is timed now, while the workspace is free
   // (backward() runs on the state this forward leaves behind), if a backward
   // run can follow and will not be resident

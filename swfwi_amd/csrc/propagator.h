@@ -317,7 +317,14 @@ class Propagator {
 
   int resident_ = -1;
   double res_wait_us_ = kResWaitUs;
-  bool res_gave_up_ = false;  // a run's wait ran out: by rule, the handle then keeps to the per-step kernels
+  // After a run whose wait ran out the handle keeps to the per-step kernels, by
+  // rule, for kResPause forward runs, and for twice as many each time a run of
+  // the kind waits in vain again, kResPauseMost at most: a wait is 0.5 s, the
+  // 64 runs in place of resident ones 0.1 to 0.2 s, so that a chip that stays
+  // shared costs a few waits and one that was shared for a moment is not lost.
+  int res_rest_ = 0;  // forward runs until the next try
+  static constexpr int kResPause = 64, kResPauseMost = 4096;
+  int res_pause_[2] = {kResPause, kResPause};
   static constexpr double kResWaitUs = 5e5;
   double ticks_per_us_ = 100;  // of the kernels' wall clock
   std::vector<std::unique_ptr<ResLayout>> res_layouts_;

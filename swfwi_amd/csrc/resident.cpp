@@ -63,7 +63,8 @@ void Propagator::set_resident(int mode, double wait_us) {
   if (!(wait_us >= 0)) fail(kErrArg, "the resident wait limit must not be negative");
   resident_ = mode;
   res_wait_us_ = wait_us;
-  res_gave_up_ = false;
+  res_rest_ = 0;
+  res_pause_[0] = res_pause_[1] = kResPause;
 }
 
 bool Propagator::res_twice(int rows) {
@@ -143,7 +144,7 @@ bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   t.ntx = (ux + t.w - 1) / t.w;
   if (t.w > most) return false;
   if (resident_ == 1) return true;
-  if (res_gave_up_) return false;  // the chip is shared: a run of this handle has waited in vain
+  if (res_rest_ > 0) return false;  // the chip is shared: a run of this handle has waited in vain
   // Measured over E (forward / backward microseconds a step, per-step kernels
   // -> resident): 201x301 E=1 4.7 -> 1.74, E=4 4.7 -> 2.7 / 8.1 -> 3.4, E=8
   // 6.2 -> 3.2 / 10.4 -> 5.2, E=11 6.9 -> 3.4 / 11.4 -> 9.1, E=16 7.9 -> 5.2,
@@ -246,9 +247,12 @@ bool Propagator::res_end(int kind, long long steps, hipEvent_t t0) {
   SWFWI_HIP(hipGetLastError());
   SWFWI_HIP(hipStreamSynchronize(stream()));
   const bool ok = *static_cast<volatile int*>(abort_host_) == 0;
-  if (!ok) {
-    res_gave_up_ = true;
+  if (ok) {
+    res_pause_[kind] = kResPause;
+  } else {
     gave_up++;
+    res_rest_ = res_pause_[kind];
+    res_pause_[kind] = std::min(2 * res_pause_[kind], kResPauseMost);
   }
   if (timing_) {
     if (ok) {

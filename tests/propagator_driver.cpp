@@ -155,10 +155,48 @@ static int no_memory() {
   return 0;
 }
 
+// runs of a kind until the next one that tries the resident loop
+static int runs_until_a_try(Run& r, int kind) {
+  for (int k = 1; k < 20000; k++) {
+    r.forward(8, true);
+    const bool forward_tried = g_resident[0] > 0;
+    if (kind == 0 && forward_tried) return k;
+    r.backward(8);
+    if (kind == 1 && g_resident[1] > 0) return k;
+  }
+  return -1;
+}
+
+static int shared_chip() {
+  for (int kind = 0; kind < 2; kind++) {
+    Run r(170);
+    g_shared[kind] = true;
+    EXPECT(runs_until_a_try(r, kind) == 1 && r.p.last_run[kind].route == Propagator::kPerStep && r.p.gave_up == 1);
+    long long last = 64;
+    EXPECT(runs_until_a_try(r, kind) == last && r.p.gave_up == 2);
+    for (int k = 0; k < 8; k++) {  // rarer each time, up to a limit
+      const long long n = runs_until_a_try(r, kind);
+      EXPECT(n == (2 * last < 4096 ? 2 * last : 4096));
+      last = n;
+    }
+    EXPECT(last == 4096 && r.p.gave_up == 10);
+    g_shared[kind] = false;  // the chip is free again
+    EXPECT(runs_until_a_try(r, kind) == 4096 && r.p.last_run[kind].route == Propagator::kResident);
+    EXPECT(runs_until_a_try(r, kind) == 1 && r.p.last_run[kind].route == Propagator::kResident);
+    g_shared[kind] = true;
+    EXPECT(runs_until_a_try(r, kind) == 1 && r.p.gave_up == 11 && runs_until_a_try(r, kind) == 64);
+    r.p.set_resident(-1, 5e5);  // asked for: at once
+    EXPECT(runs_until_a_try(r, kind) == 1);
+    g_shared[kind] = false;
+  }
+  return 0;
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "tuner") return tuner();
   if (what == "backward_trials") return backward_trials();
   if (what == "no_memory") return no_memory();
+  if (what == "shared_chip") return shared_chip();
   return 2;
 }

@@ -45,3 +45,9 @@ def test_no_memory_for_the_resident_loop(driver):
     """Where its buffers cannot be had the per-step kernels run, and the resident
     loop again once there is memory."""
     run(driver, "no_memory")
+
+
+def test_a_shared_chip_is_tried_again(driver):
+    """After a wait that ran out a handle goes back to the resident loop: 64
+    forward runs later, and after twice as many each time it is in vain again."""
+    run(driver, "shared_chip")
