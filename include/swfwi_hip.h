@@ -153,7 +153,7 @@ int swfwi_solver_set_bwd_split(swfwi_solver h, int mode);
  * keep their tiles on the chip run a whole time loop as one launch, somewhat
  * larger ones as a few, a part of the batch each), 0 never,
  * 1 wherever the tiles fit.  wait_us bounds how long a block of that launch
- * waits for its neighbours (5e5 by default) before the run is done again with
+ * waits for its neighbours (5e5 by default, 1e7 at most) before the run is done again with
  * one launch per step (and, by rule, so are the handle's next runs: up to the
  * 64th forward run from there, twice as many each time a wait runs out again,
  * 4096 at most).  A fixed tile width or backward form also means one launch per

@@ -325,7 +325,7 @@ class Propagator {
   int res_rest_ = 0;  // forward runs until the next try
   static constexpr int kResPause = 64, kResPauseMost = 4096;
   int res_pause_[2] = {kResPause, kResPause};
-  static constexpr double kResWaitUs = 5e5;
+  static constexpr double kResWaitUs = 5e5, kResWaitMostUs = 1e7;
   double ticks_per_us_ = 100;  // of the kernels' wall clock
   std::vector<std::unique_ptr<ResLayout>> res_layouts_;
   std::vector<std::unique_ptr<MarchLayout>> march_layouts_;  // by chunk length

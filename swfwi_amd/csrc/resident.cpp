@@ -1,6 +1,7 @@
 // Host side of the resident time loop: which runs take it, the tiles and point
 // lists of a run, its exchange buffer, and the launch under the device's lock.
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 
@@ -60,9 +61,9 @@ HostPoints bucket(const std::vector<long long>& idx, int ld, const ResTiles& t) 
 
 void Propagator::set_resident(int mode, double wait_us) {
   if (mode < -1 || mode > 1) fail(kErrArg, "resident mode must be -1 (by rule), 0 or 1");
-  if (!(wait_us >= 0)) fail(kErrArg, "the resident wait limit must not be negative");
+  if (!(wait_us >= 0) || std::isinf(wait_us)) fail(kErrArg, "the resident wait limit must be finite and not negative");
   resident_ = mode;
-  res_wait_us_ = wait_us;
+  res_wait_us_ = std::min(wait_us, kResWaitMostUs);
   res_rest_ = 0;
   res_pause_[0] = res_pause_[1] = kResPause;
 }

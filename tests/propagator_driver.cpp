@@ -192,11 +192,31 @@ static int shared_chip() {
   return 0;
 }
 
+static int wait_limit() {
+  Run r(170);
+  for (double bad : {-1.0, (double)NAN, (double)INFINITY}) {
+    bool refused = false;
+    try {
+      r.p.set_resident(1, bad);
+    } catch (const Error& e) {
+      refused = e.code == kErrArg;
+    }
+    EXPECT(refused);
+  }
+  for (double us : {0.0, 5e5, 1e7, 1e8, 1e300}) {
+    r.p.set_resident(1, us);
+    EXPECT(r.forward(8, true) == Propagator::kResident);
+    EXPECT(g_limit == (long long)((us < 1e7 ? us : 1e7) * 100));  // ticks of the clock above
+  }
+  return 0;
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "tuner") return tuner();
   if (what == "backward_trials") return backward_trials();
   if (what == "no_memory") return no_memory();
   if (what == "shared_chip") return shared_chip();
+  if (what == "wait_limit") return wait_limit();
   return 2;
 }

@@ -51,3 +51,8 @@ def test_a_shared_chip_is_tried_again(driver):
     """After a wait that ran out a handle goes back to the resident loop: 64
     forward runs later, and after twice as many each time it is in vain again."""
     run(driver, "shared_chip")
+
+
+def test_the_wait_limit(driver):
+    """Finite, not negative, ten seconds at most."""
+    run(driver, "wait_limit")
