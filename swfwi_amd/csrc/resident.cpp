@@ -145,6 +145,7 @@ bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   t.ntx = (ux + t.w - 1) / t.w;
   if (t.w > most) return false;
   if (resident_ == 1) return true;
+  if (g_.nt < kResSteps) return false;
   if (res_rest_ > 0) return false;  // the chip is shared: a run of this handle has waited in vain
   // Measured over E (forward / backward microseconds a step, per-step kernels
   // -> resident): 201x301 E=1 4.7 -> 1.74, E=4 4.7 -> 2.7 / 8.1 -> 3.4, E=8

@@ -42,6 +42,11 @@ constexpr int kResMaxWidthBwd = 80;          // (spills from 57 columns on; 69 c
 constexpr int kResLanesWidth = 80;           // widest for 2 to 4 forward entries
 constexpr int kResTwiceRows = 6;             // most rows a wave of which two forward blocks fit a CU
 
+// Fewest steps of a resident run: its launch, wait and clears cost about 10 us
+// (whole calls of one shot on 201x301 / 501x1501, launches -> resident: 2 steps
+// 82 -> 91 / 85 -> 104 us, 3 steps 82 -> 91 / 90 -> 105, 5 steps 107 -> 93 / 118 ->
+// 115, 10 steps 127 -> 103 / 147 -> 133).
+constexpr int kResSteps = 5;
 constexpr int kResMaxPartsFwd = 3, kResMaxPartsBwd = 8;  // most launches of one run
 constexpr int kResWideFwd = 15, kResWideBwd = 10;  // rows a wave from which parts are faster than one launch
 constexpr int kResPartRows = 7;               // most rows a wave of a part

@@ -211,6 +211,16 @@ static int wait_limit() {
   return 0;
 }
 
+static int few_steps() {
+  for (int nt = 1; nt < 8; nt++) {
+    Run r(nt);
+    EXPECT(r.forward(1, false) == (nt < 5 ? Propagator::kPerStep : Propagator::kResident));
+    r.p.set_resident(1, 5e5);
+    EXPECT(r.forward(1, false) == (nt < 2 ? Propagator::kPerStep : Propagator::kResident));
+  }
+  return 0;
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "tuner") return tuner();
@@ -218,5 +228,6 @@ int main(int, char** argv) {
   if (what == "no_memory") return no_memory();
   if (what == "shared_chip") return shared_chip();
   if (what == "wait_limit") return wait_limit();
+  if (what == "few_steps") return few_steps();
   return 2;
 }

@@ -56,3 +56,8 @@ def test_a_shared_chip_is_tried_again(driver):
 def test_the_wait_limit(driver):
     """Finite, not negative, ten seconds at most."""
     run(driver, "wait_limit")
+
+
+def test_a_few_steps_run_per_step(driver):
+    """A run of fewer than 5 steps is not worth a resident launch."""
+    run(driver, "few_steps")
