@@ -163,6 +163,8 @@ Propagator::Propagator(const Geometry& g, int precision) : g_(g), prec_(precisio
   }
   src_idx_ = si;
   rec_idx_ = gi;
+  std::vector<float> weights;
+  bwd_iters_ = std::max(1, g_.nt - xcorr_range(g_.dt, g_.nt, weights));
   sxp_.upload(sxp, s);
   szp_.upload(szp, s);
   gxp_.upload(gxp, s);
@@ -524,8 +526,8 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
   // the backward's tile width is timed now, while the workspace is free
   // (backward() runs on the state this forward leaves behind), if a backward
   // run can follow and will not be resident
-  const bool time_bwd = band && !runs_resident(1, E);
-  if (time_bwd && runs_resident(0, E)) tile_choice(1, E, rv, rvstride, rvdiv, w, true);
+  const bool time_bwd = band && !runs_resident(1, E, true);
+  if (time_bwd && runs_resident(0, E, true)) tile_choice(1, E, rv, rvstride, rvdiv, w, true);
   if (resident_forward(E, rv, rvstride, src, dcal, band, w, rvdiv)) {
     // (the widths a run of this size would fall back to, untimed)
     tile_choice(0, E, rv, rvstride, rvdiv, w, false);
@@ -537,7 +539,7 @@ void Propagator::forward(int E, const float* rv, long long rvstride, const Sourc
     return;
   }
   int tw1 = 0;  // the lanes' tile width
-  const bool lanes = E >= 2 && E <= kLanes && band == nullptr;
+  const bool lanes = side_by_side(E, band != nullptr);
   const MarchLayout* march = lanes ? nullptr : march_layout(E, rvstride == 0 ? E : rvdiv);
   const int tw = tile_choice(0, E, rv, rvstride, rvdiv, w, !march);
   tile_choice(1, E, rv, rvstride, rvdiv, w, time_bwd);

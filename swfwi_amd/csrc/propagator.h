@@ -244,8 +244,13 @@ class Propagator {
   bool strips_pay(int E, int per_model) const;
   const MarchLayout* march_layout(int E, int per_model);
   ResGrid res_grid(const ResTiles& t) const;
-  int plan_parts(int kind, int E, ResTiles& t);  // the launches a run takes, one after the other (0: not resident), and their tiles
-  bool runs_resident(int kind, int E);  // whether a run starts as resident launches
+  // the launches a run takes, one after the other (0: not resident), and their
+  // tiles; band: of a run that saves the boundary band
+  int plan_parts(int kind, int E, bool band, ResTiles& t);
+  bool two_a_cu(int kind, int E, const ResTiles& t) const { return (long long)t.n() * E > res_cap_[kind][prec_]; }
+  double part_us(int kind, int E, const ResTiles& t) const;  // estimates that plan_parts compares
+  double step_us(int kind, int E) const;
+  bool runs_resident(int kind, int E, bool band);  // whether a run starts as resident launches
   void res_begin(int kind, int E, int parts, ResComm& x);  // call with the device's lock held; E: most entries of a launch
   void res_part(int kind, int E, ResComm& x);  // before each launch
   bool res_end(int kind, long long steps, hipEvent_t t0);
@@ -270,6 +275,7 @@ class Propagator {
   // measured on the 301x921 grid, two one-entry loops on two streams take
   // 25 ms where one two-entry loop takes 30 ms.
   static constexpr int kLanes = 4;
+  static bool side_by_side(int E, bool band) { return E >= 2 && E <= kLanes && !band; }
   static constexpr long long kBwdSplitBelow = 6000;  // 64x16 tiles over the batch
   // Run a time loop (`launches` step launches of kind 0 forward / 1
   // backward): captured into a HIP graph on first use and replayed when the
@@ -330,6 +336,7 @@ class Propagator {
   std::vector<std::unique_ptr<ResLayout>> res_layouts_;
   std::vector<std::unique_ptr<MarchLayout>> march_layouts_;  // by chunk length
   std::vector<long long> src_idx_, rec_idx_;  // grid indices of the points
+  int bwd_iters_ = 1;  // backward iterations of a run
   int res_cap_[2][2] = {{-1, -1}, {-1, -1}};  // [kind][precision] blocks on the chip at once, one a CU
   int res_twice_[2][kResTwiceRows + 1] = {};   // [precision][rows a wave] two forward blocks fit a CU: 1, -1, 0 not asked
   bool res_twice(int rows);

@@ -91,25 +91,63 @@ bool Propagator::res_twice(int rows) {
 // More parts pay backward only: 201x301 E=32 24.8 -> 20.9, E=60 46.9 -> 43.5,
 // 301x921 E=8 23.7 -> 20.3, E=13 35.2 -> 35.3, E=16 43.6 -> 40.6, 90x120 E=200
 // 41.9 -> 31.3; forward the strip walk has caught up (201x301 E=40: 14.0).
-int Propagator::plan_parts(int kind, int E, ResTiles& t) {
+// All of these fill their tiles of 62 z well; where the last tile of a column is
+// nearly empty (63, 125, 187 z) parts lose: backward 700x63 E=54 25.7 -> 33.2,
+// 340x125 E=75 30.1 -> 40.3, 700x187 E=22 24.5 -> 28.6, forward 700x63 E=30 8.9 ->
+// 9.7, 340x125 E=39 9.8 -> 10.5.  So parts are taken where their time, by the
+// tables below, is under the per-step kernels': of 1518 backward and 1315 forward
+// batches (62 to 331 z, 130 to 1000 x, 2 to 90 entries, both modes) none that is
+// taken was slower by more than 2%, but one (130x63 E=90, forward 7.3 -> 7.8).
+// 2 to 4 forward entries without a band could run side by side on streams, with
+// a launch a step, and do where their tiles are wide: 501x1501 E=2 7.0 against 7.3
+// us a step, 1000x331 E=3 (9 rows) 4.9 against 5.0, E=4 (6 rows, two blocks a CU)
+// 5.0 against 5.2, 700x331 E=4 (9 rows) 4.9 against 5.1, E=3 (7 rows) 4.7 against
+// 3.9.
+int Propagator::plan_parts(int kind, int E, bool band, ResTiles& t) {
   const auto rows = [](const ResTiles& r) { return (r.w + kResWaves - 1) / kResWaves; };
   const bool one = plan_resident(kind, E, t);
   if (resident_ == 1) return one ? 1 : 0;
+  if (one && kind == 0 && side_by_side(E, band) && rows(t) > (two_a_cu(kind, E, t) ? kResLanesRows2 : kResLanesRows)) return 0;
   if (one && rows(t) < (kind == 1 ? kResWideBwd : kResWideFwd)) return 1;
+  const double margin = kind == 1 ? 1.0 : 0.92;
   for (int n = 2; n <= (kind == 1 ? kResMaxPartsBwd : kResMaxPartsFwd) && n < E; n++) {
     ResTiles p;
     if (!plan_resident(kind, (E + n - 1) / n, p)) continue;
     const int r = rows(p);
     if (kind == 1 || n == 2 ? r > kResPartRows : r != 4 && (prec_ != kExact || r != 3)) continue;
+    const double steps = kind == 1 ? bwd_iters_ : g_.nt;
+    if (n * (part_us(kind, (E + n - 1) / n, p) + kResPartUs / steps) > margin * step_us(kind, E)) continue;
     t = p;
     return n;
   }
-  return one ? 1 : 0;
+  // one launch of very wide tiles (forward 15 or 16 rows, backward 10)
+  return one && (kind == 1 || kResWideUs[prec_] < margin * step_us(kind, E)) ? 1 : 0;
 }
 
-bool Propagator::runs_resident(int kind, int E) {
+// Microseconds a step of a resident launch by its rows a wave, the medians of the
+// measurements above (each within 10%): backward, forward with one block a CU
+// and with two.
+double Propagator::part_us(int kind, int E, const ResTiles& t) const {
+  static const double us[2][3][kResPartRows] = {
+      {{2.7, 2.9, 3.3, 3.9, 4.4, 4.9, 5.7}, {2.0, 2.2, 2.6, 2.9, 3.6, 3.8, 4.0}, {2.4, 2.7, 3.0, 3.4, 4.4, 5.1, 5.1}},
+      {{2.6, 2.8, 3.1, 3.3, 4.1, 4.5, 4.9}, {1.9, 2.1, 2.5, 2.8, 3.3, 3.5, 3.7}, {2.4, 2.7, 3.1, 3.5, 4.0, 4.7, 4.7}}};
+  const int rows = std::min((t.w + kResWaves - 1) / kResWaves, kResPartRows);
+  return us[prec_][kind == 1 ? 0 : two_a_cu(kind, E, t) ? 2 : 1][rows - 1];
+}
+// ... and of the per-step kernels: a launch, the columns of 64-z tiles, and the
+// points of the boundary band and sponge (fitted to the same batches, within 10%
+// from 600 tiles of 64 x 16 on).
+double Propagator::step_us(int kind, int E) const {
+  static const double fit[2][2][3] = {{{4.54, 0.00217, 0.0061}, {5.19, 0.00546, 0.0151}},
+                                      {{4.51, 0.00180, 0.0058}, {4.84, 0.00505, 0.0155}}};
+  const int ux = g_.nxpad - 2 * kHalo, uz = g_.nzpad - 2 * kHalo;
+  const double* f = fit[prec_][kind];
+  return f[0] + E * (f[1] * g_.ntz * ux / 16 + f[2] * (2 * uz + ux) / 100);
+}
+
+bool Propagator::runs_resident(int kind, int E, bool band) {
   ResTiles t;
-  if (plan_parts(kind, E, t) < 1) return false;
+  if (plan_parts(kind, E, band, t) < 1) return false;
   const ResLayout* l = res_layout(t);
   return l && l->fits;
 }
@@ -150,11 +188,9 @@ bool Propagator::plan_resident(int kind, int E, ResTiles& t) {
   // Measured over E (forward / backward microseconds a step, per-step kernels
   // -> resident): 201x301 E=1 4.7 -> 1.74, E=4 4.7 -> 2.7 / 8.1 -> 3.4, E=8
   // 6.2 -> 3.2 / 10.4 -> 5.2, E=11 6.9 -> 3.4 / 11.4 -> 9.1, E=16 7.9 -> 5.2,
-  // E=21 9.8 -> 8.1; 301x921 E=1 5.2 -> 2.7 / 6.6 -> 3.4, E=4 5.4 -> 5.2;
-  // 501x1501 E=1 6.8 -> 4.0 / 10.4 -> 6.2.  2 to 4 entries of wide tiles run
-  // faster side by side on streams with a launch a step (501x1501 E=2 7.0
-  // against 7.3).
-  return kind == 1 || E == 1 || E > kLanes || t.w <= kResLanesWidth;
+  // E=21 9.8 -> 8.1; 301x921 E=1 5.2 -> 2.7 / 6.6 -> 3.4;
+  // 501x1501 E=1 6.8 -> 4.0 / 10.4 -> 6.2.
+  return true;
 }
 
 Propagator::ResLayout* Propagator::res_layout(const ResTiles& t) {
@@ -270,7 +306,7 @@ bool Propagator::res_end(int kind, long long steps, hipEvent_t t0) {
 bool Propagator::resident_forward(int E, const float* rv, long long rvstride, const Sources& src, float* dcal,
                                   float* band, Fields& w, int rvdiv) {
   ResTiles t;
-  const int parts = plan_parts(0, E, t);
+  const int parts = plan_parts(0, E, band != nullptr, t);
   if (parts < 1) return false;
   const ResLayout* l = res_layout(t);
   if (!l || !l->fits) return false;
@@ -330,7 +366,7 @@ bool Propagator::resident_backward(int E, const float* rv, long long rvstride, c
                                    long long vstride, const float* band, float* grad, long long gstride, Fields& w,
                                    int rvdiv, int it_min, const std::vector<float>& wts) {
   ResTiles t;
-  const int parts = plan_parts(1, E, t);
+  const int parts = plan_parts(1, E, true, t);
   if (parts < 1) return false;
   const ResLayout* l = res_layout(t);
   if (!l || !l->fits) return false;

@@ -39,7 +39,7 @@ constexpr int kResLdz = 64 + 2 * 6;         // LDS row of a tile: z from -6 to 6
 constexpr int kResMaxPts = 512;             // sources or receivers of one tile, one per thread
 constexpr int kResMaxWidthFwd = 128;        // widest tile (x)
 constexpr int kResMaxWidthBwd = 80;          // (spills from 57 columns on; 69 columns still 9.1 against 11.4 us per step)
-constexpr int kResLanesWidth = 80;           // widest for 2 to 4 forward entries
+constexpr int kResLanesRows = 8, kResLanesRows2 = 5;  // most rows a wave for 2 to 4 forward entries, one block a CU and two
 constexpr int kResTwiceRows = 6;             // most rows a wave of which two forward blocks fit a CU
 
 // Fewest steps of a resident run: its launch, wait and clears cost about 10 us
@@ -50,6 +50,8 @@ constexpr int kResSteps = 5;
 constexpr int kResMaxPartsFwd = 3, kResMaxPartsBwd = 8;  // most launches of one run
 constexpr int kResWideFwd = 15, kResWideBwd = 10;  // rows a wave from which parts are faster than one launch
 constexpr int kResPartRows = 7;               // most rows a wave of a part
+constexpr double kResWideUs[2] = {8.6, 7.5};  // a forward step of kResWideFwd rows and more, exact and FP32
+constexpr double kResPartUs = 20;             // a part's launch and clears
 
 // Tiles of one entry: w x h outputs each (the last column and row may be smaller).
 struct ResTiles {

@@ -70,18 +70,22 @@ void launch_resident_fwd(const ResFwdArgs& a, int, hipStream_t) { resident(0, a.
 void launch_resident_bwd(const ResBwdArgs& a, int, hipStream_t) { resident(1, a.x); }
 }  // namespace swfwi
 
+struct Size {
+  int ux, uz, nt = 350, receivers = 1;  // update region; dt = 2 ms: imaging from step 151 on
+};
 struct Run {
   Propagator p;
   Fields w;
   std::vector<float> v;  // stands in for every array of the caller's
   int nt;
-  static Geometry geometry(int nt, bool crowded) {
+  static Geometry geometry(const Size& s) {
     Geometry g;
-    g.nx = 301, g.nz = 201, g.nb = 20, g.dt = 0.002f, g.dx = 20, g.fm = 12, g.nt = nt;
-    g.sx = {3}, g.sz = {1}, g.gx.assign(crowded ? 700 : 1, 9), g.gz.assign(crowded ? 700 : 1, 1);
+    g.nx = s.ux - 40, g.nz = s.uz - 20, g.nb = 20, g.dt = 0.002f, g.dx = 20, g.fm = 12, g.nt = s.nt;
+    g.sx = {3}, g.sz = {1}, g.gx.assign(s.receivers, 9), g.gz.assign(s.receivers, 1);
     return g;
   }
-  explicit Run(int nt_, bool crowded = false) : p(geometry(nt_, crowded), kExact), v(64), nt(nt_) {}
+  explicit Run(const Size& s, int precision = kExact) : p(geometry(s), precision), v(64), nt(s.nt) {}
+  explicit Run(int nt_, bool crowded = false) : Run(Size{341, 221, nt_, crowded ? 700 : 1}) {}
   Propagator::Sources src() { return Propagator::Sources{v.data(), 1, 0, nullptr, nullptr}; }
   // launches of the per-step kernels (trials included), resident launches; the run's route
   int forward(int E, bool band) {
@@ -126,9 +130,9 @@ static int backward_trials() {
   EXPECT(r.p.tile_choice_cached(1, 30) > 0);
   EXPECT(r.forward(30, true) == Propagator::kPerStep && g_fwd == nt && g_bwd == kTrial);
   EXPECT(r.backward(30) == Propagator::kPerStep && r.p.last_run[1].width == r.p.tile_choice_cached(1, 30));
-  Run s(nt);  // 40 entries: the forward a launch a step, the backward resident in parts
-  EXPECT(s.forward(40, true) == Propagator::kPerStep && g_fwd == nt + kTrial && g_bwd == 0);
-  EXPECT(s.backward(40) == Propagator::kResident && g_resident[1] >= 2 && g_bwd == 0);
+  Run s(350);  // 34 entries: the forward a launch a step, the backward resident in parts
+  EXPECT(s.forward(34, true) == Propagator::kPerStep && g_fwd == 350 + kTrial && g_bwd == 0);
+  EXPECT(s.backward(34) == Propagator::kResident && g_resident[1] >= 2 && g_bwd == 0);
   Run c(nt, true);  // more receivers at a place than a resident tile takes
   EXPECT(c.forward(8, true) == Propagator::kPerStep && g_bwd == kTrial && g_resident[0] == 0);
   EXPECT(c.backward(8) == Propagator::kPerStep);
@@ -221,6 +225,50 @@ static int few_steps() {
   return 0;
 }
 
+// Batches measured both ways (launches a run, 0: a launch a step), 200 backward
+// iterations; the region's last tiles of 62 z are nearly empty in the first ones.
+static int parts() {
+  struct {
+    Size s;
+    int E, fwd, bwd;
+  } const cases[] = {
+      {{340, 63}, 75, 0, 0},   // backward 19.5 us a launch a step, 23.2 in 5 parts
+      {{700, 63}, 30, 0, 0},   // forward 8.9, 9.7 in 2; backward 16.8, 18.8 in 4
+      {{700, 125}, 19, 0, 0},  // forward 9.7, 10.2 in 2; backward 17.3, 19.1 in 4
+      {{340, 125}, 54, 0, 0},  // backward 22.7, 27.8 in 5
+      {{340, 125}, 22, 2, 2},  // backward 12.4, 9.8 in 2
+      {{700, 187}, 22, 0, 0},  // backward 24.5, 28.6 in 6
+      {{341, 221}, 16, 1, 2},  // backward 13.7, 10.4 in 2
+      {{341, 221}, 22, 2, 3},  // forward 10.0, 6.7 in 2; backward 17.9, 15.5 in 3
+      {{981, 331}, 8, 2, 4},   // forward 11.9, 10.1 in 2; backward 23.7, 20.3 in 4
+      {{160, 110}, 100, 2, -1},  // forward 11.0, 6.8 in 2
+  };
+  for (const auto& c : cases) {
+    Run r(c.s);
+    r.p.set_tuning(false);
+    const int f = r.forward(c.E, true), fl = r.p.last_run[0].launches;
+    r.backward(c.E);
+    const bool rb = r.p.last_run[1].route == Propagator::kResident;
+    std::printf("%d x %d, %d entries: forward route %d, %d launches; backward route %d, %d\n", c.s.ux, c.s.uz, c.E, f,
+                fl, r.p.last_run[1].route, r.p.last_run[1].launches);
+    EXPECT(c.fwd ? f == Propagator::kResident && fl == c.fwd : f != Propagator::kResident);
+    if (c.bwd >= 0) EXPECT(c.bwd ? rb && r.p.last_run[1].launches == c.bwd : !rb);
+  }
+  // one launch of 15 rows in FP32: 7.6 us against 7.0
+  Run wide(Size{340, 63}, kFp32);
+  EXPECT(wide.forward(39, true) == Propagator::kPerStep);
+  // a launch of each part has to pay: 20 backward iterations in place of 200
+  // (31.4 us in 3 parts against 28.9; with 200 iterations 19.1 against 19.4)
+  Run few(Size{340, 331, 170}), many(Size{340, 331, 350});
+  few.forward(16, true), many.forward(16, true);
+  EXPECT(few.backward(16) == Propagator::kPerStep && many.backward(16) == Propagator::kResident);
+  // 2 to 4 entries run side by side where their tiles are wide: 331 z, 4 of 700 x 4.9 us against 5.1
+  Run four(Size{700, 331}), three(Size{700, 331});
+  EXPECT(four.forward(4, false) == Propagator::kSideBySide && three.forward(3, false) == Propagator::kResident);
+  EXPECT(four.forward(4, true) == Propagator::kResident);  // (with a band there are no streams to take)
+  return 0;
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "tuner") return tuner();
@@ -229,5 +277,6 @@ int main(int, char** argv) {
   if (what == "shared_chip") return shared_chip();
   if (what == "wait_limit") return wait_limit();
   if (what == "few_steps") return few_steps();
+  if (what == "parts") return parts();
   return 2;
 }

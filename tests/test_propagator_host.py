@@ -61,3 +61,9 @@ def test_the_wait_limit(driver):
 def test_a_few_steps_run_per_step(driver):
     """A run of fewer than 5 steps is not worth a resident launch."""
     run(driver, "few_steps")
+
+
+def test_parts_only_where_they_pay(driver):
+    """A batch goes as several resident launches only where that is faster than
+    a launch a step, however well its tiles of 62 z are filled."""
+    run(driver, "parts")
