@@ -267,6 +267,12 @@ int swfwi_batch_set_graphs(swfwi_batch b, int on);
 int swfwi_batch_set_tuning(swfwi_batch b, int on);
 /* A fixed tile width, 16, 24 or 32, or 0 for the rule and the tuner. */
 int swfwi_batch_set_tile_x(swfwi_batch b, int tile_x);
+/* The step kernel's form: strips of up to 116 z (124 of the 4th-order step)
+ * walked along x (1), tiles of 64 z (0), or by rule (-1, the default: tiles where
+ * strips would be half empty, the tuner's choice where it is close).  Results are the same bit for bit.
+ * swfwi_batch_strips receives the form in use. */
+int swfwi_batch_set_strips(swfwi_batch b, int mode);
+int swfwi_batch_strips(swfwi_batch b, int *on);
 /* Block order of the step launches: 0 entry by entry, 1 the shots of each
  * model tile by tile (a model tile is read once from HBM and then from L2),
  * or -1 for the rule (1) and the tuner, which times both orders with the

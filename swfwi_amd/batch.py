@@ -88,6 +88,15 @@ class Batch:
         """16, 24 or 32 (fixed), or 0 for the size rule and the tuner."""
         check(load().swfwi_batch_set_tile_x(self.h, int(tx)))
 
+    def set_strips(self, mode):
+        """Strips of z (1), tiles (0), or the rule (-1)."""
+        check(load().swfwi_batch_set_strips(self.h, int(mode)))
+
+    def strips(self):
+        t = C.c_int(0)
+        check(load().swfwi_batch_strips(self.h, C.byref(t)))
+        return bool(t.value)
+
     def set_block_order(self, order):
         """0 entry by entry, 1 a model's shots tile by tile, -1 the rule and the tuner."""
         check(load().swfwi_batch_set_block_order(self.h, int(order)))

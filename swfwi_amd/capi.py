@@ -95,6 +95,8 @@ SIGNATURES = {
     "swfwi_batch_set_tuning": (_I, [_VP, _I]),
     "swfwi_batch_tile_x": (_I, [_VP, C.POINTER(_I)]),
     "swfwi_batch_set_tile_x": (_I, [_VP, _I]),
+    "swfwi_batch_set_strips": (_I, [_VP, _I]),
+    "swfwi_batch_strips": (_I, [_VP, C.POINTER(_I)]),
     "swfwi_batch_set_block_order": (_I, [_VP, _I]),
     "swfwi_batch_block_order": (_I, [_VP, C.POINTER(_I)]),
     "swfwi_batch_bind_model": (_I, [_VP, _I, _I, _f32]),

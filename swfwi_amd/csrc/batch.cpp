@@ -51,11 +51,17 @@ void Batch::drop_graphs() {
     }
 }
 
+void Batch::rule_layout() {
+  const bool was = strips_;
+  strips_ = fixed_strips_ < 0 ? rule_strips() : fixed_strips_ == 1;
+  const int tx = fixed_x_ ? fixed_x_ : rule_width(), order = fixed_order_ >= 0 ? fixed_order_ : kRuleOrder;
+  if (strips_ != was || tile_x_ != tx || blk_order_ != order) layout_tiles(tx, order);
+}
+
 void Batch::set_tuning(bool on) {
   tune_ = on;
   tuned_ = false;
-  const int tx = fixed_x_ ? fixed_x_ : rule_x_, order = fixed_order_ >= 0 ? fixed_order_ : kRuleOrder;
-  if (tile_x_ != tx || blk_order_ != order) layout_tiles(tx, order);
+  rule_layout();
 }
 
 void Batch::set_tile_x(int tx) {
@@ -63,6 +69,36 @@ void Batch::set_tile_x(int tx) {
     fail(kErrArg, "batch tile width must be 0 (rule and tuner), 16, 24 or 32");
   fixed_x_ = tx;
   set_tuning(tune_);
+}
+
+void Batch::set_strips(int mode) {
+  if (mode < -1 || mode > 1) fail(kErrArg, "batch strips must be -1 (by rule), 0 or 1");
+  fixed_strips_ = mode;
+  set_tuning(tune_);
+}
+
+bool Batch::rule_strips() const {
+  return strip_rows_ < kBatchTilesFrom || strip_rows_ >= kBatchTilesTo ||
+         (double)tile_rows_ >= kBatchTilesAStrip * strip_rows_;
+}
+
+bool Batch::close_call() const {
+  if (fixed_strips_ >= 0) return false;
+  if ((double)tile_rows_ < kBatchTilesAStrip * strip_rows_) return strip_rows_ >= kBatchClose && strip_rows_ < kBatchCloseTo;
+  return (double)tile_rows_ < kBatchCloseCall * strip_rows_ && strip_rows_ >= kBatchTilesFrom && strip_rows_ < kBatchClose;
+}
+
+int Batch::rule_width() const {
+  if (!strips_) return tiles16_ >= kBatchWideTiles ? 24 : 16;
+  return strip_rows_ < 14000 ? 16 : strip_rows_ < 25000 ? 24 : strip_rows_ < kBatchLongWalks ? 32
+         : strip_rows_ < 120000 ? 24 : 32;
+}
+
+void Batch::step(const BatchKernelArgs& a, bool fwd, int prec, int units, hipStream_t s) const {
+  if (strips_)
+    launch_batch_step(a, fwd, prec, order_, units, s);
+  else
+    launch_batch_tiles(a, fwd, prec, order_, tile_x_, units, s);
 }
 
 void Batch::set_block_order(int order) {
@@ -88,9 +124,15 @@ void Batch::layout_tiles(int tx, int order) {
   tile0_.assign(ent_.size() + 1, 0);
   for (BatchEntry& e : ent_) {
     const int ux = e.nxpad - 2 * kHalo, uz = e.nzpad - 2 * kHalo;
-    e.nstrip = strip_count(uz);
-    e.h = 2 * ((uz + 2 * e.nstrip - 1) / (2 * e.nstrip));
-    e.rows = strip_rows_ < kBatchLongWalks ? tx / 2 - 2 : tx - 2;
+    if (strips_) {
+      e.nstrip = strip_count(uz);
+      e.h = 2 * ((uz + 2 * e.nstrip - 1) / (2 * e.nstrip));
+      e.rows = strip_rows_ < kBatchLongWalks ? tx / 2 - 2 : tx - 2;
+    } else {
+      e.nstrip = (uz + kBatchTileZ - 1) / kBatchTileZ;
+      e.h = kBatchTileZ;
+      e.rows = tx;
+    }
     e.nchunk = (ux + e.rows - 1) / e.rows;
   }
   for (size_t r = 0; r < ent_.size();) {
@@ -140,12 +182,19 @@ void Batch::tune() {
     launch_fill(grad_.get(), grad_len_, 0.f, s);
     if (snap_bytes_ >= 4) launch_fill_u32(reinterpret_cast<unsigned*>(snap_.get()), snap_bytes_ / 4, 0u, s);
   }
-  // candidates: the free widths x the free block orders
-  std::vector<std::pair<int, int>> cand;
-  for (int w : {16, 24, 32})
-    for (int o : {0, 1})
-      if ((!fixed_x_ || w == fixed_x_) && (fixed_order_ < 0 || o == fixed_order_)) cand.push_back({w, o});
-  const std::pair<int, int> rule{fixed_x_ ? fixed_x_ : rule_x_, fixed_order_ >= 0 ? fixed_order_ : kRuleOrder};
+  // candidates: the free widths x the free block orders, in the form in use or both
+  struct Choice {
+    bool strips;
+    int width, order;
+    bool operator==(const Choice& o) const { return strips == o.strips && width == o.width && order == o.order; }
+  };
+  const Choice rule{strips_, tile_x_, blk_order_};
+  std::vector<Choice> cand;
+  for (bool form : {strips_, !strips_})
+    for (int w : {16, 24, 32})
+      for (int o : {0, 1})
+        if ((form == strips_ || close_call()) && (!fixed_x_ || w == fixed_x_) && (fixed_order_ < 0 || o == fixed_order_))
+          cand.push_back({form, w, o});
   if (cand.size() < 2) return;
   std::vector<float> t[2];
   t[0].assign(cand.size(), 0.f);
@@ -155,21 +204,22 @@ void Batch::tune() {
   SWFWI_HIP(hipEventCreate(&e1));
   for (int round = 0; round < 3; round++)
     for (size_t wi = 0; wi < cand.size(); wi++) {
-      layout_tiles(cand[wi].first, cand[wi].second);
+      strips_ = cand[wi].strips;
+      layout_tiles(cand[wi].width, cand[wi].order);
       BatchKernelArgs a = args(true);
       a.tap = nullptr;
       SWFWI_HIP(hipEventRecord(e0, s));
       for (int r = 0; r < kReps; r++) {
         a.it_or_k = r;
         a.rot = r;
-        launch_batch_step(a, true, prec_, order_, tile0_[n], s);
+        step(a, true, prec_, tile0_[n], s);
       }
       if (bwd) {
         BatchKernelArgs b = args(false);
         for (int r = 0; r < kReps; r++) {
           b.it_or_k = r;
           b.rot = r;
-          launch_batch_step(b, false, prec_, order_, tile0_[n], s);
+          step(b, false, prec_, tile0_[n], s);
         }
       }
       SWFWI_HIP(hipEventRecord(e1, s));
@@ -189,7 +239,8 @@ void Batch::tune() {
     const bool faster = t[0][i] < (1.f - kBatchTuneMargin) * t[0][ri] && t[1][i] < (1.f - kBatchTuneMargin) * t[1][ri];
     if (faster && std::max(t[0][i], t[1][i]) < std::max(t[0][best], t[1][best])) best = i;
   }
-  layout_tiles(cand[best].first, cand[best].second);
+  strips_ = cand[best].strips;
+  layout_tiles(cand[best].width, cand[best].order);
 }
 
 void Batch::set_snap_prec(int p) {
@@ -214,14 +265,16 @@ void Batch::build() {
   std::vector<float> amp, wts;
   long long model_len = 0, dcal_len = 0, grad_len = 0;
   int mbase = 0;
-  // chunk length from the batch's size in strip rows
+  // the kernel's form and width from the batch's size
   for (const BatchGroup& G : g_) {
-    const int strips = strip_count(G.nz + G.nb);
-    strip_rows_ += (long long)G.nmodels * (long long)G.sx.size() * strips * (G.nx + 2 * G.nb);
+    const long long n = (long long)G.nmodels * (long long)G.sx.size(), ux = G.nx + 2 * G.nb, uz = G.nz + G.nb;
+    const long long tz = (uz + kBatchTileZ - 1) / kBatchTileZ;
+    strip_rows_ += n * strip_count((int)uz) * ux;
+    tile_rows_ += n * tz * ux;
+    tiles16_ += n * tz * ((ux + 15) / 16);
   }
-  rule_x_ = strip_rows_ < 14000 ? 16 : strip_rows_ < 25000 ? 24 : strip_rows_ < kBatchLongWalks ? 32
-            : strip_rows_ < 120000 ? 24 : 32;
-  tile_x_ = rule_x_;
+  strips_ = rule_strips();
+  tile_x_ = rule_width();
   for (size_t gi = 0; gi < g_.size(); gi++) {
     const BatchGroup& G = g_[gi];
     const int ns = (int)G.sx.size();
@@ -387,7 +440,7 @@ void Batch::run_loop(bool fwd) {
         launch_batch_tap(a, columns, n, s);
         a.tap_k = -1;
       }
-      launch_batch_step(a, true, prec_, order_, tile0_[act], s);
+      step(a, true, prec_, tile0_[act], s);
       if (hook_ && (it + 2) % kSnapEvery == 0) {
         // after step it the buffer step it wrote holds the field at it+1
         float* cur = (it & 1) == 0 ? fa_.get() : fb_.get();
@@ -405,7 +458,7 @@ void Batch::run_loop(bool fwd) {
       while (act > 0 && ent_[act - 1].nt - ent_[act - 1].it_last <= k) act--;
       a.it_or_k = k;
       a.rot = k;
-      launch_batch_step(a, false, prec_, order_, tile0_[act], s);
+      step(a, false, prec_, tile0_[act], s);
     }
   }
 }
@@ -497,7 +550,7 @@ void Batch::step_from(const float* prev_host, const float* cur_host, int it0, in
     while (act > 0 && ent_[act - 1].nt <= it) act--;
     a.it_or_k = it;
     a.rot = k;
-    launch_batch_step(a, true, kSnapNone, order_, tile0_[act], s);
+    step(a, true, kSnapNone, tile0_[act], s);
     if (hook_ && (it + 2) % kSnapEvery == 0) {  // the correction, as in forward runs
       float* cur = (k & 1) == 0 ? fa_.get() : fb_.get();
       float* prev = (k & 1) == 0 ? fb_.get() : fa_.get();

@@ -32,6 +32,23 @@ constexpr int kSnapEvery = 4;
 // or 30, 74 with 46, 78 with 62; backward 27.4 / 26.2 / 26.2).
 constexpr int kBatchStrip10 = 116, kBatchStrip4 = 124;
 constexpr int kBatchLongWalks = 60000;
+// A batch whose strips would be half empty runs in tiles of 64 z x 16, 24 or 32 x
+// (one a block; 24 from kBatchWideTiles tiles of 64 x 16 on: 16 entries of the
+// 501x1501 grid, 14112 of them, forward + backward 300.6 ms at 24, 310.4 at 32,
+// 329.4 at 16; 16 entries of the 793x277 padded coarse grid, 3920, 54.4 / 55.1 /
+// 61.1 ms at 16 / 24 / 32).  A strip's row costs the same however few of its z are
+// outputs, a column of tiles by their number.  Measured, a forward and a backward
+// run, speed of strips over tiles at one tile a strip (44, 64, 117, 125, 128 z) by
+// strip rows: below 7000 1.06-1.16 (10th and 4th order alike; so few waves are
+// bound by their own walk), 7200 to 16800 0.81-1.10, to 43200 0.82-0.93, 54000 to
+// 60000 0.84-1.02, to 125000 0.82-1.07 (30 to 54 z) and 0.95-1.11, 0.95-1.14 above.
+// At 4 tiles in 3 strips (233 to 256 z) 0.91-1.12 between 7000 and 45000 and
+// 1.12-1.26 above; at 3 in 2 (140 to 192 z) 0.94-1.36, at 2 a strip 0.97-1.6.
+// Where it is close the tuner times both forms.
+constexpr int kBatchTileZ = 64;
+constexpr int kBatchWideTiles = 8000;
+constexpr int kBatchTilesFrom = 7000, kBatchTilesTo = 60000, kBatchClose = 45000, kBatchCloseTo = 130000;
+constexpr double kBatchTilesAStrip = 1.2, kBatchCloseCall = 1.45;
 constexpr int kBlkTileBits = 20;  // tiles per entry < 2^20, entries < 2^11
 constexpr int kRuleOrder = 1;      // block order without tuning: a model's shots tile by tile
 constexpr float kBatchTuneMargin = 0.03f;
@@ -60,8 +77,8 @@ struct BatchGroup {
 // Device description of one entry (one shot of one model).
 struct BatchEntry {
   int nxpad, nzpad;      // padded grid; z contiguous (ld = nzpad)
-  int nstrip, h;         // strips along z of the update region [6, n-6), h outputs each
-  int nchunk, rows;      // chunks along x of `rows` rows each
+  int nstrip, h;         // strips (or tiles) along z of the update region [6, n-6), h outputs each
+  int nchunk, rows;      // chunks (or tiles) along x of `rows` rows each
   int damp;              // width of the sponge profile (bx0 = nb + 6)
   float dscale;          // sponge strength factor
   int nt, it_last;       // forward steps; last backward iteration run
@@ -102,6 +119,8 @@ struct BatchKernelArgs {
 void launch_batch_init_fwd(const BatchKernelArgs& a, int nentries, hipStream_t s);
 // one step of the first `units` waves of work of the block list
 void launch_batch_step(const BatchKernelArgs& a, bool fwd, int prec, int order, int units, hipStream_t s);
+// the same in tiles: the first `tiles` blocks of the list
+void launch_batch_tiles(const BatchKernelArgs& a, bool fwd, int prec, int order, int tile_x, int tiles, hipStream_t s);
 // tap slot a.tap_k of every entry (columns: the most coarse columns of one)
 void launch_batch_tap(const BatchKernelArgs& a, int columns, int nentries, hipStream_t s);
 void launch_batch_init_bwd(const BatchKernelArgs& a, int nentries, hipStream_t s);
@@ -134,6 +153,9 @@ class Batch {
   // A fixed tile width (16, 24 or 32), or 0 for the rule and the tuner.
   void set_tile_x(int tx);
   int tile_x() const { return tile_x_; }
+  // Strips (1), tiles (0), or the rule (-1).  Same results.
+  void set_strips(int mode);
+  bool strips() const { return strips_; }
   // Block order of a launch: 0 entry by entry (the tiles of one entry, then
   // the next), 1 the shots of each model tile by tile (a model tile is read
   // from HBM once and from L2 by the model's other shots), or -1 for the
@@ -199,6 +221,7 @@ class Batch {
   void build();
   void layout_tiles(int tx, int order);  // entry tile counts and the block list
   void tune();
+  void rule_layout();
   void drop_graphs();
   void run_loop(bool fwd);
   BatchKernelArgs args(bool fwd);
@@ -221,8 +244,15 @@ class Batch {
   std::vector<int> tile0_;           // per run index, prefix of tiles
   int strip_count(int uz) const;     // strips of an update region uz high
   long long strip_rows_ = 0;         // strips x rows of x over all entries
+  long long tile_rows_ = 0;          // tiles along z x rows of x
+  long long tiles16_ = 0;            // tiles of 64 x 16
+  bool strips_ = true;
+  int fixed_strips_ = -1;
+  bool rule_strips() const;
+  bool close_call() const;  // the tuner decides between strips and tiles
+  int rule_width() const;
+  void step(const BatchKernelArgs& a, bool fwd, int prec, int units, hipStream_t s) const;
   int tile_x_ = 16;                  // step-kernel tile width
-  int rule_x_ = 16;                  // the size rule's width
   bool tune_ = true, tuned_ = false;
   int fixed_x_ = 0;                  // a width set by the caller, 0 for none
   int blk_order_ = 1;                // block order in use

@@ -763,6 +763,21 @@ int swfwi_batch_set_tile_x(swfwi_batch b, int tile_x) {
   });
 }
 
+int swfwi_batch_set_strips(swfwi_batch b, int mode) {
+  return guarded([&] {
+    NEED(b);
+    b->b->set_strips(mode);
+  });
+}
+
+int swfwi_batch_strips(swfwi_batch b, int* on) {
+  return guarded([&] {
+    NEED(b);
+    NEED(on);
+    *on = b->b->strips() ? 1 : 0;
+  });
+}
+
 int swfwi_batch_set_block_order(swfwi_batch b, int order) {
   return guarded([&] {
     NEED(b);
