@@ -432,14 +432,9 @@ void Batch::run_loop(bool fwd) {
       while (act > 0 && ent_[act - 1].nt <= it) act--;
       a.it_or_k = it;
       a.rot = it;
+      a.tap_k = -1;
       for (size_t k = 0; k < taps_.size(); k++)
         if (taps_[k] == it) a.tap_k = (int)k;  // the last listed slot of the step
-      if (a.tap_k >= 0) {
-        int columns = 0;
-        for (const BatchEntry& e : ent_) columns = std::max(columns, e.tap_nx);
-        launch_batch_tap(a, columns, n, s);
-        a.tap_k = -1;
-      }
       step(a, true, prec_, tile0_[act], s);
       if (hook_ && (it + 2) % kSnapEvery == 0) {
         // after step it the buffer step it wrote holds the field at it+1

@@ -121,8 +121,6 @@ void launch_batch_init_fwd(const BatchKernelArgs& a, int nentries, hipStream_t s
 void launch_batch_step(const BatchKernelArgs& a, bool fwd, int prec, int order, int units, hipStream_t s);
 // the same in tiles: the first `tiles` blocks of the list
 void launch_batch_tiles(const BatchKernelArgs& a, bool fwd, int prec, int order, int tile_x, int tiles, hipStream_t s);
-// tap slot a.tap_k of every entry (columns: the most coarse columns of one)
-void launch_batch_tap(const BatchKernelArgs& a, int columns, int nentries, hipStream_t s);
 void launch_batch_init_bwd(const BatchKernelArgs& a, int nentries, hipStream_t s);
 void launch_fill_u32(unsigned* p, long long n, unsigned v, hipStream_t s);
 void launch_sub(const float* a, const float* b, float* out, long long n, hipStream_t s);  // out = a - b

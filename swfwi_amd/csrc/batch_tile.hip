@@ -281,6 +281,11 @@ __global__ __launch_bounds__(kBT) void k_batch_step(BatchKernelArgs a) {
       if (inject_next && p == E.src) v += a.amp[E.amp0 + it + 1];
       vmax = fmaxf(vmax, fabsf(v));
       if (rec && a.dcal) a.dcal[E.dcal + (long long)it * E.ng + (gx - rx0)] = c;
+      if (a.tap_k >= 0 && ((gx | (gz - E.tap_oz)) & 1) == 0) {  // a point of the 2x-coarser grid
+        const int xc = (gx + kBH) >> 1, zc = (gz + kBH - E.tap_oz) >> 1;
+        if (xc < E.tap_nx && zc < E.tap_nz)
+          a.tap[E.tap + ((long long)a.tap_k * E.tap_nx + xc) * E.tap_nz + zc] = c;
+      }
       if constexpr (PREC != kSnapNone) {
         if (snap_now) snap_store<PREC>(snapb, p, c, scale);
       }

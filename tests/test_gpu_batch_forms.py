@@ -72,6 +72,39 @@ def test_steps_and_taps_in_tiles():
     b.close()
 
 
+# one strip, two of 59 and 58 rows, three; odd and even sizes, both row offsets
+@pytest.mark.parametrize("order", [capi.ORDER_10, capi.ORDER_4])
+@pytest.mark.parametrize("nx,nz,oz", [(33, 37, 0), (34, 38, 1), (41, 109, 0), (40, 109, 1), (70, 244, 1)])
+def test_taps_hold_the_field_of_their_step(nx, nz, oz, order):
+    """A tap is the field at its step (taken by step_from from the first row of
+    data, where the receivers see the source's first sample) at the even points."""
+    nb, h, steps = 8, 6, [0, 1, 39, 40]
+    g = group(nx, nz, nb, 2, 160, gz=1)
+    b = Batch([g], snap_prec=capi.SNAP_NONE, order=order)
+    b.bind_model(0, 0, models_for(g, 3)[0])
+    b.set_taps(steps, oz)
+    for mode in (0, 1):
+        b.set_strips(mode)
+        print(f"taps {nx}x{nz} order {order} offset {oz}, strips {mode}", flush=True)
+        d = b.forward().reshape(g.ns, g.nt, nx)
+        taps = b.taps()
+        prev, cur = np.zeros((2, g.ns) + g.shape, np.float32)
+        for e in range(g.ns):
+            cur[e, h + nb + g.sx[e], h + 1] = d[e, 0, g.sx[e]]
+        assert np.all(np.count_nonzero(cur, axis=(1, 2)) == 1)
+        at = 0
+        for k, step in enumerate(steps):
+            if step > at:
+                prev, cur = (f.reshape((g.ns,) + g.shape) for f in b.step_from(prev, cur, at, step - at))
+                at = step
+            for e in range(g.ns):
+                want = np.zeros_like(taps[e][k])
+                inner = cur[e, h:-h, h + oz:-h][::2, ::2][:want.shape[0] - h, :want.shape[1] - h]
+                want[h:, h:][:inner.shape[0], :inner.shape[1]] = inner
+                assert same(taps[e][k], want), (mode, step, e)
+    b.close()
+
+
 @pytest.mark.parametrize("nx,nz,nb,ns,order,strips", [
     (270, 49, 15, 12, capi.ORDER_10, True),    # 64 z, 3600 strip rows: too few waves for tiles to pay
     (270, 49, 15, 48, capi.ORDER_10, False),   # 14400: 0.83 of the tiles' speed as strips
