@@ -29,14 +29,13 @@
 // entry by entry (a tile's x-halo, the neighbouring columns of the same
 // entry, is re-read from L2); the launcher picks the order.
 //
-// Precision: kExact reproduces the reference's expression trees
-// (fd4t10s-damp-zjh.c:44-54,85-88; fd4t10s-zjh.c:28-38,49-52): float ring
-// sums, float coefficient products, double accumulation of -4.0*a0*p and the
-// (2-2d+d^2)p / 2p terms, one rounding to float on store, no contraction.  The
-// library is compiled with -ffp-contract=off; kFp32 uses explicit fmaf.
-#include "kernels.h"
-
+// Precision: the arithmetic of a point is step_math.h's, shared with the
+// resident time loop and the strip walk.  The library is compiled with
+// -ffp-contract=off, so only the fused products written there are fused.
 #include <type_traits>
+
+#include "kernels.h"
+#include "step_math.h"
 
 namespace swfwi {
 namespace {
@@ -74,35 +73,6 @@ struct Tile {
   static_assert(2 * UX <= kThreads - (UX % kRows) * kTZ, "ring points fit the wavefronts with fewer rows");
 };
 
-// Zhang Jinhai coefficients as float, as the reference stores them.
-constexpr float A0 = 1.53400796f, A1 = 1.78858721f, A2 = -0.31660756f;
-constexpr float A3 = 0.07612173f, A4 = -0.01626042f, A5 = 0.00216736f;
-constexpr double M4A0 = -4.0 * (double)A0;
-constexpr float C12 = 1.0f / 12;
-
-// u2 from the centre value and the five ring sums r_k = ((z-k + z+k) + x-k)
-// + x+k, summed as the reference does.
-template <int P>
-__device__ __forceinline__ float u2_sum(float s0, float r1, float r2, float r3, float r4, float r5) {
-  if constexpr (P == kExact) {
-    double acc = M4A0 * (double)s0;
-    acc = acc + (double)(A1 * r1);
-    acc = acc + (double)(A2 * r2);
-    acc = acc + (double)(A3 * r3);
-    acc = acc + (double)(A4 * r4);
-    acc = acc + (double)(A5 * r5);
-    return (float)acc;
-  } else {
-    float acc = (-4.0f * A0) * s0;
-    acc = __builtin_fmaf(A1, r1, acc);
-    acc = __builtin_fmaf(A2, r2, acc);
-    acc = __builtin_fmaf(A3, r3, acc);
-    acc = __builtin_fmaf(A4, r4, acc);
-    acc = __builtin_fmaf(A5, r5, acc);
-    return acc;
-  }
-}
-
 template <int P, int LZ>
 __device__ __forceinline__ float u2_at(const float* __restrict__ s) {
   // s: LDS element; z neighbours at +-k, x neighbours at +-k*LZ
@@ -131,33 +101,10 @@ __device__ __forceinline__ float u2_window(const float* __restrict__ s, const fl
 template <bool DAMPED, int P>
 __device__ __forceinline__ float update_vals(float c, float p, float rv, float u0, float zm, float zp, float xm,
                                              float xp, float delta) {
-  float lap = ((zm + zp) + xm) + xp;
-  lap = lap - 4 * u0;
-  const float cc = (C12 * rv) * rv;
-  if constexpr (P == kExact) {
-    double acc;
-    if constexpr (DAMPED) {
-      const double a = (2. - (double)(2 * delta)) + (double)(delta * delta);
-      const float b = 1 - 2 * delta;
-      acc = a * (double)c;
-      acc = acc - (double)(b * p);
-    } else {
-      acc = 2. * (double)c;
-      acc = acc - (double)p;
-    }
-    acc = acc + (double)(rv * u0);
-    acc = acc + (double)(cc * lap);
-    return (float)acc;
-  } else {
-    float a = 2.0f, b = 1.0f;
-    if constexpr (DAMPED) {
-      a = (2.0f - 2 * delta) + delta * delta;
-      b = 1 - 2 * delta;
-    }
-    float acc = __builtin_fmaf(a, c, -(b * p));
-    acc = __builtin_fmaf(rv, u0, acc);
-    return __builtin_fmaf(cc, lap, acc);
-  }
+  const float lap = lap_of<P>(u0, zm, zp, xm, xp), cc = cc_of(rv);
+  Damp<P> d{};
+  if constexpr (DAMPED) d = damp_coeffs<P>(delta);
+  return update_lap<DAMPED, P>(c, p, rv, cc, u0, lap, d);
 }
 
 // The u2 column of a thread's outputs: the thread's z, the rows of its PER
