@@ -40,6 +40,22 @@ def measured_traffic(kernel, workload):
     return None
 
 
+def ran(s, kind):
+    """(kernel, how it went) of the solver's last forward (0) or backward (1)
+    run: which of its routes it took, launches and tile width."""
+    route, launches, width, _ = s.last_run(kind)
+    if route == "resident":
+        parts = f"{launches} launches" if launches > 1 else "one launch"
+        return ("k_resident_fwd", "k_resident_bwd")[kind], (
+            f"a whole time loop is {parts} (tiles {width} wide) that keeps its tiles on the chip, so launches, "
+            "avg_launch_us and algorithmic_bytes_per_launch count time steps, and achieved is an effective "
+            "(algorithmic) bandwidth: the fields do not pass through memory at all")
+    if route == "strips":
+        return "k_fwd_march", f"one launch a step, strips of z in chunks of {width} rows"
+    name = "k_fwd_step" if kind == 0 else "k_bwd_step or, for few tiles, k_bwd_split"
+    return name, f"one launch a step{' and lane' if route == 'side by side' else ''}, tiles {width} wide"
+
+
 def cpu_epoch(case, encoded, dobs):
     """One whole epoch of the oracle with the reference's threading (ESS:
     EssFwiFramework::epoch, essfwiframework.cpp:191-239; plain FWI:
@@ -183,6 +199,7 @@ def mixed_workload(args):
                         "backward_ms": float(np.mean(bms)), "points": pts, "snapshot_bytes": inf["snapshot_bytes"],
                         "entries": inf["entries"], "gpts": pts / wall / 1e9, "bytes": byts,
                         "tile_x": b.tile_x(), "block_order": b.block_order(),
+                        "kernel": "k_batch_march" if b.strips() else "k_batch_step",
                         # one launch per step of the longest entry, forward, and per backward
                         # iteration (the taper ends the backward ~0.3 s early)
                         "launches": max(g.nt for g in groups) + max(g.nt - int(round(0.3 / g.dt)) for g in groups)}
@@ -208,7 +225,7 @@ def mixed_workload(args):
         "roofline": {"bound": "hbm", "achieved": round(timing["bytes"] / (timing["device_ms"] * 1e-3) / 1e9, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(timing["bytes"] / (timing["device_ms"] * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                     "traffic": None, "kernel": "k_batch_march",
+                     "traffic": None, "kernel": timing["kernel"],
                      "algorithmic_bytes_per_launch": round(timing["bytes"] / timing["launches"]),
                      "avg_launch_us": round(1e3 * timing["device_ms"] / timing["launches"], 2),
                      "launches": timing["launches"],
@@ -437,6 +454,7 @@ def main():
     t_obs = time.perf_counter() - t0
     obs_ms, obs_n = s.kernel_times()["fwd"]
     obs_pu = s.counters()[0][0] - pu_obs0
+    obs_kernel, obs_how = ran(s, 0)
     s.set_timing(False)
     print(f"[bench] observed data {case.ns} shots in {t_obs:.2f} s", file=sys.stderr, flush=True)
     s.bind_velocity(vi)
@@ -479,30 +497,27 @@ def main():
     fwd_pu = pu1[0] - pu0[0]
     bwd_pu = (pu1[1] - pu0[1]) / 2.0
     if bwd_ms >= fwd_ms:
-        name, ms, n, byts = "k_resident_bwd", bwd_ms, bwd_n, bwd_pu * BWD_BYTES_PER_PT
+        (name, how), ms, n, byts = ran(s, 1), bwd_ms, bwd_n, bwd_pu * BWD_BYTES_PER_PT
     else:
-        name, ms, n, byts = "k_resident_fwd", fwd_ms, fwd_n, fwd_pu * FWD_BYTES_PER_PT
+        (name, how), ms, n, byts = ran(s, 0), fwd_ms, fwd_n, fwd_pu * FWD_BYTES_PER_PT
     achieved = byts / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic(name, args.workload), "kernel": name,
             "algorithmic_bytes_per_launch": round(byts / max(n, 1)),
             "avg_launch_us": round(1e3 * ms / max(n, 1), 3), "launches": n,
             "note": ("one supershot, and the two line-search trials as a batch of two" if ess else
-                     "batches of 11 and 22 small-grid entries (22 as two launches)") +
-                    ": a whole time loop is one launch that keeps its tiles on the chip, so launches, "
-                    "avg_launch_us and algorithmic_bytes_per_launch count time steps, and achieved is an effective "
-                    "(algorithmic) bandwidth: the fields do not pass through memory at all"}
+                     "batches of 11 and 22 small-grid entries") + "; the last run of this direction: " + how}
 
     obs_bytes = obs_pu * FWD_BYTES_PER_PT
     obs_achieved = obs_bytes / (obs_ms * 1e-3) / 1e9 if obs_ms > 0 else 0.0
     roof_batched = {"bound": "hbm", "achieved": round(obs_achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(obs_achieved / HBM_PEAK_GBS, 4),
-                    "traffic": None, "kernel": "k_fwd_march" if ess else "k_resident_fwd",
+                    "traffic": None, "kernel": obs_kernel,
                     "entries": case.ns, "algorithmic_bytes_per_launch": round(obs_bytes / max(obs_n, 1)),
                     "avg_launch_us": round(1e3 * obs_ms / max(obs_n, 1), 3), "launches": obs_n,
                     "note": "the observed-data generation before the timed epochs (fm-damp): every shot in one "
                             "batched forward loop, untimed for value; algorithmic bytes charge the shared model "
-                            "per shot"}
+                            "per shot; " + obs_how}
 
     cpu = None
     if not args.no_cpu_baseline:

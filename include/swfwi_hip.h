@@ -86,8 +86,12 @@ int swfwi_random_codes(int seed, int skip, int n, int *codes);
 
 /* ---- device-resident propagator (Damp4t10d) ------------------------------ */
 /* Damp4t10d(allSrcPos, allGeoPos, dt, dx, fm, nb, nt) (damp4t10d.cpp:367-376)
- * on the current HIP device, one stream per handle; handles are not
- * thread-safe, many may coexist.  nb must be >= 6. */
+ * on the current HIP device, one stream per handle; a handle is not
+ * thread-safe, but many may coexist and run from threads of their own.  A run
+ * that takes the resident time loop (swfwi_solver_set_resident) holds the
+ * device's other resident runs, of any handle of the process, until it has
+ * ended, and its call waits for it; all other runs go onto their handle's
+ * stream side by side.  nb must be >= 6. */
 int swfwi_solver_create(swfwi_solver *out, int nx, int nz, int nb, float dt, float dx, float fm, int nt, int ns,
                         const int *sx, const int *sz, int ng, const int *gx, const int *gz, int precision);
 int swfwi_solver_destroy(swfwi_solver h);

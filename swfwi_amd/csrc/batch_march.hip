@@ -13,9 +13,9 @@
 // four, and the update lags the Laplacian by one row.
 //
 // What bounds it: memory in large batches (112 entries of three grid sizes,
-// 29.8 M points: 72 us a step, against 101 us of the tiled form this replaces,
-// which issued about 116 vector instructions per point for staging, ring
-// recomputation and index arithmetic around the ~32 of the step itself and was
+// 29.8 M points: 72 us a step, against 101 us of the tiled form (batch_tile.hip),
+// which issues about 116 vector instructions per point for staging, ring
+// recomputation and index arithmetic around the ~32 of the step itself and is
 // bound by them at any size); in small ones the walk itself (a lone wave issues
 // one instruction per 4 cycles, about 0.35 us a row), hence the short chunks.
 //

@@ -84,7 +84,9 @@ bool Propagator::res_twice(int rows) {
 // entries of 250x500, 7.07 -> 7.3).  Parts of 9 rows a wave lose: 301x921 E=5
 // 9.4 -> 10.0 (in three of 3 rows 8.35).  Three parts pay at 4 rows, in exact
 // mode also at 3 (250x500 E=12 10.0 -> 9.7, in FP32 9.35 -> 10.15); 301x921
-// E=12 in FP32, 6 rows, 13.6 -> 14.3.  Backward: 201x301 E=13 12.6 -> 9.2,
+// E=12 in FP32, 6 rows, 13.6 -> 14.3.  Three of 5 rows are left to the per-step
+// kernels: whole calls of 201x301 E=38 13.8 -> 14.2 in exact mode, 12.9 -> 12.6 in
+// FP32, 301x921 E=9 13.1 -> 13.2, but 90x120 E=160 16.3 -> 13.5.  Backward: 201x301 E=13 12.6 -> 9.2,
 // E=16 13.7 -> 10.4, E=22 17.9 -> 15.5, 301x921 E=6 19.1 -> 15.5, 90x120
 // E=100 20.6 -> 18.4; one launch of 10 rows 12.4 -> 9.2 (90x120 E=60), of 9
 // rows the same, of 8 rows 7.8 -> 8.1 (201x301 E=10).

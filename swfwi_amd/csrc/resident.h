@@ -33,7 +33,7 @@
 
 namespace swfwi {
 
-constexpr int kResWaves = 8;                // waves of a field in the backward kernel (two fields), half the forward's
+constexpr int kResWaves = 8;                // waves of a field (the forward kernel has one, the backward two)
 constexpr int kResTileZ = 62;               // most outputs along z: lanes 1..62, lanes 0 and 63 the u2 ring
 constexpr int kResLdz = 64 + 2 * 6;         // LDS row of a tile: z from -6 to 69
 constexpr int kResMaxPts = 512;             // sources or receivers of one tile, one per thread

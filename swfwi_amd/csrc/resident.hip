@@ -639,7 +639,13 @@ __device__ __forceinline__ void bwd_half(const ResBwdArgs& a, BwdTile<P, R>& t) 
     if (has) pt.amp[(it - 1) & 1][p.tid] = anext;
     if (more) {
       __syncthreads();  // both fields' new edges are in LDS
-      // the emptied words have arrived before any word of this step leaves
+      // the emptied words have arrived before any word of this step leaves.
+      // Both are relaxed stores, so what orders them is this wait and that the
+      // hardware acknowledges an agent-scope store only once it is past the
+      // L2, where a reader's polls go.  A word whose emptying came late would
+      // be taken as data unnoticed (a late stamp of the forward loop is only
+      // polled again).  Per word is enough: a word has one writer and one
+      // reader thread, the same at every step.
       __builtin_amdgcn_s_waitcnt(0);
       asm volatile("" ::: "memory");
       u64* now = words + turn * copy;

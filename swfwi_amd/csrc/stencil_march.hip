@@ -7,8 +7,9 @@
 //
 // What bounds it: vector issue in exact mode (about 100 instructions per two
 // points, 48 of them FP64 or conversions at 4 cycles each): 60 entries of
-// 301x921 with one model take 46 us a step, 56 tiled (their fields alone would
-// move in 38); 60 members of 201x301 with a model each 17.1, 20.8 tiled.
+// 301x921 with one model take 46 us a step over 400 steps and 50 over 4000, 56
+// tiled over 400 (their fields alone would move in 38); 60 members of 201x301
+// with a model each 17.1, 20.8 tiled.
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
