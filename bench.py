@@ -47,7 +47,7 @@ def ran(s, kind):
     if route == "resident":
         parts = f"{launches} launches" if launches > 1 else "one launch"
         return ("k_resident_fwd", "k_resident_bwd")[kind], (
-            f"a whole time loop is {parts} (tiles {width} wide) that keeps its tiles on the chip, so launches, "
+            f"a whole time loop is {parts} with its tiles ({width} wide) kept on the chip, so launches, "
             "avg_launch_us and algorithmic_bytes_per_launch count time steps, and achieved is an effective "
             "(algorithmic) bandwidth: the fields do not pass through memory at all")
     if route == "strips":

@@ -8,6 +8,7 @@
     python -m swfwi_amd.profile_workloads enfwi     # ensemble-Kalman FWI epochs, 301x921, N members
     python -m swfwi_amd.profile_workloads sweep     # step-kernel time per tile width and batch size
     python -m swfwi_amd.profile_workloads net       # network apply kernel over 16 coarse fields of the 501x1501 case
+    python -m swfwi_amd.profile_workloads mixed     # a mixed-size batch's forward and backward run, 112 entries, short
 """
 import argparse
 import sys
@@ -217,9 +218,35 @@ def run_net(reps):
               flush=True)
 
 
+def run_mixed(nt):
+    """One forward and one backward run of a mixed-size batch: 4 models of
+    201x301 over nt steps, 2 of 301x921 over 2 nt, 1 of 501x1501 over 3 nt,
+    16 shots each, BF16 checkpoints, direct launches."""
+    from .batch import Batch, Group
+
+    groups = []
+    for nx, nz, nb, nmodels, dx, steps in ((301, 201, 20, 4, 10.0, nt), (921, 301, 30, 2, 12.5, 2 * nt),
+                                           (1501, 501, 30, 1, 12.5, 3 * nt)):
+        sx = np.linspace(0, nx - 1, 18)[1:-1].astype(np.int32)
+        groups.append(Group(nx, nz, nb, dx, 0.001, 10.0, steps, sx, np.full_like(sx, 2), 0, nx, 0, nmodels, 1.0))
+    b = Batch(groups, snap_prec=capi.SNAP_BF16)
+    b.set_graphs(False)
+    for gi, g in enumerate(groups):
+        for m in range(g.nmodels):
+            v = workloads.layered_model(g.nz, g.nx, 1500.0, 4500.0, seed=100 + 10 * gi + m)
+            b.bind_model(gi, m, capi.expand_domain(v, g.nb, g.dx, g.dt))
+    dobs = b.forward()
+    b.adjoint_source(dobs, want=False)
+    b.forward(want_data=False)
+    b.backward(None, want_entries=False, want_models=False)
+    inf = b.info()
+    print(f"mixed: {inf['entries']} entries, forward {inf['forward_ms']:.1f} ms, backward {inf['backward_ms']:.1f} ms, "
+          f"{'strips' if b.strips() else 'tiles'}", flush=True)
+
+
 def main(argv=None):
     ap = argparse.ArgumentParser()
-    ap.add_argument("mode", choices=["copy", "shots", "ess", "fwi", "enkf", "enfwi", "sweep", "net"])
+    ap.add_argument("mode", choices=["copy", "shots", "ess", "fwi", "enkf", "enfwi", "sweep", "net", "mixed"])
     ap.add_argument("--entries", default="1,2,3,4,8,16,60,100,200")
     ap.add_argument("--reps", type=int, default=100)
     ap.add_argument("--precision", choices=["exact", "fp32"], default="exact")
@@ -247,6 +274,8 @@ def main(argv=None):
         run_fwi(a.nt or 2000, a.epochs)
     elif a.mode == "net":
         run_net(a.reps)
+    elif a.mode == "mixed":
+        run_mixed(a.nt or 400)
     else:
         run_ess(a.nt or 1000, a.epochs, graphs=not a.no_graphs)
     return 0
